@@ -323,10 +323,12 @@ void dense_assemble_invert_batch(hipStream_t s, int nx, int ny, int nz, int N,
 // diagonal D, then invert it in place (Gauss-Jordan, SPD, one workgroup).
 void dense_assemble(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* D,
                     double* M, int N);
-// form 0: registers for N <= 64 (one barrier per pivot), else LDS / global;
+// form 0: registers for N <= 64 (one barrier per pivot), else LDS, else blocks;
 // form 1: never the register form.  flag (host-mapped, may be null) receives
-// the 1-based index of a pivot that is not positive and finite (the operator
+// the 1-based index of the first pivot that is not positive and finite (the operator
 // is not positive definite); it is left alone otherwise.
+// work holds dense_work(N) doubles.
+size_t dense_work(int N);
 void dense_invert(hipStream_t s, double* M, double* work, int N, int form = 0,
                   double* flag = nullptr);
 // x(interior) = Minv * f(interior); boundary untouched

@@ -199,7 +199,7 @@ int gsrb_impl(int nx, int ny, int nz, int st, const double* a, const double* cc,
 int pmgtest_dense_invert(int N, const double* M, double* out, int form) {
   if (N <= 0 || N > 4096 || form < 0 || form > 1) return 0;
   const size_t nn = (size_t)N * N;
-  double *dM = up(M, nn), *dw = up(nullptr, (size_t)N);
+  double *dM = up(M, nn), *dw = up(nullptr, pmg::dense_work(N));
   pmg::dense_invert(0, dM, dw, N, form);
   TCHECK(hipDeviceSynchronize());
   down(out, dM, nn);

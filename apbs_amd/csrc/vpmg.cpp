@@ -1087,7 +1087,7 @@ size_t pmgint::footprint_bytes(int nx, int ny, int nz, int nlev, bool newton, bo
   if (newton) h += 4 * blk(8 * n);                   // wn1..3, nlw
   if (mixed) h += 2 * blk(4 * n);                    // w1f, xs32
   const double dn = (double)(dims[nt - 1][0] - 2) * (dims[nt - 1][1] - 2) * (dims[nt - 1][2] - 2);
-  h += blk(8 * dn * dn) + blk(8 * dn);
+  h += blk(8 * dn * dn) + blk(8.0 * pmg::dense_work((int)dn));
   return (size_t)(b + std::max(fill, h));
 }
 
@@ -1208,7 +1208,7 @@ void alloc_hierarchy(PmgDev* d, int nlev, bool newton, bool mixed) {
   const DLevel& C = d->L[d->ntot - 1];
   d->dn = (C.nx - 2) * (C.ny - 2) * (C.nz - 2);
   d->dense = dalloc<double>((size_t)d->dn * d->dn);
-  d->dwork = dalloc<double>(d->dn);
+  d->dwork = dalloc<double>(pmg::dense_work(d->dn));
 }
 
 // Vbuildops (mgsubd.c:61-258): fine FV operator, Galerkin coarse operators,

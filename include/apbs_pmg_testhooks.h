@@ -83,7 +83,7 @@ int pmgtest_resid32(int nx, int ny, int nz, const float *oE, const float *oN, co
 int pmgtest_gs27_sweeps(int n, int word, int sweeps, int mode, double *us_per_sweep);
 /* No reference counterpart (the reference factors its coarsest operator in
  * band form, mgsubd.c:244-255): the dense inverse of the coarsest level's
- * operator, form 0 (by size: registers for N <= 64) or 1 (LDS / global). */
+ * operator, form 0 (by size: registers for N <= 64) or 1 (LDS / blocks). */
 int pmgtest_dense_invert(int N, const double *M, double *out, int form);
 /* No reference counterpart: microseconds per Galerkin call (form as above)
  * on a synthetic nf^3 operator of stencil st (nf odd). */

@@ -1,0 +1,69 @@
+"""Forms of the coarse-level kernels at the sizes where their tiling turns.
+
+The blocked dense inverse (coarsest grids that cannot halve down to 64
+unknowns) against numpy, at one unknown past the one-workgroup form, at whole
+and partial 64-pivot blocks, and at N = 1000 (the 12^3 coarsest grid under
+353^3); and a whole solve whose coarsest grid takes that form, against the
+oracle.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import orc_driver as od
+from apbs_amd import driver, synth
+
+pytestmark = pytest.mark.gpu
+
+dp = ctypes.POINTER(ctypes.c_double)
+
+
+def P(a):
+    return a.ctypes.data_as(dp)
+
+
+@pytest.fixture(scope="module")
+def L():
+    import apbs_amd
+    return ctypes.CDLL(apbs_amd.LIB_PATH)
+
+
+@pytest.mark.parametrize("N", [90, 127, 128, 129, 216, 1000])
+def test_blocked_dense_inverse(L, N):
+    """Both sides within the backward error of an elimination without
+    pivoting of a diagonally dominant matrix, 4 N eps cond(A)."""
+    rng = np.random.default_rng(N)
+    A = rng.uniform(-1, 0, (N, N))
+    A = 0.5 * (A + A.T)
+    np.fill_diagonal(A, 0.0)
+    A[np.diag_indices(N)] = -A.sum(axis=1) + rng.uniform(0.5, 2.0, N)
+    A = np.ascontiguousarray(A)
+    out = np.zeros((N, N))
+    assert L.pmgtest_dense_invert(N, P(A), P(out), 0) == 1
+    ref = np.linalg.inv(A)
+    tol = 4 * N * np.finfo(float).eps * np.linalg.cond(A)
+    err = np.linalg.norm(out - ref) / np.linalg.norm(ref)
+    print(f"N {N}: relative difference {err:.2e}, bound {tol:.2e}")
+    assert err <= tol
+    assert np.abs(A @ out - np.eye(N)).max() <= tol
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("dims", [(57, 57, 57), (49, 57, 57)])
+def test_solve_on_a_large_coarsest_grid(dims, precision):
+    """Grids that stop halving at 8^3 (216 unknowns) and at 7 x 8 x 8 (180):
+    converged energy and potential against the oracle."""
+    atoms = synth.globule(60, (6.0,) * 3, 9, net_charge=1)[:3]
+    pbe = dict(pdie=2.0, sdie=78.54, srfm="spl2", chgm="spl2", swin=0.3, srad=1.4, sdens=10.0,
+               temp=298.15, bcfl="mdh", ions=[(1, 0.15, 2.0), (-1, 0.15, 2.0)], etol=1e-12)
+    c = od.mol_center(atoms[0])
+    mol = driver.Molecule(*atoms)
+    eg, g = driver.run_manual(mol, list(dims), c, pbe, grid=[0.45] * 3, precision=precision)
+    eo, o = od.run_manual(atoms, list(dims), c, dict(pbe, coarse_smoother=1, deep_coarse=1),
+                          grid=[0.45] * 3)
+    ug, uo = g.array("u"), o.array("u")
+    rel = abs(eg - eo) / abs(eo)
+    l2 = np.linalg.norm(ug - uo) / np.linalg.norm(uo)
+    print(f"{dims} precision {precision}: energy {rel:.2e}, potential {l2:.2e}, {g.stats()}")
+    assert rel < 1e-9 and l2 < 1e-9
