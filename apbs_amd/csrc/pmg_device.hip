@@ -8,6 +8,8 @@
 // in-place lexicographic sweep (gsd.c:230-327), whose dependencies are serial.
 #include "pmg_device.h"
 
+#include "stencil27.h"
+
 #include <type_traits>
 
 #include <cstdio>
@@ -19,24 +21,6 @@
 namespace pmg {
 
 namespace {
-
-constexpr int kBlock = 256;
-
-// Kernel-argument container of a batched launch: one argument set per
-// calculation (at most kMaxBatch).
-template <class P>
-struct Batch {
-  P v[kMaxBatch];
-};
-
-__host__ __device__ inline size_t IX(int i, int j, int k, int nx, int ny) {
-  return ((size_t)k * ny + j) * nx + i;
-}
-
-inline dim3 grid_interior(int nx, int ny, int nz) {
-  long cnt = (long)(nx - 2) * (ny - 2);
-  return dim3((unsigned)((cnt + kBlock - 1) / kBlock), (unsigned)(nz - 2), 1);
-}
 
 // ------------------------------------------------------------------ 7-point
 // fc + north + south + east + west + down + up, left to right.
@@ -488,57 +472,6 @@ __global__ void __launch_bounds__(kNT)
                                              a.xi, a.xo, first);
 }
 
-// ----------------------------------------------------------------- 27-point
-template <class T>
-struct P27 {
-  T o, u, d;
-};
-
-template <class T>
-__device__ inline P27<T> part27(const T* const* a, const T* __restrict__ x, size_t p, int nx,
-                                size_t nxy) {
-  const T *oE = a[1], *oN = a[2], *uC = a[3], *oNE = a[4], *oNW = a[5], *uE = a[6], *uW = a[7],
-          *uN = a[8], *uS = a[9], *uNE = a[10], *uNW = a[11], *uSE = a[12], *uSW = a[13];
-  P27<T> r;
-  T o = oN[p] * x[p + nx];
-  o += oN[p - nx] * x[p - nx];
-  o += oE[p] * x[p + 1];
-  o += oE[p - 1] * x[p - 1];
-  o += oNE[p] * x[p + nx + 1];
-  o += oNW[p] * x[p + nx - 1];
-  o += oNW[p - nx + 1] * x[p - nx + 1];
-  o += oNE[p - nx - 1] * x[p - nx - 1];
-  const size_t q = p + nxy;
-  T u = uC[p] * x[q];
-  u += uN[p] * x[q + nx];
-  u += uS[p] * x[q - nx];
-  u += uE[p] * x[q + 1];
-  u += uW[p] * x[q - 1];
-  u += uNE[p] * x[q + nx + 1];
-  u += uNW[p] * x[q + nx - 1];
-  u += uSE[p] * x[q - nx + 1];
-  u += uSW[p] * x[q - nx - 1];
-  const size_t m = p - nxy;
-  T d = uC[m] * x[m];
-  d += uS[m + nx] * x[m + nx];
-  d += uN[m - nx] * x[m - nx];
-  d += uW[m + 1] * x[m + 1];
-  d += uE[m - 1] * x[m - 1];
-  d += uSW[m + nx + 1] * x[m + nx + 1];
-  d += uSE[m + nx - 1] * x[m + nx - 1];
-  d += uNW[m - nx + 1] * x[m - nx + 1];
-  d += uNE[m - nx - 1] * x[m - nx - 1];
-  r.o = o;
-  r.u = u;
-  r.d = d;
-  return r;
-}
-
-template <class T>
-struct Ops27 {
-  const T* a[14];
-};
-
 // One colour of the 8-colour sweep: 0-based parities (c&1, (c>>1)&1, (c>>2)&1).
 // Latency-bound on the small coarse levels: up to 128 VGPRs, so that all 54
 // operands of a point are in flight at once.
@@ -561,17 +494,6 @@ __device__ __forceinline__ void gsrb27_body(int nx, int ny, int nz, const Ops27<
   P27<T> s = part27<T>(A.a, x, p, nx, nxy);
   x[p] = (fc[p] + (s.o + s.u + s.d)) / D[p];
 }
-
-// One calculation of a 27-point smoothing, residual or damping launch.
-template <class T>
-struct Args27 {
-  Ops27<T> A;
-  const T* D;
-  const T* f;
-  T* x;
-  T* y;  // plane form: the neighbour planes' values; residual: the output
-  T* z;  // plane form: the output
-};
 
 template <class T>
 __global__ void __launch_bounds__(kBlock)
@@ -830,100 +752,6 @@ __global__ void __launch_bounds__(kBlock)
   stageB(std::integral_constant<int, 0>{});
   if constexpr (kH > 1) stageB(std::integral_constant<int, 1>{});
   if (act) vst16(x + p, out);
-}
-
-// The four colours of one plane parity of that sweep in one launch: colours
-// 4ck .. 4ck+3 (4ck+3 .. 4ck for the adjoint sweep).  Planes of one parity do
-// not touch each other, so a workgroup owns a TX x TY tile of one plane.  It
-// loads the plane's values over the tile and a 4-point margin into LDS and
-// runs the four colours there in order: colour s over the tile grown by 3 - s
-// points, so the margin holds every value the tile's later colours read.
-// Margin points are computed by several workgroups, identically, and only the
-// tile is written.  In-plane values come from src, the neighbouring planes
-// from nbr, and the result goes to dst, so no workgroup reads what another
-// writes.  The arithmetic is part27's, term for term.
-template <class T, int TX, int TY, int NTH>
-__device__ __forceinline__ void plane_body(int nx, int ny, int nz, const Ops27<T>& A,
-                                           const T* __restrict__ D, const T* __restrict__ fc,
-                                           const T* __restrict__ src, const T* __restrict__ nbr,
-                                           T* __restrict__ dst, int ck, int adj) {
-  constexpr int M = 4, LX = TX + 2 * M, LY = TY + 2 * M;
-  __shared__ T sx[LX * LY];
-  const T *oE = A.a[1], *oN = A.a[2], *uC = A.a[3], *oNE = A.a[4], *oNW = A.a[5], *uE = A.a[6],
-          *uW = A.a[7], *uN = A.a[8], *uS = A.a[9], *uNE = A.a[10], *uNW = A.a[11],
-          *uSE = A.a[12], *uSW = A.a[13];
-  const int tilesx = (nx - 2 + TX - 1) / TX;
-  const int tx0 = 1 + (int)(blockIdx.x % tilesx) * TX;
-  const int ty0 = 1 + (int)(blockIdx.x / tilesx) * TY;
-  const int k = (ck ? 1 : 2) + 2 * (int)blockIdx.y;
-  const size_t nxy = (size_t)nx * ny;
-  const size_t kp = (size_t)k * nxy;
-  const int bx = tx0 - M, by = ty0 - M;  // grid coordinates of sx[0]
-  for (int t = threadIdx.x; t < LX * LY; t += NTH) {
-    const int i = bx + t % LX, j = by + t / LX;
-    sx[t] = (i >= 0 && i < nx && j >= 0 && j < ny) ? src[kp + (size_t)j * nx + i] : T(0);
-  }
-  __syncthreads();
-  for (int s = 0; s < 4; s++) {
-    const int q = adj ? 3 - s : s;  // in-plane colour: i parity (q & 1), j parity (q >> 1)
-    const int pi = q & 1, pj = q >> 1;
-    const int g = 3 - s;
-    int ilo = max(1, tx0 - g), jlo = max(1, ty0 - g);
-    const int ihi = min(nx - 2, tx0 + TX - 1 + g), jhi = min(ny - 2, ty0 + TY - 1 + g);
-    // colour parity 0 is the even indices (first interior point 2), 1 the odd
-    ilo += (ilo & 1) != pi;
-    jlo += (jlo & 1) != pj;
-    const int ni = ilo <= ihi ? (ihi - ilo) / 2 + 1 : 0;
-    const int nj = jlo <= jhi ? (jhi - jlo) / 2 + 1 : 0;
-    for (int t = threadIdx.x; t < ni * nj; t += NTH) {
-      const int i = ilo + 2 * (t % ni), j = jlo + 2 * (t / ni);
-      const int e = (j - by) * LX + (i - bx);
-      const size_t p = kp + (size_t)j * nx + i;
-      T o = oN[p] * sx[e + LX];
-      o += oN[p - nx] * sx[e - LX];
-      o += oE[p] * sx[e + 1];
-      o += oE[p - 1] * sx[e - 1];
-      o += oNE[p] * sx[e + LX + 1];
-      o += oNW[p] * sx[e + LX - 1];
-      o += oNW[p - nx + 1] * sx[e - LX + 1];
-      o += oNE[p - nx - 1] * sx[e - LX - 1];
-      const size_t qa = p + nxy;
-      T u = uC[p] * nbr[qa];
-      u += uN[p] * nbr[qa + nx];
-      u += uS[p] * nbr[qa - nx];
-      u += uE[p] * nbr[qa + 1];
-      u += uW[p] * nbr[qa - 1];
-      u += uNE[p] * nbr[qa + nx + 1];
-      u += uNW[p] * nbr[qa + nx - 1];
-      u += uSE[p] * nbr[qa - nx + 1];
-      u += uSW[p] * nbr[qa - nx - 1];
-      const size_t m = p - nxy;
-      T d = uC[m] * nbr[m];
-      d += uS[m + nx] * nbr[m + nx];
-      d += uN[m - nx] * nbr[m - nx];
-      d += uW[m + 1] * nbr[m + 1];
-      d += uE[m - 1] * nbr[m - 1];
-      d += uSW[m + nx + 1] * nbr[m + nx + 1];
-      d += uSE[m + nx - 1] * nbr[m + nx - 1];
-      d += uNW[m - nx + 1] * nbr[m - nx + 1];
-      d += uNE[m - nx - 1] * nbr[m - nx - 1];
-      sx[e] = (fc[p] + (o + u + d)) / D[p];
-    }
-    __syncthreads();
-  }
-  for (int t = threadIdx.x; t < TX * TY; t += NTH) {
-    const int i = tx0 + t % TX, j = ty0 + t / TX;
-    if (i <= nx - 2 && j <= ny - 2) dst[kp + (size_t)j * nx + i] = sx[(j - by) * LX + (i - bx)];
-  }
-}
-
-// (x, y, z) of a calculation: the plane's own values, the neighbour planes'
-// values and the output.
-template <class T, int TX, int TY, int NTH>
-__global__ void __launch_bounds__(NTH)
-    k_gs27_plane(int nx, int ny, int nz, Batch<Args27<T>> B, int ck, int adj) {
-  const Args27<T>& a = B.v[blockIdx.z];
-  plane_body<T, TX, TY, NTH>(nx, ny, nz, a.A, a.D, a.f, a.x, a.y, a.z, ck, adj);
 }
 
 template <class T>
@@ -2331,21 +2159,6 @@ inline unsigned nblocks(size_t n) {
   return (unsigned)b;
 }
 
-template <class T>
-Ops27<T> to27(const Ops<T>& A) {
-  Ops27<T> o;
-  for (int s = 0; s < 14; s++) o.a[s] = A.a[s];
-  return o;
-}
-
-// A batched launch takes at most kMaxBatch calculations.
-inline void check_batch(int nb) {
-  if (nb < 1 || nb > kMaxBatch) {
-    fprintf(stderr, "pmg: a batched launch takes 1 to %d calculations, not %d\n", kMaxBatch, nb);
-    abort();
-  }
-}
-
 }  // namespace
 
 // =================================================================== wrappers
@@ -2676,58 +2489,6 @@ void gsrb27_pairs(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const 
                   const T* fc, T* x, int nu, int iadjoint) {
   const LevelArgs<T> c{A, D, fc, x, nullptr, nullptr};
   gsrb27_pairs_batch<T>(s, nx, ny, nz, &c, 1, nu, iadjoint);
-}
-
-// Workgroups of a plane-parity launch with TX x TY tiles.
-static long gs27_groups(int nx, int ny, int nz, int tx, int ty) {
-  return (long)((nx - 2 + tx - 1) / tx) * ((ny - 2 + ty - 1) / ty) * ((nz - 2) / 2);
-}
-
-int gsrb27_planes_tile(int nx, int ny, int nz) {
-  if (gs27_groups(nx, ny, nz, 32, 32) >= 256) return 32;
-  if (gs27_groups(nx, ny, nz, 16, 16) >= 64) return 16;
-  return 8;
-}
-
-template <class T>
-void gsrb27_planes_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,
-                         int nu, int iadjoint, int tile) {
-  check_batch(nb);
-  if (nx < 3 || ny < 3 || nz < 3) return;
-  if (tile != 8 && tile != 16 && tile != 32) tile = gsrb27_planes_tile(nx, ny, nz);
-  for (int it = 0; it < nu; it++) {
-    // sweep it reads x (even it) or xs and writes the other one
-    const int first = iadjoint ? 1 : 0;
-    for (int h = 0; h < 2; h++) {
-      const int ck = h == 0 ? first : 1 - first;
-      const int k0 = ck ? 1 : 2;
-      if (k0 > nz - 2) continue;
-      const int nk = (nz - 2 - k0) / 2 + 1;
-      Batch<Args27<T>> B;
-      for (int b = 0; b < nb; b++) {
-        T* in = (it & 1) ? c[b].xs : c[b].x;
-        T* out = (it & 1) ? c[b].x : c[b].xs;
-        B.v[b] = Args27<T>{to27(c[b].A), c[b].D, c[b].f, in, h == 0 ? in : out, out};
-      }
-      const unsigned tiles = (unsigned)(((nx - 2 + tile - 1) / tile) * ((ny - 2 + tile - 1) / tile));
-      const dim3 g(tiles, (unsigned)nk, (unsigned)nb);
-      if (tile == 32)
-        k_gs27_plane<T, 32, 32, kBlock><<<g, kBlock, 0, s>>>(nx, ny, nz, B, ck, iadjoint);
-      else if (tile == 16)
-        k_gs27_plane<T, 16, 16, kBlock><<<g, kBlock, 0, s>>>(nx, ny, nz, B, ck, iadjoint);
-      else
-        k_gs27_plane<T, 8, 8, kBlock><<<g, kBlock, 0, s>>>(nx, ny, nz, B, ck, iadjoint);
-    }
-  }
-  if (nu & 1)
-    for (int b = 0; b < nb; b++) copy_interior<T>(s, nx, ny, nz, c[b].xs, c[b].x);
-}
-
-template <class T>
-void gsrb27_planes(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D,
-                   const T* fc, T* x, T* xs, int nu, int iadjoint, int tile) {
-  const LevelArgs<T> c{A, D, fc, x, xs, nullptr};
-  gsrb27_planes_batch<T>(s, nx, ny, nz, &c, 1, nu, iadjoint, tile);
 }
 
 bool gsrb27_use_planes(int nx, int ny, int nz) { return nx <= 49 && ny <= 49 && nz >= 3; }
@@ -3110,8 +2871,6 @@ void dense_solve(hipStream_t s, int nx, int ny, int nz, const double* Minv, int 
                          int);                                                                  \
   template void gsrb27<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*, T*, int, \
                           int);                                                                 \
-  template void gsrb27_planes<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*,  \
-                                 T*, T*, int, int, int);                                        \
   template void gsrb27_pairs<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*,   \
                                 T*, int, int);                                                  \
   template void resid<T>(hipStream_t, int, int, int, int, const Ops<T>&, const T*, const T*,     \
@@ -3138,8 +2897,6 @@ void dense_solve(hipStream_t s, int nx, int ny, int nz, const double* Minv, int 
                                       int);                                                     \
   template void gsrb27_pairs_form<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int, int,  \
                                      int, int);                                                 \
-  template void gsrb27_planes_batch<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int,     \
-                                       int, int, int);                                          \
   template void resid_batch<T>(hipStream_t, int, int, int, int, const LevelArgs<T>*, int);       \
   template void restrict3_batch<T>(hipStream_t, int, int, int, int, int, int,                     \
                                    const TransferArgs<T>*, int);                                \
