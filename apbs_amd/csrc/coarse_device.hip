@@ -117,7 +117,340 @@ __global__ void __launch_bounds__(256 * W)
 }
 
 
+// ------------------------------------------------------------ bottom of the cycle
+// The last smoothed level and the coarsest one in one workgroup: restriction of
+// the residual above, the pre-smoothing sweeps from zero, the residual and its
+// restriction, the product with the dense inverse, the damping factor, the
+// prolongation, the adjoint sweeps, and the damping factor of the level itself.
+// Launched one by one these are 17 launches of 3 to 9 us on data that fits one
+// CU.  Here a thread owns a point: its 26 coefficients, diagonal and right-hand
+// side stay in registers, the level's values in LDS, and a colour step is 26
+// LDS reads, the sums and a division between two barriers.  Points are dealt to
+// threads colour by colour, so a colour step is a few whole wavefronts.  Every
+// value is formed by the separate kernels' expressions in their order (the
+// reductions in the trees of k_damp_part and k_finish), so the cycle keeps its
+// bits.
+constexpr int kBotPts = 1728;     // points of the level with its boundary
+constexpr int kBotInner = 1024;   // interior points, one per thread
+constexpr int kBotCoarse = 512;   // points of the coarsest level with its boundary
+constexpr int kBotN = 64;         // unknowns of the coarsest level
+
+template <class T>
+struct BottomPart {
+  Ops27<T> A, Ac;
+  const T *D, *Dc;
+  const T* r;
+  T* x;
+  const double* Minv;
+  double* damp;
+};
+
+// part27's sums at LDS index e of x (rows of nx, planes of nxy) with the 26
+// coefficients in its order.
+template <class T>
+__device__ __forceinline__ P27<T> part27_lds(const T (&c)[26], const T* x, int e, int nx,
+                                             int nxy) {
+  P27<T> r;
+  T o = c[0] * x[e + nx];
+  o += c[1] * x[e - nx];
+  o += c[2] * x[e + 1];
+  o += c[3] * x[e - 1];
+  o += c[4] * x[e + nx + 1];
+  o += c[5] * x[e + nx - 1];
+  o += c[6] * x[e - nx + 1];
+  o += c[7] * x[e - nx - 1];
+  const int q = e + nxy, m = e - nxy;
+  T u = c[8] * x[q];
+  u += c[9] * x[q + nx];
+  u += c[10] * x[q - nx];
+  u += c[11] * x[q + 1];
+  u += c[12] * x[q - 1];
+  u += c[13] * x[q + nx + 1];
+  u += c[14] * x[q + nx - 1];
+  u += c[15] * x[q - nx + 1];
+  u += c[16] * x[q - nx - 1];
+  T d = c[17] * x[m];
+  d += c[18] * x[m + nx];
+  d += c[19] * x[m - nx];
+  d += c[20] * x[m + 1];
+  d += c[21] * x[m - 1];
+  d += c[22] * x[m + nx + 1];
+  d += c[23] * x[m + nx - 1];
+  d += c[24] * x[m - nx + 1];
+  d += c[25] * x[m - nx - 1];
+  r.o = o;
+  r.u = u;
+  r.d = d;
+  return r;
+}
+
+template <class T>
+__device__ __forceinline__ void coef27(T (&c)[26], const Ops27<T>& A, size_t p, int nx,
+                                       size_t nxy) {
+  const T *oE = A.a[1], *oN = A.a[2], *uC = A.a[3], *oNE = A.a[4], *oNW = A.a[5], *uE = A.a[6],
+          *uW = A.a[7], *uN = A.a[8], *uS = A.a[9], *uNE = A.a[10], *uNW = A.a[11],
+          *uSE = A.a[12], *uSW = A.a[13];
+  const size_t m = p - nxy;
+  c[0] = oN[p];
+  c[1] = oN[p - nx];
+  c[2] = oE[p];
+  c[3] = oE[p - 1];
+  c[4] = oNE[p];
+  c[5] = oNW[p];
+  c[6] = oNW[p - nx + 1];
+  c[7] = oNE[p - nx - 1];
+  c[8] = uC[p];
+  c[9] = uN[p];
+  c[10] = uS[p];
+  c[11] = uE[p];
+  c[12] = uW[p];
+  c[13] = uNE[p];
+  c[14] = uNW[p];
+  c[15] = uSE[p];
+  c[16] = uSW[p];
+  c[17] = uC[m];
+  c[18] = uS[m + nx];
+  c[19] = uN[m - nx];
+  c[20] = uW[m + 1];
+  c[21] = uE[m - 1];
+  c[22] = uSW[m + nx + 1];
+  c[23] = uSE[m + nx - 1];
+  c[24] = uNW[m - nx + 1];
+  c[25] = uNE[m - nx - 1];
+}
+
+// restrict_body's sum at index c of in (strides 1, sy, sz).
+template <class T, class I>
+__device__ __forceinline__ T restrict27(const T* in, I c, I sy, I sz) {
+  const T W1 = T(1.0), W2 = T(0.5), W4 = T(0.25), W8 = T(0.125);
+  T o = W1 * in[c];
+  o += W2 * in[c + sy];
+  o += W2 * in[c - sy];
+  o += W2 * in[c + 1];
+  o += W2 * in[c - 1];
+  o += W4 * in[c + 1 + sy];
+  o += W4 * in[c - 1 + sy];
+  o += W4 * in[c + 1 - sy];
+  o += W4 * in[c - 1 - sy];
+  const I u0 = c + sz, d0 = c - sz;
+  T u = W2 * in[u0];
+  u += W4 * in[u0 + sy];
+  u += W4 * in[u0 - sy];
+  u += W4 * in[u0 + 1];
+  u += W4 * in[u0 - 1];
+  u += W8 * in[u0 + 1 + sy];
+  u += W8 * in[u0 - 1 + sy];
+  u += W8 * in[u0 + 1 - sy];
+  u += W8 * in[u0 - 1 - sy];
+  T d = W2 * in[d0];
+  d += W4 * in[d0 + sy];
+  d += W4 * in[d0 - sy];
+  d += W4 * in[d0 + 1];
+  d += W4 * in[d0 - 1];
+  d += W8 * in[d0 + 1 + sy];
+  d += W8 * in[d0 - 1 + sy];
+  d += W8 * in[d0 + 1 - sy];
+  d += W8 * in[d0 - 1 - sy];
+  return o + u + d;
+}
+
+// The halving sum of a 64-entry block over a wavefront; valid in lane 0.
+__device__ __forceinline__ double wave_tree(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  return v;
+}
+
+template <class T>
+__global__ void __launch_bounds__(1024)
+    k_bottom(int nxf, int nyf, int nx, int ny, int nz, int nxc, int nyc, int nzc,
+             Batch<BottomPart<T>> B, int nu) {
+  __shared__ T sx[kBotPts];
+  __shared__ double pool[kBotN * (kBotN + 1)];  // residual, then Minv, then the level's products
+  __shared__ T sxc[kBotCoarse];
+  __shared__ double sfc[kBotN], spart[8], sdamp;
+  const BottomPart<T>& a = B.v[blockIdx.x];
+  const int tid = threadIdx.x, NT = blockDim.x;
+  const int ni = nx - 2, nj = ny - 2, nk = nz - 2, n = ni * nj * nk, nxy = nx * ny;
+  const int cni = nxc - 2, cnj = nyc - 2, N = cni * cnj * (nzc - 2), cxy = nxc * nyc;
+  T* sr = reinterpret_cast<T*>(pool);
+  // the thread's point: colour by colour, x fastest within a colour
+  int col = -1, i = 1, j = 1, k = 1;
+  if (tid < n) {
+    int t = tid;
+    for (int c = 0; c < 8; c++) {
+      const int i0 = (c & 1) ? 1 : 2, j0 = (c & 2) ? 1 : 2, k0 = (c & 4) ? 1 : 2;
+      const int ci = max(0, (nx - 2 - i0) / 2 + 1), cj = max(0, (ny - 2 - j0) / 2 + 1),
+                ck = max(0, (nz - 2 - k0) / 2 + 1);
+      const int m = nx - 2 < i0 || ny - 2 < j0 || nz - 2 < k0 ? 0 : ci * cj * ck;
+      if (t < m) {
+        col = c;
+        i = i0 + 2 * (t % ci);
+        j = j0 + 2 * ((t / ci) % cj);
+        k = k0 + 2 * (t / (ci * cj));
+        break;
+      }
+      t -= m;
+    }
+  }
+  const bool act = col >= 0;
+  const int e = k * nxy + j * nx + i;
+  T c[26], D = T(1), f = T(0);
+  if (act) {
+    coef27<T>(c, a.A, (size_t)e, nx, (size_t)nxy);
+    D = a.D[e];
+    f = restrict27<T, size_t>(a.r, IX(2 * i, 2 * j, 2 * k, nxf, nyf), (size_t)nxf,
+                              (size_t)nxf * nyf);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 26; q++) c[q] = T(0);
+  }
+  // Minv's entries, in flight through the first sweeps
+  double mv[16];
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int t = tid + q * NT;
+    mv[q] = t < N * N ? a.Minv[t] : 0.0;
+  }
+  for (int t = tid; t < nxy * nz; t += NT) sx[t] = T(0);
+  for (int t = tid; t < cxy * nzc; t += NT) sxc[t] = T(0);
+  __syncthreads();
+  auto smooth = [&](bool adj) {
+    for (int it = 0; it < nu; it++)
+      for (int cc = 0; cc < 8; cc++) {
+        if (act && col == (adj ? 7 - cc : cc)) {
+          const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
+          sx[e] = (f + (s.o + s.u + s.d)) / D;
+        }
+        __syncthreads();
+      }
+  };
+  smooth(false);
+  if (act) {
+    const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
+    sr[e] = f + s.o + s.u + s.d - D * sx[e];
+  }
+  __syncthreads();
+  const int ci = tid % cni + 1, cj = (tid / cni) % cnj + 1, ck = tid / (cni * cnj) + 1;
+  if (tid < N)
+    sfc[tid] = (double)restrict27<T, int>(sr, (2 * ck * ny + 2 * cj) * nx + 2 * ci, nx, nxy);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 16; q++) {
+    const int t = tid + q * NT;
+    if (t < N * N) pool[(t / N) * (kBotN + 1) + t % N] = mv[q];
+  }
+  __syncthreads();
+  if (tid < N) {
+    const double* row = pool + tid * (kBotN + 1);
+    double s = 0.0;
+#pragma unroll 8
+    for (int q = 0; q < N; q++) s += row[q] * sfc[q];
+    sxc[(ck * nyc + cj) * nxc + ci] = (T)s;
+  }
+  __syncthreads();
+  if (tid < 64) {  // the coarsest level's damping factor (one block of k_damp_part)
+    double num = 0.0, den = 0.0;
+    if (tid < N) {
+      const int p = (ck * nyc + cj) * nxc + ci;
+      T cc[26];
+      coef27<T>(cc, a.Ac, (size_t)p, nxc, (size_t)cxy);
+      const P27<T> s = part27_lds<T>(cc, sxc, p, nxc, cxy);
+      const T xv = sxc[p];
+      const T ax = (-s.o) + (-s.u) + (-s.d) + a.Dc[p] * xv;
+      num += (double)xv * sfc[tid];
+      den += (double)xv * (double)ax;
+    }
+    num = wave_tree(num);
+    den = wave_tree(den);
+    if (tid == 0) sdamp = num / den;
+  }
+  __syncthreads();
+  if (act) {  // prolong_body
+    const int bx = i & 1, by = j & 1, bz = k & 1;
+    const T W = (bx ? T(0.5) : T(1.0)) * (by ? T(0.5) : T(1.0)) * (bz ? T(0.5) : T(1.0));
+    const int c0 = ((k >> 1) * nyc + (j >> 1)) * nxc + (i >> 1);
+    T v = W * sxc[c0];
+    if (bx) v += W * sxc[c0 + 1];
+    if (by) {
+      v += W * sxc[c0 + nxc];
+      if (bx) v += W * sxc[c0 + nxc + 1];
+    }
+    if (bz) {
+      v += W * sxc[c0 + cxy];
+      if (bx) v += W * sxc[c0 + cxy + 1];
+      if (by) {
+        v += W * sxc[c0 + cxy + nxc];
+        if (bx) v += W * sxc[c0 + cxy + nxc + 1];
+      }
+    }
+    sx[e] = sx[e] + T(sdamp) * v;
+  }
+  __syncthreads();
+  smooth(true);
+  // the level's damping factor: products in interior order (x fastest), one
+  // block of 256 per wavefront as k_damp_part sums them, then k_finish's sum
+  double* num = pool;
+  double* den = pool + kBotInner;
+  for (int t = tid; t < 2 * kBotInner; t += NT) pool[t] = 0.0;
+  __syncthreads();
+  if (act) {
+    const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
+    const T xv = sx[e];
+    const T ax = (-s.o) + (-s.u) + (-s.d) + D * xv;
+    const int q = (i - 1) + ni * ((j - 1) + nj * (k - 1));
+    double nv = 0.0, dv = 0.0;
+    nv += (double)xv * (double)f;
+    dv += (double)xv * (double)ax;
+    num[q] = nv;
+    den[q] = dv;
+    a.x[e] = xv;
+  }
+  __syncthreads();
+  const int w = tid >> 6, lane = tid & 63;
+  if (w < 4) {
+    auto block = [&](const double* v) {
+      const double* b = v + 256 * w;
+      const double b0 = b[lane] + b[lane + 128], b1 = b[lane + 64] + b[lane + 192];
+      return wave_tree(b0 + b1);
+    };
+    const double sn = block(num), sd = block(den);
+    if (lane == 0) {
+      spart[w] = sn;
+      spart[4 + w] = sd;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const double sa = (spart[0] + spart[2]) + (spart[1] + spart[3]);
+    const double sb = (spart[4] + spart[6]) + (spart[5] + spart[7]);
+    a.damp[0] = sa / sb;
+    a.damp[1] = sa;
+    a.damp[2] = sb;
+  }
+}
+
 }  // namespace
+
+bool bottom_fits(int nx, int ny, int nz, int nxc, int nyc, int nzc) {
+  if (nx < 3 || ny < 3 || nz < 3 || nxc < 3 || nyc < 3 || nzc < 3) return false;
+  return (long)(nx - 2) * (ny - 2) * (nz - 2) <= kBotInner && (long)nx * ny * nz <= kBotPts &&
+         (long)(nxc - 2) * (nyc - 2) * (nzc - 2) <= kBotN && (long)nxc * nyc * nzc <= kBotCoarse;
+}
+
+template <class T>
+void bottom_batch(hipStream_t s, const int above[3], const int level[3], const int coarsest[3],
+                  const BottomArgs<T>* c, int nb, int nu) {
+  check_batch(nb);
+  Batch<BottomPart<T>> B;
+  for (int b = 0; b < nb; b++)
+    B.v[b] = BottomPart<T>{to27(c[b].A), to27(c[b].Ac), c[b].D,    c[b].Dc,
+                           c[b].r,       c[b].x,        c[b].Minv, c[b].damp};
+  const int n = (level[0] - 2) * (level[1] - 2) * (level[2] - 2);
+  // at least 256 threads: Minv is held by them, 16 entries each
+  const int nt = n <= 256 ? 256 : (n + 63) / 64 * 64;
+  k_bottom<T><<<nb, nt, 0, s>>>(above[0], above[1], level[0], level[1], level[2], coarsest[0],
+                                coarsest[1], coarsest[2], B, nu);
+}
 
 int gsrb27_planes_tile(int nx, int ny, int nz) {
   const long groups = (long)((nx - 2 + 15) / 16) * ((ny - 2 + 15) / 16) * ((nz - 2) / 2);
@@ -168,7 +501,9 @@ void gsrb27_planes(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const
   template void gsrb27_planes<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*, \
                                  T*, T*, int, int, int);                                       \
   template void gsrb27_planes_batch<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int,    \
-                                       int, int, int);
+                                       int, int, int);                                         \
+  template void bottom_batch<T>(hipStream_t, const int[3], const int[3], const int[3],          \
+                                const BottomArgs<T>*, int, int);
 INST(double)
 INST(float)
 #undef INST

@@ -307,6 +307,25 @@ struct DenseArgs {
 template <class T>
 void dense_solve_batch(hipStream_t s, int nx, int ny, int nz, int N, const DenseArgs<T>* c,
                        int nb);
+// The last smoothed level and the coarsest one of a V-cycle in one launch, from
+// the residual r of the level above: restriction, nu sweeps from zero,
+// residual, restriction, dense inverse, damped prolongation, nu adjoint
+// sweeps.  x gets the level's interior, damp its damping factor (damp_factor's
+// three values).  Every value is the separate launches' bit for bit.
+// bottom_fits: one workgroup holds the two levels.
+template <class T>
+struct BottomArgs {
+  Ops<T> A, Ac;
+  const T *D, *Dc;
+  const T* r;
+  T* x;
+  const double* Minv;
+  double* damp;
+};
+bool bottom_fits(int nx, int ny, int nz, int nxc, int nyc, int nzc);
+template <class T>
+void bottom_batch(hipStream_t s, const int above[3], const int level[3], const int coarsest[3],
+                  const BottomArgs<T>* c, int nb, int nu);
 // dense_assemble then dense_invert per calculation (form and flag as there)
 struct InvertArgs {
   Ops<double> A;

@@ -1390,11 +1390,17 @@ void vcycle_batch(PmgDev* const* ds, CycleArgs<T>* cs, int n) {
       pmg::gsrb27_batch<T>(s, L[l].nx, L[l].ny, L[l].nz, la, n, 2, adj);
   };
   const int ecyc = n == 1 ? tbegin(d0) : -1;
+  // the last smoothed level and the coarsest one in one launch where they fit
+  // one workgroup
+  const bool bottom = d0->smoother27 == 0 && nt >= 3 &&
+                      pmg::bottom_fits(L[nt - 2].nx, L[nt - 2].ny, L[nt - 2].nz, L[nt - 1].nx,
+                                       L[nt - 1].ny, L[nt - 1].nz);
+  const int nsep = bottom ? nt - 2 : nt;  // levels that are launched one by one
   // calculations of a batch start alike (every mixed-precision cycle from zero)
   fine_smooth(0, cs[0].zero_x);
   level(0, true);
   pmg::resid_batch<T>(s, 7, L[0].nx, L[0].ny, L[0].nz, la, n);
-  for (int l = 1; l < nt; l++) {
+  for (int l = 1; l < nsep; l++) {
     // the coarse solution starts at zero (interior cleared with the
     // restriction; the boundary layer is never written)
     for (int b = 0; b < n; b++)
@@ -1409,21 +1415,33 @@ void vcycle_batch(PmgDev* const* ds, CycleArgs<T>* cs, int n) {
     }
   }
   const DLevel& C = L[nt - 1];
-  pmg::DenseArgs<T> da[pmg::kMaxBatch];
-  for (int b = 0; b < n; b++) {
-    join_dense(ds[b]);
-    da[b] = pmg::DenseArgs<T>{ds[b]->dense, cs[b].w0[nt - 1], cs[b].X[nt - 1]};
+  for (int b = 0; b < n; b++) join_dense(ds[b]);
+  if (bottom) {
+    pmg::BottomArgs<T> ba[pmg::kMaxBatch];
+    for (int b = 0; b < n; b++)
+      ba[b] = pmg::BottomArgs<T>{cs[b].A[nt - 2], cs[b].A[nt - 1], cs[b].Dl[nt - 2],
+                                 cs[b].Dl[nt - 1], cs[b].w1, cs[b].X[nt - 2], ds[b]->dense,
+                                 ds[b]->scal + 4};
+    const int dims[3][3] = {{L[nt - 3].nx, L[nt - 3].ny, L[nt - 3].nz},
+                            {L[nt - 2].nx, L[nt - 2].ny, L[nt - 2].nz},
+                            {C.nx, C.ny, C.nz}};
+    pmg::bottom_batch<T>(s, dims[0], dims[1], dims[2], ba, n, 2);
+  } else {
+    pmg::DenseArgs<T> da[pmg::kMaxBatch];
+    for (int b = 0; b < n; b++)
+      da[b] = pmg::DenseArgs<T>{ds[b]->dense, cs[b].w0[nt - 1], cs[b].X[nt - 1]};
+    pmg::dense_solve_batch<T>(s, C.nx, C.ny, C.nz, d0->dn, da, n);
   }
-  pmg::dense_solve_batch<T>(s, C.nx, C.ny, C.nz, d0->dn, da, n);
   pmg::DampArgs<T> pa[pmg::kMaxBatch];
-  for (int l = nt - 2; l >= 0; l--) {
+  for (int l = bottom ? nt - 3 : nt - 2; l >= 0; l--) {
     const DLevel& Cl = L[l + 1];
+    const bool damped = bottom && l == nt - 3;  // the bottom launch left its factor
     for (int b = 0; b < n; b++) {
       pa[b] = pmg::DampArgs<T>{cs[b].A[l + 1], cs[b].Dl[l + 1], cs[b].X[l + 1], cs[b].w0[l + 1],
                                ds[b]->part, ds[b]->scal + 4};
       ta[b] = pmg::TransferArgs<T>{cs[b].X[l + 1], cs[b].X[l], nullptr, ds[b]->scal + 4};
     }
-    pmg::damp_factor_batch<T>(s, Cl.nx, Cl.ny, Cl.nz, pa, n);
+    if (!damped) pmg::damp_factor_batch<T>(s, Cl.nx, Cl.ny, Cl.nz, pa, n);
     pmg::prolong_add_batch<T>(s, Cl.nx, Cl.ny, Cl.nz, L[l].nx, L[l].ny, L[l].nz, ta, n);
     if (l == 0)
       fine_smooth(1, false);

@@ -67,3 +67,29 @@ def test_solve_on_a_large_coarsest_grid(dims, precision):
     l2 = np.linalg.norm(ug - uo) / np.linalg.norm(uo)
     print(f"{dims} precision {precision}: energy {rel:.2e}, potential {l2:.2e}, {g.stats()}")
     assert rel < 1e-9 and l2 < 1e-9
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("npbe", [False, True])
+@pytest.mark.parametrize("dims", [(17, 17, 17), (33, 33, 33), (41, 41, 41), (49, 33, 17),
+                                  (81, 65, 33), (97, 33, 33)])
+def test_bottom_of_the_cycle_bitwise(dims, npbe, precision, monkeypatch):
+    """The one-launch bottom of the V-cycle (a level of at most 1,024 interior
+    points above a coarsest one of at most 64) against the separate launches:
+    the same potential bit for bit and the same iteration counts, cubic and
+    ragged levels, both words.  The separate launches run in the colour form
+    (APBS_PMG_SMOOTHER27), itself bitwise the oracle's sweep."""
+    atoms = synth.globule(40, (5.0,) * 3, 9, net_charge=1)[:3]
+    pbe = dict(npbe=npbe, pdie=2.0, sdie=78.54, srfm="spl2", chgm="spl2", swin=0.3, srad=1.4,
+               sdens=10.0, temp=298.15, bcfl="mdh", ions=[(1, 0.15, 2.0), (-1, 0.15, 2.0)])
+    c = od.mol_center(atoms[0])
+    mol = driver.Molecule(*atoms)
+    out = []
+    for form in (None, "colour"):
+        if form:
+            monkeypatch.setenv("APBS_PMG_SMOOTHER27", form)
+        e, g = driver.run_manual(mol, list(dims), c, pbe, grid=[0.6] * 3, precision=precision)
+        out.append((e, g.array("u"), g.stats()))
+    (ea, ua, sa), (eb, ub, sb) = out
+    assert (sa["iters"], sa["inner"], sa["nlev"]) == (sb["iters"], sb["inner"], sb["nlev"])
+    assert ea == eb and np.array_equal(ua, ub)
