@@ -117,6 +117,151 @@ __global__ void __launch_bounds__(256 * W)
 }
 
 
+// The plane-parity sweep over whole rows: a workgroup owns 2m consecutive rows
+// of a plane and a lane a run of kV consecutive points of a row (both colours).
+// With whole rows only the rows one above and one below the tile are computed
+// twice (the square tiles above recompute 3 columns and rows a side), and a
+// lane's 26 coefficient terms, f and D are one 8- or 16-byte load each, where
+// the form above loads single words two apart, four of its 46 loads a point
+// going through the addresser at a time.  Lanes: the m + 1 rows of the first
+// row parity (colours 0 and 1 of the plane), then the m rows of the second.
+// The neighbour planes' sums are formed before the first colour; a colour step
+// reads the plane's values from LDS.  part27's terms in its order.
+// us per sweep of two launches (the best other form, then this one): 49^3 FP64
+// 14.3, 11.4, FP32 11.1, 10.7; 65^3 20.3, 15.4 and 15.3, 11.7; 81^3 35.4, 26.9
+// and 22.8, 18.4; 97^3 45.7, 41.8 and 29.2, 24.4; 177^3 506, 266 and 262, 122
+// (one launch per colour: its rows are too long for the pair form).
+template <class T, int kV>
+__global__ void __launch_bounds__(512)
+    k_gs27_rows(int nx, int ny, int nz, Batch<Args27<T>> B, int ck, int adj, int R, int m) {
+  extern __shared__ unsigned char rows_smem[];
+  T* sx = reinterpret_cast<T*>(rows_smem);
+  const Args27<T>& ar = B.v[blockIdx.z];
+  const T* const* a = ar.A.a;
+  const T *src = ar.x, *nbr = ar.y;
+  const int j0 = 1 + (int)blockIdx.x * 2 * m;  // the tile's first row
+  const int k = (ck ? 1 : 2) + 2 * (int)blockIdx.y;
+  const size_t nxy = (size_t)nx * ny;
+  const size_t kp = (size_t)k * nxy;
+  // row parity of the first two colours; the lane's row and run
+  const int first = adj ? 1 : 0;
+  const int lr = (int)threadIdx.x / R, run = (int)threadIdx.x % R;
+  const int g = lr <= m ? 0 : 1;  // row group
+  int j = g == 0 ? j0 - 1 + 2 * lr + (((j0 - 1) & 1) != first)
+                 : j0 + 2 * (lr - m - 1) + ((j0 & 1) == first);
+  const bool act = lr < 2 * m + 1 && j >= 1 && j <= ny - 2;
+  if (!act) j = 1;
+  const int ib = min(1 + kV * run, nx - 1 - kV);
+  const size_t p = kp + (size_t)j * nx + ib;
+  const int e = (j - (j0 - 2)) * nx + ib;  // LDS index of the run
+  T co[8][kV], f[kV], D[kV], u[kV], d[kV];
+  if (act) {
+    const T *oE = a[1], *oN = a[2], *uC = a[3], *oNE = a[4], *oNW = a[5], *uE = a[6], *uW = a[7],
+            *uN = a[8], *uS = a[9], *uNE = a[10], *uNW = a[11], *uSE = a[12], *uSW = a[13];
+    vld16(co[0], oN + p);
+    vld16(co[1], oN + p - nx);
+    vld16(co[2], oE + p);
+    vld16(co[3], oE + p - 1);
+    vld16(co[4], oNE + p);
+    vld16(co[5], oNW + p);
+    vld16(co[6], oNW + p - nx + 1);
+    vld16(co[7], oNE + p - nx - 1);
+    vld16(f, ar.f + p);
+    vld16(D, ar.D + p);
+    const size_t q = p + nxy, mm = p - nxy;
+    T c[9][kV], w0[kV + 2], w1[kV + 2], w2[kV + 2];
+    vld16(c[0], uC + p);
+    vld16(c[1], uN + p);
+    vld16(c[2], uS + p);
+    vld16(c[3], uE + p);
+    vld16(c[4], uW + p);
+    vld16(c[5], uNE + p);
+    vld16(c[6], uNW + p);
+    vld16(c[7], uSE + p);
+    vld16(c[8], uSW + p);
+    vldw<T, kV>(w0, nbr + q - 1);
+    vldw<T, kV>(w1, nbr + q + nx - 1);
+    vldw<T, kV>(w2, nbr + q - nx - 1);
+#pragma unroll
+    for (int v = 0; v < kV; v++) {
+      T s = c[0][v] * w0[v + 1];
+      s += c[1][v] * w1[v + 1];
+      s += c[2][v] * w2[v + 1];
+      s += c[3][v] * w0[v + 2];
+      s += c[4][v] * w0[v];
+      s += c[5][v] * w1[v + 2];
+      s += c[6][v] * w1[v];
+      s += c[7][v] * w2[v + 2];
+      s += c[8][v] * w2[v];
+      u[v] = s;
+    }
+    vld16(c[0], uC + mm);
+    vld16(c[1], uS + mm + nx);
+    vld16(c[2], uN + mm - nx);
+    vld16(c[3], uW + mm + 1);
+    vld16(c[4], uE + mm - 1);
+    vld16(c[5], uSW + mm + nx + 1);
+    vld16(c[6], uSE + mm + nx - 1);
+    vld16(c[7], uNW + mm - nx + 1);
+    vld16(c[8], uNE + mm - nx - 1);
+    vldw<T, kV>(w0, nbr + mm - 1);
+    vldw<T, kV>(w1, nbr + mm + nx - 1);
+    vldw<T, kV>(w2, nbr + mm - nx - 1);
+#pragma unroll
+    for (int v = 0; v < kV; v++) {
+      T s = c[0][v] * w0[v + 1];
+      s += c[1][v] * w1[v + 1];
+      s += c[2][v] * w2[v + 1];
+      s += c[3][v] * w0[v + 2];
+      s += c[4][v] * w0[v];
+      s += c[5][v] * w1[v + 2];
+      s += c[6][v] * w1[v];
+      s += c[7][v] * w2[v + 2];
+      s += c[8][v] * w2[v];
+      d[v] = s;
+    }
+  }
+  // the plane's values: rows j0 - 2 .. j0 + 2m + 1 (rows outside the grid are
+  // not read by any point)
+  for (int r = threadIdx.x; r < (2 * m + 4) * nx; r += blockDim.x) {
+    const int jj = j0 - 2 + r / nx;
+    sx[r] = jj >= 0 && jj < ny ? src[kp + (size_t)(j0 - 2) * nx + r] : T(0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    if (act && g == s / 2) {
+      // colours in order: column parity 0 then 1 (adjoint: 1 then 0)
+      const int pi = (s & 1) ^ first;
+      const int e0 = (pi - ib) & 1;
+#pragma unroll
+      for (int h = 0; h < kV / 2; h++) {
+        auto pk = [&](const T(&v)[kV]) {
+          const T lo = v[2 * h], hi = v[2 * h + 1];
+          return e0 ? hi : lo;
+        };
+        const T* x = sx + e + e0 + 2 * h;
+        T o = pk(co[0]) * x[nx];
+        o += pk(co[1]) * x[-nx];
+        o += pk(co[2]) * x[1];
+        o += pk(co[3]) * x[-1];
+        o += pk(co[4]) * x[nx + 1];
+        o += pk(co[5]) * x[nx - 1];
+        o += pk(co[6]) * x[-nx + 1];
+        o += pk(co[7]) * x[-nx - 1];
+        sx[e + e0 + 2 * h] = (pk(f) + (o + pk(u) + pk(d))) / pk(D);
+      }
+    }
+    __syncthreads();
+  }
+  if (act && j >= j0 && j < j0 + 2 * m) {
+    T out[kV];
+#pragma unroll
+    for (int v = 0; v < kV; v++) out[v] = sx[e + v];
+    vst16(ar.z + p, out);
+  }
+}
+
 // ------------------------------------------------------------ bottom of the cycle
 // The last smoothed level and the coarsest one in one workgroup: restriction of
 // the residual above, the pre-smoothing sweeps from zero, the residual and its
@@ -452,7 +597,40 @@ void bottom_batch(hipStream_t s, const int above[3], const int level[3], const i
                                 coarsest[1], coarsest[2], B, nu);
 }
 
-int gsrb27_planes_tile(int nx, int ny, int nz) {
+// Whether a rows code (100 kV + m) fits a level: a run and its boundary points
+// in a row, the tile's runs in one workgroup.
+static bool rows_fit(int nx, int word, int code) {
+  const int kV = code / 100, m = code % 100;
+  if ((kV != 2 && !(kV == 4 && word == 4)) || m < 1 || nx < kV + 2) return false;
+  const int R = (nx - 2 + kV - 1) / kV;
+  return (2 * m + 1) * R <= 512 && (long)(2 * m + 4) * nx * word <= 64 * 1024;
+}
+
+// The rows form of a level, or 0.  Below rows of 40 points the square tiles
+// are faster (33^3: FP64 9.7 us a sweep against 10.8, FP32 9.0 against 9.8),
+// from 115 to 130 in FP64 the colour pairs no slower (129^3 94.2 against
+// 95.5).  FP32 takes 8-byte runs up to rows of 104 points (97^3 24.4 against
+// 25.4), 16-byte runs above (129^3 48.0 against 50.4).  m, the row pairs of a
+// workgroup, follows how its runs fill whole wavefronts and its tiles the 256
+// CUs: 3 up to 52 points and from 93 to 104 (49^3 FP64 m = 3 11.4, 4 13.3;
+// 97^3 41.8, 45.4), else 4 (65^3 m = 3 18.3, 4 15.4, 5 17.2; 81^3 30.3, 26.9,
+// 27.7), and 2 where 4 no longer fits or rows are longer than 144.
+static int rows_code(int nx, int word) {
+  if (nx < 40 || (word == 8 && nx > 114 && nx <= 130)) return 0;
+  const int kV = word == 4 && nx > 104 ? 4 : 2;
+  int m = kV == 4 ? (nx <= 144 ? 4 : 2) : (nx <= 52 || (nx > 92 && nx <= 104) ? 3 : 4);
+  while (m > 1 && !rows_fit(nx, word, 100 * kV + m)) m = m == 4 ? 2 : m - 1;
+  return rows_fit(nx, word, 100 * kV + m) ? 100 * kV + m : 0;
+}
+
+// The square tiles are for levels of at most 49^2 points a plane: larger planes
+// with short rows take the colour pairs.
+bool gsrb27_use_planes(int nx, int ny, int nz, int word) {
+  return nz >= 3 && (rows_code(nx, word) != 0 || (nx <= 49 && ny <= 49));
+}
+
+int gsrb27_planes_tile(int nx, int ny, int nz, int word) {
+  if (const int code = rows_code(nx, word)) return code;
   const long groups = (long)((nx - 2 + 15) / 16) * ((ny - 2 + 15) / 16) * ((nz - 2) / 2);
   return groups >= 64 ? 16 : 8;
 }
@@ -462,8 +640,11 @@ void gsrb27_planes_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<
                          int nu, int iadjoint, int tile) {
   check_batch(nb);
   if (nx < 3 || ny < 3 || nz < 3) return;
-  if (tile != 8 && tile != 16 && tile != 32) tile = gsrb27_planes_tile(nx, ny, nz);
+  constexpr int word = (int)sizeof(T);
+  if (tile != 8 && tile != 16 && tile != 32 && !(tile >= 100 && rows_fit(nx, word, tile)))
+    tile = gsrb27_planes_tile(nx, ny, nz, word);
   if (tile == 32) tile = 16;
+  const bool rows = tile >= 100;
   for (int it = 0; it < nu; it++) {
     // sweep it reads x (even it) or xs and writes the other one
     const int first = iadjoint ? 1 : 0;
@@ -477,6 +658,19 @@ void gsrb27_planes_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<
         T* in = (it & 1) ? c[b].xs : c[b].x;
         T* out = (it & 1) ? c[b].x : c[b].xs;
         B.v[b] = Args27<T>{to27(c[b].A), c[b].D, c[b].f, in, h == 0 ? in : out, out};
+      }
+      if (rows) {
+        const int kV = tile / 100, m = tile % 100, R = (nx - 2 + kV - 1) / kV;
+        const int nt = ((2 * m + 1) * R + 63) / 64 * 64;
+        const dim3 gr((unsigned)((ny - 2 + 2 * m - 1) / (2 * m)), (unsigned)nk, (unsigned)nb);
+        const size_t lds = (size_t)(2 * m + 4) * nx * sizeof(T);
+        if (kV == 4) {
+          if constexpr (sizeof(T) == 4)
+            k_gs27_rows<T, 4><<<gr, nt, lds, s>>>(nx, ny, nz, B, ck, iadjoint, R, m);
+        } else {
+          k_gs27_rows<T, 2><<<gr, nt, lds, s>>>(nx, ny, nz, B, ck, iadjoint, R, m);
+        }
+        continue;
       }
       const unsigned tiles = (unsigned)(((nx - 2 + tile - 1) / tile) * ((ny - 2 + tile - 1) / tile));
       const dim3 g(tiles, (unsigned)nk, (unsigned)nb);

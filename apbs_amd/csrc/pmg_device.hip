@@ -269,26 +269,6 @@ __global__ void __launch_bounds__(kNT)
 // row and runs near the grid edge may overlap (they then write the same
 // values).  The boundary columns 0 and nx-1 come from the x(p-1) / x(p+1)
 // vectors of the runs beside them.
-template <class T, int N>
-__device__ __forceinline__ void vld16(T (&v)[N], const T* p) {
-  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
-  typedef T vT __attribute__((ext_vector_type(N)));
-  vT a;
-  __builtin_memcpy(&a, p, sizeof(T) * N);
-#pragma unroll
-  for (int i = 0; i < N; i++) v[i] = a[i];
-}
-
-template <class T, int N>
-__device__ __forceinline__ void vst16(T* p, const T (&v)[N]) {
-  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
-  typedef T vT __attribute__((ext_vector_type(N)));
-  vT a;
-#pragma unroll
-  for (int i = 0; i < N; i++) a[i] = v[i];
-  __builtin_memcpy(p, &a, sizeof(T) * N);
-}
-
 template <class T, int kTY, int kKC, int kTX, int kNT, bool kZeroX>
 __device__ __forceinline__ void vfused_body(int nx, int ny, int nz, int tile,
                                             const T* __restrict__ oE, const T* __restrict__ oN,
@@ -596,21 +576,6 @@ __global__ void __launch_bounds__(kBlock)
 // The last run of a row is moved inwards so that every load stays inside its
 // row; overlapping runs compute and write the same values.  part27's terms in
 // its order, so the results are the scalar form's bit for bit.
-template <class T, int N>
-__device__ __forceinline__ void vldw(T (&w)[N + 2], const T* p) {
-  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
-  typedef T vT __attribute__((ext_vector_type(N)));
-  typedef T v2 __attribute__((ext_vector_type(2)));
-  vT a;
-  v2 b;
-  __builtin_memcpy(&a, p, sizeof(T) * N);
-  __builtin_memcpy(&b, p + N, 2 * sizeof(T));
-#pragma unroll
-  for (int i = 0; i < N; i++) w[i] = a[i];
-  w[N] = b[0];
-  w[N + 1] = b[1];
-}
-
 // R runs per row, RB rows per workgroup; LDS holds RB rows of new A values.
 template <class T, int kV>
 __global__ void __launch_bounds__(kBlock)
@@ -2490,8 +2455,6 @@ void gsrb27_pairs(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const 
   const LevelArgs<T> c{A, D, fc, x, nullptr, nullptr};
   gsrb27_pairs_batch<T>(s, nx, ny, nz, &c, 1, nu, iadjoint);
 }
-
-bool gsrb27_use_planes(int nx, int ny, int nz) { return nx <= 49 && ny <= 49 && nz >= 3; }
 
 bool gsrb27_use_pairs(int nx) { return nx >= 3 && nx <= 130; }
 

@@ -29,6 +29,43 @@ inline dim3 grid_interior(int nx, int ny, int nz) {
   return dim3((unsigned)((cnt + kBlock - 1) / kBlock), (unsigned)(nz - 2), 1);
 }
 
+// Vectors of 16 or 8 bytes at any element alignment, and windows of N + 2
+// elements.
+template <class T, int N>
+__device__ __forceinline__ void vld16(T (&v)[N], const T* p) {
+  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
+  typedef T vT __attribute__((ext_vector_type(N)));
+  vT a;
+  __builtin_memcpy(&a, p, sizeof(T) * N);
+#pragma unroll
+  for (int i = 0; i < N; i++) v[i] = a[i];
+}
+
+template <class T, int N>
+__device__ __forceinline__ void vst16(T* p, const T (&v)[N]) {
+  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
+  typedef T vT __attribute__((ext_vector_type(N)));
+  vT a;
+#pragma unroll
+  for (int i = 0; i < N; i++) a[i] = v[i];
+  __builtin_memcpy(p, &a, sizeof(T) * N);
+}
+
+template <class T, int N>
+__device__ __forceinline__ void vldw(T (&w)[N + 2], const T* p) {
+  static_assert(sizeof(T) * N == 16 || sizeof(T) * N == 8, "8- or 16-byte vectors");
+  typedef T vT __attribute__((ext_vector_type(N)));
+  typedef T v2 __attribute__((ext_vector_type(2)));
+  vT a;
+  v2 b;
+  __builtin_memcpy(&a, p, sizeof(T) * N);
+  __builtin_memcpy(&b, p + N, 2 * sizeof(T));
+#pragma unroll
+  for (int i = 0; i < N; i++) w[i] = a[i];
+  w[N] = b[0];
+  w[N + 1] = b[1];
+}
+
 // ----------------------------------------------------------------- 27-point
 template <class T>
 struct P27 {

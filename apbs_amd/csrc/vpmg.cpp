@@ -1382,7 +1382,7 @@ void vcycle_batch(PmgDev* const* ds, CycleArgs<T>* cs, int n) {
   };
   auto coarse_smooth = [&](int l, int adj) {
     level(l, false);
-    if (d0->smoother27 == 0 && pmg::gsrb27_use_planes(L[l].nx, L[l].ny, L[l].nz))
+    if (d0->smoother27 == 0 && pmg::gsrb27_use_planes(L[l].nx, L[l].ny, L[l].nz, (int)sizeof(T)))
       pmg::gsrb27_planes_batch<T>(s, L[l].nx, L[l].ny, L[l].nz, la, n, 2, adj);
     else if (d0->smoother27 == 0 && pmg::gsrb27_use_pairs(L[l].nx))
       pmg::gsrb27_pairs_batch<T>(s, L[l].nx, L[l].ny, L[l].nz, la, n, 2, adj);

@@ -93,3 +93,58 @@ def test_bottom_of_the_cycle_bitwise(dims, npbe, precision, monkeypatch):
     (ea, ua, sa), (eb, ub, sb) = out
     assert (sa["iters"], sa["inner"], sa["nlev"]) == (sb["iters"], sb["inner"], sb["nlev"])
     assert ea == eb and np.array_equal(ua, ub)
+
+
+def _level(n3, seed):
+    rng = np.random.default_rng(seed)
+    nx, ny, nz = n3
+    n = nx * ny * nz
+    a = np.zeros((14, nz, ny, nx))
+    for s in range(14):
+        a[s, 1:-1, 1:-1, 1:-1] = rng.uniform(0.1, 1.0, (nz - 2, ny - 2, nx - 2))
+    a[0, 1:-1, 1:-1, 1:-1] = rng.uniform(18.0, 36.0, (nz - 2, ny - 2, nx - 2))
+    x = np.zeros((nz, ny, nx))
+    x[1:-1, 1:-1, 1:-1] = rng.normal(size=(nz - 2, ny - 2, nx - 2))
+    return np.ascontiguousarray(a.reshape(-1)), rng.uniform(0, 1, n), rng.normal(size=n), \
+        x.reshape(-1)
+
+
+@pytest.mark.parametrize("n3", [(17, 17, 17), (9, 11, 13), (45, 43, 41), (4, 5, 4), (70, 21, 6),
+                                (81, 81, 9), (131, 8, 7), (177, 13, 5)])
+@pytest.mark.parametrize("code", [201, 202, 203, 205, 210])
+def test_row_tiles_bitwise(L, n3, code):
+    """The whole-row plane sweep (code 100 kV + m: runs of kV points, 2m rows
+    a workgroup) against the oracle's 8-colour sweep, bit for bit: partial
+    tiles, rows of 2 to 175 points, odd ends of the last run, both orders and
+    odd and even sweep counts.  Codes that do not fit a row take the square
+    tiles."""
+    nx, ny, nz = n3
+    a, cc, fc, x0 = _level(n3, sum(n3) + code)
+    O = od.lib()
+    for adj in (0, 1):
+        for nu in (2, 3):
+            xg, xo = x0.copy(), x0.copy()
+            L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj, code)
+            O.orc_gsrb(nx, ny, nz, 27, P(a), P(cc), P(fc), P(xo), nu, adj, 1)
+            assert np.array_equal(xg, xo), (adj, nu)
+
+
+@pytest.mark.parametrize("n3", [(17, 17, 17), (9, 11, 13), (45, 43, 41), (6, 5, 4), (81, 81, 9),
+                                (131, 8, 7), (178, 13, 5)])
+@pytest.mark.parametrize("code", [203, 401, 402, 404, 405, 410])
+def test_row_tiles_fp32_bitwise(L, n3, code):
+    """The FP32 rows forms (8- and 16-byte runs) against one launch per colour."""
+    fp = ctypes.POINTER(ctypes.c_float)
+    nx, ny, nz = n3
+    a, cc, fc, x0 = (v.astype(np.float32) for v in _level(n3, sum(n3) + code))
+    D = a[:nx * ny * nz] + cc
+    for adj in (0, 1):
+        for nu in (2, 3):
+            out = []
+            for mode in (code, 0):
+                x = x0.copy()
+                assert L.pmgtest_gsrb27_32(nx, ny, nz, a.ctypes.data_as(fp), D.ctypes.data_as(fp),
+                                           fc.ctypes.data_as(fp), x.ctypes.data_as(fp), nu, adj,
+                                           mode) == 1
+                out.append(x)
+            assert np.array_equal(out[0], out[1]), (adj, nu)
