@@ -13,7 +13,8 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libapbs_pmg.so")
-SOURCES = ["pmg_device.hip", "coarse_device.hip", "fill_device.hip", "pool.cpp", "vpmg.cpp", "server.cpp", "testhooks.cpp"]
+SOURCES = ["pmg_device.hip", "sweep_device.hip", "coarse_device.hip", "dense_device.hip",
+           "fill_device.hip", "pool.cpp", "vpmg.cpp", "server.cpp", "testhooks.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "--offload-arch=gfx950", "-ffp-contract=off", "-fPIC", "-std=c++17",
@@ -44,7 +45,7 @@ def build(verbose=False):
             cmd = [HIPCC] + FLAGS + ["-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj]
         cmds.append(cmd)
         objs.append(obj)
-    jobs = max(1, min(len(cmds), int(os.environ.get("MAX_JOBS", "6"))))
+    jobs = max(1, min(len(cmds), int(os.environ.get("MAX_JOBS", "8"))))
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         for out in ex.map(_run, cmds):
             if verbose and out:

@@ -58,400 +58,6 @@ __global__ void __launch_bounds__(kBlock)
   x[p] = acc7(fc[p], oE, oN, uC, x, p, nx, nxy) / D[p];
 }
 
-// One complete red-black sweep, out of place: xo = sweep(xi).  In the 7-point
-// stencil every neighbour of a point has the other colour, so the first colour
-// F reads only old values of the second colour S, and S reads only new F
-// values.  A workgroup owns a TX x TY tile of (i, j) and marches over a chunk
-// of k planes: the new F values of plane k+1 (tile plus a one-point halo) go
-// to a three-plane LDS ring, then the S points of plane k are updated from the
-// ring and the whole tile row of plane k is written.  Each value is the
-// in-place sweep's value bit for bit (same terms, same order, no FMA).
-// Points outside the interior are not written.
-constexpr int kFT = 256, kXCD = 8;
-
-// kTX columns (even), kTY rows and kKC planes per workgroup of kNT threads.
-// The arrays of one calculation in a fused-sweep launch.
-template <class T>
-struct SweepArgs {
-  const T *oE, *oN, *uC, *D, *fc, *xi;
-  T* xo;
-};
-
-// kZeroX: xi is zero everywhere (a solve of the correction equation from a
-// zero start); its values are not read, and the sweep's values are those of
-// reading the zeros.
-template <class T, int kTY, int kKC, int kTX, int kNT, bool kZeroX>
-__device__ __forceinline__ void fused_body(int nx, int ny, int nz, int tile,
-                                           const T* __restrict__ oE, const T* __restrict__ oN,
-                                           const T* __restrict__ uC, const T* __restrict__ D,
-                                           const T* __restrict__ fc, const T* __restrict__ xi,
-                                           T* __restrict__ xo, int first) {
-  constexpr int RX = kTX + 2, RY = kTY + 2, RN = RX * RY;
-  constexpr int FPR = RX / 2, FN = FPR * RY;  // F points per region row / per plane
-  __shared__ T ring[3][RN];
-  const int tid = threadIdx.x;
-  const int nbx = (nx - 2 + kTX - 1) / kTX, nby = (ny - 2 + kTY - 1) / kTY;
-  const int i0 = 1 + (tile % nbx) * kTX, j0 = 1 + ((tile / nbx) % nby) * kTY;
-  const int k0 = 1 + (tile / (nbx * nby)) * kKC;
-  const int k1 = min(k0 + kKC, nz - 1);  // planes k0 .. k1-1
-  const size_t nxy = (size_t)nx * ny;
-  const int F = first;                   // parity of the first colour
-
-  // New F values of plane kk over the tile and its halo, one thread per F
-  // point in kFR rounds.  loadF issues every round's loads at once into
-  // registers; storeF computes the values (acc7's terms and order) into the
-  // plane's LDS slot.
-  constexpr int kFR = (FN + kNT - 1) / kNT;
-  struct FRegs {
-    T v[kFR][14];
-    int slot[kFR];  // LDS index in the ring plane
-    int kind[kFR];  // 0 nothing, 1 boundary copy, 2 interior update
-  };
-  auto loadF = [&](int kk, FRegs& R) {
-#pragma unroll
-    for (int u = 0; u < kFR; u++) {
-      R.kind[u] = 0;
-      const int f = tid + u * kNT;
-      if (f >= FN) continue;
-      const int row = f / FPR, c = f % FPR;
-      const int j = j0 - 1 + row;
-      const int ib = i0 - 1;
-      const int i = ib + ((F - ib - j - kk) & 1) + 2 * c;
-      if (i > nx - 1 || j > ny - 1) continue;
-      const size_t p = ((size_t)kk * ny + j) * nx + i;
-      R.slot[u] = row * RX + (i - ib);
-      if (i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2 && kk >= 1 && kk <= nz - 2) {
-        R.kind[u] = 2;
-        R.v[u][0] = fc[p];
-        R.v[u][1] = oN[p];
-        R.v[u][2] = kZeroX ? T(0) : xi[p + nx];
-        R.v[u][3] = oN[p - nx];
-        R.v[u][4] = kZeroX ? T(0) : xi[p - nx];
-        R.v[u][5] = oE[p];
-        R.v[u][6] = kZeroX ? T(0) : xi[p + 1];
-        R.v[u][7] = oE[p - 1];
-        R.v[u][8] = kZeroX ? T(0) : xi[p - 1];
-        R.v[u][9] = uC[p - nxy];
-        R.v[u][10] = kZeroX ? T(0) : xi[p - nxy];
-        R.v[u][11] = uC[p];
-        R.v[u][12] = kZeroX ? T(0) : xi[p + nxy];
-        R.v[u][13] = D[p];
-      } else {
-        R.kind[u] = 1;
-        R.v[u][0] = kZeroX ? T(0) : xi[p];
-      }
-    }
-  };
-  auto storeF = [&](int kk, const FRegs& R) {
-    T* r = ring[kk % 3];
-#pragma unroll
-    for (int u = 0; u < kFR; u++) {
-      if (R.kind[u] == 2) {
-        T acc = R.v[u][0];
-        acc += R.v[u][1] * R.v[u][2];
-        acc += R.v[u][3] * R.v[u][4];
-        acc += R.v[u][5] * R.v[u][6];
-        acc += R.v[u][7] * R.v[u][8];
-        acc += R.v[u][9] * R.v[u][10];
-        acc += R.v[u][11] * R.v[u][12];
-        r[R.slot[u]] = acc / R.v[u][13];
-      } else if (R.kind[u] == 1) {
-        r[R.slot[u]] = R.v[u][0];
-      }
-    }
-  };
-
-  // The S step: thread u owns the (i, i+1) pair u % 32 of tile row u / 32 (one
-  // F and one S point).  The eight operands of the S point of plane kk are
-  // loaded one plane ahead, together with stageF(kk), so each coefficient
-  // line is fetched once for both colours while it is still cached.
-  constexpr int kSP = (kTX / 2 * kTY + kNT - 1) / kNT;
-  T cur[kSP][8], nxt[kSP][8];
-  auto loadS = [&](int kk, T (&r)[kSP][8]) {
-#pragma unroll
-    for (int u = 0; u < kSP; u++) {
-      const int sidx = tid + u * kNT;
-      if (sidx >= kTX / 2 * kTY) continue;
-      const int j = j0 + sidx / (kTX / 2);
-      const int is = i0 + 2 * (sidx % (kTX / 2)) + ((1 - F - i0 - j - kk) & 1);
-      if (is > nx - 2 || j > ny - 2) continue;
-      const size_t p = ((size_t)kk * ny + j) * nx + is;
-      r[u][0] = fc[p];
-      r[u][1] = oN[p];
-      r[u][2] = oN[p - nx];
-      r[u][3] = oE[p];
-      r[u][4] = oE[p - 1];
-      r[u][5] = uC[p - nxy];
-      r[u][6] = uC[p];
-      r[u][7] = D[p];
-    }
-  };
-
-  FRegs fr;
-  loadS(k0, cur);
-  loadF(k0 - 1, fr);
-  storeF(k0 - 1, fr);
-  loadF(k0, fr);
-  storeF(k0, fr);
-  loadF(k0 + 1, fr);
-  for (int k = k0; k < k1; k++) {
-    // F(k+1) from registers loaded one step earlier; the loads of F(k+2) and
-    // of S(k+1)'s operands are in flight while S(k) is computed
-    if (k + 1 < k1) loadS(k + 1, nxt);
-    storeF(k + 1, fr);
-    __syncthreads();
-    if (k + 1 < k1) loadF(k + 2, fr);
-    const T* rm = ring[(k - 1) % 3];
-    const T* r0 = ring[k % 3];
-    const T* rp = ring[(k + 1) % 3];
-#pragma unroll
-    for (int u = 0; u < kSP; u++) {
-      const int sidx = tid + u * kNT;
-      if (sidx >= kTX / 2 * kTY) continue;
-      const int jj = sidx / (kTX / 2);
-      const int j = j0 + jj;
-      if (j > ny - 2) continue;
-      const int ia = i0 + 2 * (sidx % (kTX / 2));
-      const int is = ia + ((1 - F - i0 - j - k) & 1);
-      const int iF = ia + ((F - i0 - j - k) & 1);
-      const size_t row = ((size_t)k * ny + j) * nx;
-      if (iF <= nx - 2) xo[row + iF] = r0[(jj + 1) * RX + (iF - i0 + 1)];
-      if (is <= nx - 2) {
-        const int e = (jj + 1) * RX + (is - i0 + 1);
-        T acc = cur[u][0];
-        acc += cur[u][1] * r0[e + RX];
-        acc += cur[u][2] * r0[e - RX];
-        acc += cur[u][3] * r0[e + 1];
-        acc += cur[u][4] * r0[e - 1];
-        acc += cur[u][5] * rm[e];
-        acc += cur[u][6] * rp[e];
-        xo[row + is] = acc / cur[u][7];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kSP; u++)
-#pragma unroll
-      for (int w = 0; w < 8; w++) cur[u][w] = nxt[u][w];
-  }
-}
-
-// Workgroups are dealt round-robin to the 8 XCDs: XCD x gets the (calculation,
-// tile) items [x*per, (x+1)*per) in calculation-major, z-major order, so tiles
-// that share halo rows and planes share an L2.
-template <class T, int kTY, int kKC, int kTX, int kNT, bool kZeroX = false>
-__global__ void __launch_bounds__(kNT)
-    k_gsrb7_fused(int nx, int ny, int nz, Batch<SweepArgs<T>> B, int nreq, int first) {
-  const int nbx = (nx - 2 + kTX - 1) / kTX, nby = (ny - 2 + kTY - 1) / kTY;
-  const int nb = nbx * nby * ((nz - 2 + kKC - 1) / kKC);
-  const int total = nb * nreq;
-  const int per = (total + kXCD - 1) / kXCD;
-  const int item = (blockIdx.x % kXCD) * per + blockIdx.x / kXCD;
-  if (item >= total) return;
-  const SweepArgs<T>& a = B.v[item / nb];
-  fused_body<T, kTY, kKC, kTX, kNT, kZeroX>(nx, ny, nz, item % nb, a.oE, a.oN, a.uC, a.D, a.fc,
-                                            a.xi, a.xo, first);
-}
-
-// The vector form of the fused sweep.  The scalar form above loads one
-// 4- or 8-byte word per lane and operand with the lanes two words apart, so
-// the texture addresser (four lanes per clock) and the L1 limit it long
-// before memory does.  Here a lane owns a run of kV consecutive elements of
-// one row (16 bytes: 4 floats or 2 doubles, both colours) and loads every
-// operand as a 16-byte vector; the coefficient vectors that the F step of
-// plane k loads are the S step's operands of plane k one step later, so the
-// S step loads nothing from memory.  Values and their order are the scalar
-// form's (acc7's terms, no FMA).
-//
-// Lanes: region row r (0 .. kTY+1, row j = j0-1+r) and run c of that row
-// (columns i0-1+kV*c ..); a run is moved inwards to [1, nx-1-kV] when it would
-// cross the first or last interior column, so every load stays inside the
-// row and runs near the grid edge may overlap (they then write the same
-// values).  The boundary columns 0 and nx-1 come from the x(p-1) / x(p+1)
-// vectors of the runs beside them.
-template <class T, int kTY, int kKC, int kTX, int kNT, bool kZeroX>
-__device__ __forceinline__ void vfused_body(int nx, int ny, int nz, int tile,
-                                            const T* __restrict__ oE, const T* __restrict__ oN,
-                                            const T* __restrict__ uC, const T* __restrict__ D,
-                                            const T* __restrict__ fc, const T* __restrict__ xi,
-                                            T* __restrict__ xo, int first) {
-  constexpr int kV = 16 / (int)sizeof(T), kH = kV / 2;
-  constexpr int RX = kTX + 2, RY = kTY + 2, RN = RX * RY;
-  constexpr int NSEG = (RX + kV - 1) / kV;
-  static_assert(RY * NSEG <= kNT, "one lane per run");
-  __shared__ T ring[3][RN];
-  const int tid = threadIdx.x;
-  const int nbx = (nx - 2 + kTX - 1) / kTX, nby = (ny - 2 + kTY - 1) / kTY;
-  const int i0 = 1 + (tile % nbx) * kTX, j0 = 1 + ((tile / nbx) % nby) * kTY;
-  const int k0 = 1 + (tile / (nbx * nby)) * kKC;
-  const int k1 = min(k0 + kKC, nz - 1);  // planes k0 .. k1-1
-  const size_t nxy = (size_t)nx * ny;
-  const int F = first;
-
-  const bool lane = tid < RY * NSEG;
-  const int r = lane ? tid / NSEG : 0, c = lane ? tid % NSEG : 0;
-  const int j = j0 - 1 + r;
-  const bool rowin = lane && j <= ny - 1;
-  const bool rowint = j >= 1 && j <= ny - 2;
-  const bool srow = lane && r >= 1 && r <= kTY && j <= ny - 2;
-  const int jr = min(j, ny - 1), jc = min(max(j, 1), ny - 2);
-  const int is = i0 - 1 + kV * c;
-  const int ib = min(max(is, 1), nx - 1 - kV);
-  const int chi = min(i0 + kTX - 1, nx - 2);  // last column this tile writes
-  // a lane holds, per plane: fc, oN, oN(-nx), oE, oE(-1), uC(-nxy), uC, D and
-  // x(+nx), x(-nx), x(+1), x(-1), x(+nxy), x(-nxy), each at columns ib ..
-  struct Set {
-    T a[8][kV];
-    T x[6][kV];
-  };
-  auto load = [&](int kk, Set& S) {
-    const int kc = min(max(kk, 1), nz - 2);
-    const size_t q = ((size_t)kc * ny + jc) * nx + ib;   // interior row / plane
-    const size_t pr = ((size_t)kk * ny + jr) * nx + ib;  // the lane's own row and plane
-    vld16(S.a[0], fc + q);
-    vld16(S.a[1], oN + q);
-    vld16(S.a[2], oN + q - nx);
-    vld16(S.a[3], oE + q);
-    vld16(S.a[4], oE + q - 1);
-    vld16(S.a[5], uC + q - nxy);
-    vld16(S.a[6], uC + q);
-    vld16(S.a[7], D + q);
-    if (!kZeroX) {
-      vld16(S.x[0], xi + q + nx);
-      vld16(S.x[1], xi + q - nx);
-      vld16(S.x[2], xi + pr + 1);
-      vld16(S.x[3], xi + pr - 1);
-      vld16(S.x[4], xi + q + nxy);
-      vld16(S.x[5], xi + q - nxy);
-    } else {
-#pragma unroll
-      for (int v = 0; v < 6; v++)
-#pragma unroll
-        for (int e = 0; e < kV; e++) S.x[v][e] = T(0);
-    }
-  };
-  // New F values of plane kk into the ring (and fv: the lane's F elements
-  // e0, e0+2, ..., with e0 the first element of F colour)
-  auto stageF = [&](int kk, const Set& S, T (&fv)[kH]) {
-    if (!rowin) return;
-    T* rg = ring[kk % 3] + r * RX - (i0 - 1);
-    const bool inner = rowint && kk >= 1 && kk <= nz - 2;
-    const int e0 = (F - ib - j - kk) & 1;
-#pragma unroll
-    for (int m = 0; m < kH; m++) {
-      // (selects between values, not addresses, so the vectors stay in registers)
-      auto pk = [&](const T(&v)[kV]) {
-        const T lo = v[2 * m], hi = v[2 * m + 1];
-        return e0 ? hi : lo;
-      };
-      T val;
-      if (inner) {
-        T acc = pk(S.a[0]);
-        acc += pk(S.a[1]) * pk(S.x[0]);
-        acc += pk(S.a[2]) * pk(S.x[1]);
-        acc += pk(S.a[3]) * pk(S.x[2]);
-        acc += pk(S.a[4]) * pk(S.x[3]);
-        acc += pk(S.a[5]) * pk(S.x[5]);
-        acc += pk(S.a[6]) * pk(S.x[4]);
-        val = acc / pk(S.a[7]);
-      } else {
-        // a boundary row or plane keeps its values: x at element e is
-        // x(p-1)[e+1], or x(p+1)[e-1] for the last element
-        const T xe = 2 * m + 2 < kV ? S.x[3][(2 * m + 2) % kV] : S.x[2][2 * m];
-        const T xo1 = S.x[3][2 * m + 1];
-        val = e0 ? xe : xo1;
-      }
-      fv[m] = val;
-      const int col = ib + e0 + 2 * m;
-      if (col >= i0 - 1 && col <= i0 + kTX) rg[col] = val;
-    }
-    // boundary columns 0 and nx-1 when they are in the region and of F colour
-    if (is <= 0 && ((j + kk) & 1) == F) rg[0] = S.x[3][0];
-    if (ib == nx - 1 - kV && nx - 1 <= i0 + kTX && ((nx - 1 + j + kk) & 1) == F)
-      rg[nx - 1] = S.x[2][kV - 1];
-  };
-  // S values of plane k from the coefficient vectors of plane k and the ring;
-  // both colours of the lane's tile columns are written
-  auto stageS = [&](int k, const Set& S, const T(&fv)[kH]) {
-    if (!srow) return;
-    const int off = r * RX - (i0 - 1);
-    const T* rm = ring[(k - 1) % 3] + off;
-    const T* r0 = ring[k % 3] + off;
-    const T* rp = ring[(k + 1) % 3] + off;
-    const int e0 = (F - ib - j - k) & 1;
-    T* row = xo + ((size_t)k * ny + j) * nx;
-    // a run wholly inside the tile's columns is written with one 16-byte
-    // store; the runs at the tile's edges element by element
-    const bool full = ib >= i0 && ib + kV - 1 <= chi;
-    T out[kV];
-#pragma unroll
-    for (int m = 0; m < kH; m++) {
-      const int cf = ib + e0 + 2 * m;
-      const int cs = ib + (1 - e0) + 2 * m;
-      T sv = T(0);
-      if (full || (cs >= i0 && cs <= chi)) {
-        auto pk = [&](const T(&v)[kV]) {
-          const T lo = v[2 * m], hi = v[2 * m + 1];
-          return e0 ? lo : hi;
-        };
-        T acc = pk(S.a[0]);
-        acc += pk(S.a[1]) * r0[cs + RX];
-        acc += pk(S.a[2]) * r0[cs - RX];
-        acc += pk(S.a[3]) * r0[cs + 1];
-        acc += pk(S.a[4]) * r0[cs - 1];
-        acc += pk(S.a[5]) * rm[cs];
-        acc += pk(S.a[6]) * rp[cs];
-        sv = acc / pk(S.a[7]);
-      }
-      const T f = fv[m];
-      out[2 * m] = e0 ? sv : f;
-      out[2 * m + 1] = e0 ? f : sv;
-      if (!full) {
-        if (cf >= i0 && cf <= chi) row[cf] = f;
-        if (cs >= i0 && cs <= chi) row[cs] = sv;
-      }
-    }
-    if (full) vst16(row + ib, out);
-  };
-  // one plane step: F(k+1) from n (loaded one step earlier), then S(k) from
-  // c, whose registers then take the loads of plane k+2
-  auto step = [&](int k, Set& cur, T(&fc_)[kH], const Set& nxt, T(&fn)[kH]) {
-    stageF(k + 1, nxt, fn);
-    __syncthreads();
-    stageS(k, cur, fc_);
-    if (k + 2 <= k1) load(k + 2, cur);
-    __syncthreads();
-  };
-
-  Set A, B;
-  T fa[kH], fb[kH];
-  load(k0 - 1, A);
-  stageF(k0 - 1, A, fa);
-  load(k0, A);
-  stageF(k0, A, fa);
-  load(k0 + 1, B);
-  int k = k0;
-  for (; k + 1 < k1; k += 2) {
-    step(k, A, fa, B, fb);
-    step(k + 1, B, fb, A, fa);
-  }
-  if (k < k1) step(k, A, fa, B, fb);
-}
-
-template <class T, int kTY, int kKC, int kTX, int kNT, bool kZeroX = false>
-__global__ void __launch_bounds__(kNT)
-    k_gsrb7_vfused(int nx, int ny, int nz, Batch<SweepArgs<T>> B, int nreq, int first) {
-  const int nbx = (nx - 2 + kTX - 1) / kTX, nby = (ny - 2 + kTY - 1) / kTY;
-  const int nb = nbx * nby * ((nz - 2 + kKC - 1) / kKC);
-  const int total = nb * nreq;
-  const int per = (total + kXCD - 1) / kXCD;
-  const int item = (blockIdx.x % kXCD) * per + blockIdx.x / kXCD;
-  if (item >= total) return;
-  const SweepArgs<T>& a = B.v[item / nb];
-  vfused_body<T, kTY, kKC, kTX, kNT, kZeroX>(nx, ny, nz, item % nb, a.oE, a.oN, a.uC, a.D, a.fc,
-                                             a.xi, a.xo, first);
-}
-
 // One colour of the 8-colour sweep: 0-based parities (c&1, (c>>1)&1, (c>>2)&1).
 // Latency-bound on the small coarse levels: up to 128 VGPRs, so that all 54
 // operands of a point are in flight at once.
@@ -1793,330 +1399,6 @@ __global__ void __launch_bounds__(kBlock)
   out.a[s][pc] = (s == 0) ? sum : -sum;
 }
 
-// ------------------------------------------------------------ dense coarse
-// kAsmRows rows per workgroup, 16 lanes per row: the rows are cleared with
-// consecutive stores, then each lane writes up to two of the row's 26
-// couplings (forward ones from this point's coefficients, backward ones from
-// the neighbour's) and lane 0 the diagonal.
-constexpr int kAsmRows = kBlock / 16;
-
-__global__ void __launch_bounds__(kBlock)
-    k_dense_assemble(int nx, int ny, int nz, Batch<InvertArgs> B, int N) {
-  const Ops<double>& A = B.v[blockIdx.y].A;
-  const double* D = B.v[blockIdx.y].D;
-  double* M = B.v[blockIdx.y].M;
-  const int r0 = blockIdx.x * kAsmRows, rows = min(kAsmRows, N - r0);
-  double* Mb = M + (size_t)r0 * N;
-  for (int t = threadIdx.x; t < rows * N; t += kBlock) Mb[t] = 0.0;
-  __syncthreads();
-  const int r = r0 + threadIdx.x / 16, lane = threadIdx.x % 16;
-  if (r >= N) return;
-  const int ni = nx - 2, nj = ny - 2;
-  const int i = r % ni + 1, j = (r / ni) % nj + 1, k = r / (ni * nj) + 1;
-  if (lane == 0) M[(size_t)r * N + r] = D[IX(i, j, k, nx, ny)];
-  for (int e = lane; e < 26; e += 16) {
-    const int s = 1 + e / 2, dir = (e & 1) ? 1 : -1;
-    const int i2 = i + dir * c_fwd[s][0], j2 = j + dir * c_fwd[s][1], k2 = k + dir * c_fwd[s][2];
-    if (i2 < 1 || i2 > nx - 2 || j2 < 1 || j2 > ny - 2 || k2 < 1 || k2 > nz - 2) continue;
-    const int c = (i2 - 1) + ni * ((j2 - 1) + nj * (k2 - 1));
-    const double v = dir > 0 ? -A.a[s][IX(i, j, k, nx, ny)] : -A.a[s][IX(i2, j2, k2, nx, ny)];
-    M[(size_t)r * N + c] = v;
-  }
-}
-
-// A pivot that is not positive and finite means the operator is not positive
-// definite (Vdpbfa's leading-minor test, mlinpckd.c:194-233): the 1-based
-// index of the first one goes to *flag (host-mapped memory) with a
-// system-scope store; a flag that an earlier block raised is kept.
-__device__ inline void flag_pivot(int k, double* flag) {
-  if (flag && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0.0)
-    __hip_atomic_store(flag, (double)(k + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// The Gauss-Jordan inverse in one workgroup with the matrix held in LDS
-// (N*N + 2N doubles, N <= 89).  Per pivot: stage column k and the scaled
-// pivot row (v / piv), then update every element; each thread's (i, j) pairs
-// are decoded once.
-constexpr int kInvPer = 8;  // elements per thread: 89 * 89 <= 8 * 1024
-
-__global__ void __launch_bounds__(1024) k_dense_invert_lds(Batch<InvertArgs> B, int N) {
-  double* Mg = B.v[blockIdx.x].M;
-  double* flag = B.v[blockIdx.x].flag;
-  extern __shared__ double sm[];
-  double* M = sm;
-  double* col = sm + (size_t)N * N;
-  double* prow = col + N;
-  const int tid = threadIdx.x;
-  int ei[kInvPer], ej[kInvPer];
-  int ne = 0;
-  for (int e = tid; e < N * N && ne < kInvPer; e += 1024, ne++) {
-    ei[ne] = e / N;
-    ej[ne] = e - ei[ne] * N;
-  }
-  for (int e = tid; e < N * N; e += 1024) M[e] = Mg[e];
-  __syncthreads();
-  int bad = -1;
-  for (int k = 0; k < N; k++) {
-    if (tid == 0 && bad < 0 && !(M[k * N + k] > 0.0 && M[k * N + k] <= DBL_MAX)) bad = k;
-    if (tid < N) {
-      col[tid] = M[tid * N + k];
-      const double v = (tid == k) ? 1.0 : M[k * N + tid];
-      prow[tid] = v / M[k * N + k];
-    }
-    __syncthreads();
-    for (int q = 0; q < ne; q++) {
-      const int i = ei[q], j = ej[q];
-      if (i == k) {
-        M[i * N + j] = prow[j];
-      } else {
-        const double base = (j == k) ? 0.0 : M[i * N + j];
-        M[i * N + j] = base - col[i] * prow[j];
-      }
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < N * N; e += 1024) Mg[e] = M[e];
-  if (tid == 0 && bad >= 0) flag_pivot(bad, flag);
-}
-
-// The same Gauss-Jordan inverse for N <= 64 with the matrix in registers:
-// thread t holds 16 entries of row t / 4.  Each pivot step publishes the
-// pivot row and column through double-buffered LDS (one barrier per pivot)
-// and scales the pivot row by the pivot's reciprocal.  Reads N rows of src
-// (leading dimension lds), writes dst (ldd; rows and columns up to nout, zero
-// past N); pivot p is reported as base + p.
-__device__ __forceinline__ void invert_reg_body(const double* src, size_t lds, double* dst,
-                                                size_t ldd, int N, int nout, int base,
-                                                double* flag) {
-  __shared__ double colb[2][64], rowb[2][64];
-  const int t = threadIdx.x, r = t >> 2, cb = t & 3, c0 = cb * 16;
-  double m[16];
-#pragma unroll
-  for (int q = 0; q < 16; q++)
-    m[q] = (r < N && c0 + q < N) ? src[(size_t)r * lds + c0 + q] : 0.0;
-  int bad = -1;
-  for (int k = 0; k < N; k++) {
-    const int b = k & 1;
-    if (r < N && (k >> 4) == cb) {
-      double v = 0.0;
-#pragma unroll
-      for (int q = 0; q < 16; q++)
-        if (q == (k & 15)) v = m[q];
-      colb[b][r] = v;
-    }
-    if (r == k) {
-#pragma unroll
-      for (int q = 0; q < 16; q++) rowb[b][c0 + q] = m[q];
-    }
-    __syncthreads();
-    if (t == 0 && bad < 0 && !(rowb[b][k] > 0.0 && rowb[b][k] <= DBL_MAX)) bad = k;
-    const double inv = 1.0 / rowb[b][k];
-    const double ci = r < N ? colb[b][r] : 0.0;
-#pragma unroll
-    for (int q = 0; q < 16; q++) {
-      const int j = c0 + q;
-      const double pj = ((j == k) ? 1.0 : rowb[b][j]) * inv;
-      m[q] = (r == k) ? pj : ((j == k) ? 0.0 : m[q]) - ci * pj;
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 16; q++)
-    if (r < nout && c0 + q < nout)
-      dst[(size_t)r * ldd + c0 + q] = (r < N && c0 + q < N) ? m[q] : 0.0;
-  if (t == 0 && bad >= 0) flag_pivot(base + bad, flag);
-}
-
-__global__ void __launch_bounds__(256) k_dense_invert_reg(Batch<InvertArgs> B, int N) {
-  double* Mg = B.v[blockIdx.x].M;
-  invert_reg_body(Mg, N, Mg, N, N, N, 0, B.v[blockIdx.x].flag);
-}
-
-// Larger N (a coarsest level that cannot halve again, as 12^3 under 353^3:
-// N = 1000): Gauss-Jordan by blocks of kGJ = 64 pivots.  Per block k, with P
-// the inverse of the diagonal block, C the block's column panel and
-// R = P A[k, :] its row panel: A[i, j] -= C_i R_j, A[k, :] = R,
-// A[:, k] = -C P, A[k, k] = P.  Three launches a block: the diagonal block
-// (registers, one workgroup), the panels, and the rank-64 update in 64 x 64
-// tiles on the FP64 matrix cores.  One pivot at a time over the whole matrix
-// takes three launches a pivot and 16 N^2 bytes of traffic each: 9.4 ms and
-// 3,000 launches at N = 1000, the largest part of a 353^3 solve.
-constexpr int kGJ = 64;
-constexpr int kGjLda = 36, kGjLdb = 72;  // LDS strides: every bank twice per access
-
-typedef double gj_d4 __attribute__((ext_vector_type(4)));
-
-// acc[ti][tj] += the 16 x 16 tiles of A B over K = 64 owned by this wavefront
-// (rows 32 (w / 2) + 16 ti, columns 32 (w % 2) + 16 tj): A is am x ak (lda),
-// B ak x bn (ldb), taken as zero outside.
-__device__ __forceinline__ void gj_mm(const double* __restrict__ A, size_t lda, int am, int ak,
-                                      const double* __restrict__ B, size_t ldb, int bn,
-                                      gj_d4 (&acc)[2][2]) {
-  __shared__ double sA[kGJ * kGjLda], sB[32 * kGjLdb];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int r0 = 32 * (w >> 1), c0 = 32 * (w & 1), li = lane & 15, lk = lane >> 4;
-  for (int h = 0; h < 2; h++) {
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int x = t + 256 * e;
-      const int ar = x >> 5, ac = x & 31;
-      sA[ar * kGjLda + ac] = (ar < am && 32 * h + ac < ak) ? A[ar * lda + 32 * h + ac] : 0.0;
-      const int br = x >> 6, bc = x & 63;
-      sB[br * kGjLdb + bc] = (32 * h + br < ak && bc < bn) ? B[(32 * h + br) * ldb + bc] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 32; kk += 4) {
-      double a[2], b[2];
-#pragma unroll
-      for (int q = 0; q < 2; q++) {
-        a[q] = sA[(r0 + 16 * q + li) * kGjLda + kk + lk];
-        b[q] = sB[(kk + lk) * kGjLdb + c0 + 16 * q + li];
-      }
-#pragma unroll
-      for (int ti = 0; ti < 2; ti++)
-#pragma unroll
-        for (int tj = 0; tj < 2; tj++)
-          acc[ti][tj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ti], b[tj], acc[ti][tj], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-}
-
-// Calls f(row, column, value) for the tile elements this lane holds.
-template <class F>
-__device__ __forceinline__ void gj_each(const gj_d4 (&acc)[2][2], F f) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-  for (int ti = 0; ti < 2; ti++)
-#pragma unroll
-    for (int tj = 0; tj < 2; tj++)
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        f(32 * (w >> 1) + 16 * ti + 4 * v + (lane >> 4), 32 * (w & 1) + 16 * tj + (lane & 15),
-          acc[ti][tj][v]);
-}
-
-// work: P (64 x 64), R (64 x N), C (N x 64)
-struct GjWork {
-  double *P, *R, *C;
-  __device__ explicit GjWork(double* w, int N)
-      : P(w), R(w + kGJ * kGJ), C(w + kGJ * kGJ + (size_t)kGJ * N) {}
-};
-
-__global__ void __launch_bounds__(256) k_gj_diag(Batch<InvertArgs> B, int N, int kb) {
-  const InvertArgs& a = B.v[blockIdx.x];
-  const GjWork W(a.work, N);
-  const int p0 = kb * kGJ;
-  invert_reg_body(a.M + (size_t)p0 * N + p0, N, W.P, kGJ, min(kGJ, N - p0), kGJ, p0, a.flag);
-}
-
-// blockIdx.y 0: R of column tile blockIdx.x; 1: C of row tile blockIdx.x.
-__global__ void __launch_bounds__(256) k_gj_panels(Batch<InvertArgs> B, int N, int kb) {
-  const InvertArgs& a = B.v[blockIdx.z];
-  const GjWork W(a.work, N);
-  const int q0 = blockIdx.x * kGJ, p0 = kb * kGJ, bk = min(kGJ, N - p0), bq = min(kGJ, N - q0);
-  if ((int)blockIdx.x == kb) return;
-  if (blockIdx.y == 0) {
-    gj_d4 acc[2][2] = {};
-    gj_mm(W.P, kGJ, bk, bk, a.M + (size_t)p0 * N + q0, N, bq, acc);
-    gj_each(acc, [&](int r, int c, double v) {
-      if (r < bk && c < bq) W.R[(size_t)r * N + q0 + c] = v;
-    });
-  } else {
-    for (int x = threadIdx.x; x < kGJ * kGJ; x += 256) {
-      const int r = x >> 6, c = x & 63;
-      if (r < bq && c < bk) W.C[(size_t)(q0 + r) * kGJ + c] = a.M[(size_t)(q0 + r) * N + p0 + c];
-    }
-  }
-}
-
-__global__ void __launch_bounds__(256) k_gj_update(Batch<InvertArgs> B, int N, int kb) {
-  const InvertArgs& a = B.v[blockIdx.z];
-  const GjWork W(a.work, N);
-  const int j0 = blockIdx.x * kGJ, i0 = blockIdx.y * kGJ, p0 = kb * kGJ;
-  const int bi = min(kGJ, N - i0), bj = min(kGJ, N - j0), bk = min(kGJ, N - p0);
-  const bool prow = (int)blockIdx.y == kb, pcol = (int)blockIdx.x == kb;
-  double* T = a.M + (size_t)i0 * N + j0;
-  if (prow) {
-    for (int x = threadIdx.x; x < kGJ * kGJ; x += 256) {
-      const int r = x >> 6, c = x & 63;
-      if (r < bi && c < bj) T[(size_t)r * N + c] = pcol ? W.P[x] : W.R[(size_t)r * N + j0 + c];
-    }
-    return;
-  }
-  gj_d4 acc[2][2] = {};
-  if (pcol)
-    gj_mm(W.C + (size_t)i0 * kGJ, kGJ, bi, bk, W.P, kGJ, bj, acc);
-  else
-    gj_mm(W.C + (size_t)i0 * kGJ, kGJ, bi, bk, W.R + j0, N, bj, acc);
-  gj_each(acc, [&](int r, int c, double v) {
-    if (r < bi && c < bj) T[(size_t)r * N + c] = (pcol ? 0.0 : T[(size_t)r * N + c]) - v;
-  });
-}
-
-// x_r = sum_c Minv[r][c] f_c over the interior unknowns, N <= kDenseSmall:
-// one workgroup gathers f into LDS, then each row sums in column order.
-constexpr int kDenseSmall = 96;
-
-template <class T>
-__global__ void __launch_bounds__(128) k_dense_solve(int nx, int ny, int nz, Batch<DenseArgs<T>> B,
-                                                     int N) {
-  __shared__ double fv[kDenseSmall];
-  const double* Minv = B.v[blockIdx.x].Minv;
-  const T* f = B.v[blockIdx.x].f;
-  T* x = B.v[blockIdx.x].x;
-  const int ni = nx - 2, nj = ny - 2;
-  for (int c = threadIdx.x; c < N; c += blockDim.x) {
-    const int i = c % ni + 1, j = (c / ni) % nj + 1, k = c / (ni * nj) + 1;
-    fv[c] = (double)f[IX(i, j, k, nx, ny)];
-  }
-  __syncthreads();
-  const int r = threadIdx.x;
-  if (r >= N) return;
-  const double* row = Minv + (size_t)r * N;
-  double s = 0.0;
-#pragma unroll 8
-  for (int c = 0; c < N; c++) s += row[c] * fv[c];
-  const int i = r % ni + 1, j = (r / ni) % nj + 1, k = r / (ni * nj) + 1;
-  x[IX(i, j, k, nx, ny)] = (T)s;
-}
-
-// The same product for larger N: one wavefront per row (its lanes stride over
-// the columns, so a row is read in whole lines), f gathered into LDS in chunks.
-// One thread per row took 413 us at N = 1000 (four workgroups, a chain of
-// 1,000 additions).
-constexpr int kDenseChunk = 2048;
-
-template <class T>
-__global__ void __launch_bounds__(kBlock)
-    k_dense_solve_rows(int nx, int ny, int nz, Batch<DenseArgs<T>> B, int N) {
-  __shared__ double fv[kDenseChunk];
-  const double* Minv = B.v[blockIdx.y].Minv;
-  const T* f = B.v[blockIdx.y].f;
-  T* x = B.v[blockIdx.y].x;
-  const int ni = nx - 2, nj = ny - 2;
-  const int lane = threadIdx.x & 63, r = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  double s = 0.0;
-  for (int c0 = 0; c0 < N; c0 += kDenseChunk) {
-    const int m = min(kDenseChunk, N - c0);
-    __syncthreads();
-    for (int t = threadIdx.x; t < m; t += kBlock) {
-      const int c = c0 + t, i = c % ni + 1, j = (c / ni) % nj + 1, k = c / (ni * nj) + 1;
-      fv[t] = (double)f[IX(i, j, k, nx, ny)];
-    }
-    __syncthreads();
-    if (r < N) {
-      const double* row = Minv + (size_t)r * N + c0;
-#pragma unroll 4
-      for (int t = lane; t < m; t += 64) s += row[t] * fv[t];
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_down(s, o, 64);
-  if (r >= N || lane != 0) return;
-  const int i = r % ni + 1, j = (r / ni) % nj + 1, k = r / (ni * nj) + 1;
-  x[IX(i, j, k, nx, ny)] = (T)s;
-}
-
 inline unsigned nblocks(size_t n) {
   size_t b = (n + kBlock - 1) / kBlock;
   if (b > 65535) b = 65535;
@@ -2127,204 +1409,6 @@ inline unsigned nblocks(size_t n) {
 }  // namespace
 
 // =================================================================== wrappers
-
-template <class T, int TY, int KC, int TX, int NT = kFT, bool ZX = false>
-void fused_sweep(hipStream_t s, int nx, int ny, int nz, const Batch<SweepArgs<T>>& B, int nb,
-                 int first) {
-  const int tiles = ((nx - 2 + TX - 1) / TX) * ((ny - 2 + TY - 1) / TY) * ((nz - 2 + KC - 1) / KC);
-  const long total = (long)tiles * nb;
-  const unsigned g = (unsigned)(((total + kXCD - 1) / kXCD) * kXCD);
-  k_gsrb7_fused<T, TY, KC, TX, NT, ZX><<<g, NT, 0, s>>>(nx, ny, nz, B, nb, first);
-}
-
-// The vector form: one lane per 16-byte run of a region row, the workgroup
-// rounded up to whole wavefronts.
-template <class T, int TY, int KC, int TX, bool ZX = false>
-void vfused_sweep(hipStream_t s, int nx, int ny, int nz, const Batch<SweepArgs<T>>& B, int nb,
-                  int first) {
-  constexpr int kV = 16 / (int)sizeof(T);
-  constexpr int NT = (((TY + 2) * ((TX + 2 + kV - 1) / kV) + 63) / 64) * 64;
-  const int tiles = ((nx - 2 + TX - 1) / TX) * ((ny - 2 + TY - 1) / TY) * ((nz - 2 + KC - 1) / KC);
-  const long total = (long)tiles * nb;
-  const unsigned g = (unsigned)(((total + kXCD - 1) / kXCD) * kXCD);
-  k_gsrb7_vfused<T, TY, KC, TX, NT, ZX><<<g, NT, 0, s>>>(nx, ny, nz, B, nb, first);
-}
-
-// The vector-form shapes (70TP or 7TPP: TY rows x P planes) need rows of at
-// least 16 bytes plus the two boundary points.
-static bool vector_shape(int rp) {
-  switch (rp) {
-    case 7048: case 7088: case 7410: case 7412: case 7416: case 7816:
-      return true;
-    default:
-      return false;
-  }
-}
-
-// Launches the vector form of shape rp (vector_shape(rp) holds).
-template <class T, int TX, bool ZX>
-void vfused_dispatch(hipStream_t s, int rp, int nx, int ny, int nz, const Batch<SweepArgs<T>>& B,
-                     int nb, int first) {
-  switch (rp) {
-    case 7048: vfused_sweep<T, 4, 8, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-    case 7088: vfused_sweep<T, 8, 8, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-    case 7410: vfused_sweep<T, 4, 10, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-    case 7412: vfused_sweep<T, 4, 12, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-    case 7416: vfused_sweep<T, 4, 16, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-    default: vfused_sweep<T, 8, 16, TX, ZX>(s, nx, ny, nz, B, nb, first); break;
-  }
-}
-
-// The scalar shapes 4 rows x 8 planes and 8 rows x 8 planes with 512
-// threads and every vector shape also come in the zero-start form; other
-// shapes start from a cleared x.
-static bool zero_start_shape(int rp) { return rp == 48 || rp == 5088 || vector_shape(rp); }
-
-static bool valid_tile(int v) {
-  const int w = v / 10000, rp = v % 10000;
-  const bool shape = rp == 416 || rp == 48 || rp == 816 || rp == 88 || rp == 84 || rp == 1616 ||
-                     rp == 832 || rp == 44 || rp == 68 || rp == 5088 || rp == 5084 ||
-                     rp == 5816 || vector_shape(rp);
-  return shape && (w == 0 || w == 64 || w == 80 || w == 96);
-}
-
-// tile shape of the fused sweep: rows x planes per workgroup
-// An APBS_PMG_FUSED_TILE shape, or 0.
-static int fused_tile_env() {
-  static int t = [] {
-    const char* e = getenv("APBS_PMG_FUSED_TILE");
-    if (!e) return 0;
-    const int v = atoi(e);
-    return valid_tile(v) ? v : 0;
-  }();
-  return t;
-}
-
-// Default shape for a grid and word size: the vector form, with the rows x
-// planes per workgroup that were fastest in standalone sweeps (us per sweep;
-// the best shape moves with how the workgroups fill the chip):
-//   FP32: up to 2.5M points 4 x 8 (65^3 12.2, 97^3 15.0, 129^3 20.3); up to
-//         5.5M 4 x 10 (161^3 29.7 against 36.5 for 4 x 8 and 50.2 for the
-//         scalar form); up to 20M 8 x 16 (193^3 49.3 against 70.8 for the
-//         scalar 8 x 8 with 512 threads); above 8 x 16 in 96-column tiles
-//         (353^3 403, against 421 in 64-column tiles and 573 scalar).
-//   FP64: up to 0.5M points 4 x 8 (65^3 12.9); up to 1M 4 x 10 (97^3 18.7);
-//         up to 3M 4 x 12 (129^3 31.8); up to 5.5M 4 x 10 (161^3 48.9 against
-//         65.4 scalar); up to 20M 4 x 12 (193^3 125.4 against 137.9); above
-//         4 x 12 in 80-column tiles (353^3 786, against 822 for 4 x 16 in
-//         64-column tiles and 931 scalar).
-// The column width otherwise follows fused_width; at 353^3 the widths above
-// leave fewer idle lanes (a run is 16 bytes, the workgroup whole wavefronts).
-int fused_tile(int nx, int ny, int nz, int word) {
-  if (const int t = fused_tile_env()) return t;
-  const long n = (long)nx * ny * nz;
-  if (word == 4) {
-    if (n <= 2500000L) return 7048;
-    if (n <= 5500000L) return 7410;
-    return n <= 20000000L ? 7816 : 967816;
-  }
-  if (n <= 500000L) return 7048;
-  if (n <= 1000000L) return 7410;
-  if (n <= 3000000L) return 7412;
-  if (n <= 5500000L) return 7410;
-  return n <= 20000000L ? 7412 : 807412;
-}
-
-// Whether the default fused sweep of a grid runs in the vector form.
-bool fused_vector(int nx, int ny, int nz, int word) {
-  return vector_shape(fused_tile(nx, ny, nz, word) % 10000) && nx >= 16 / word + 2;
-}
-
-// Tile width for an x extent: the one of 64 / 80 / 96 columns that leaves
-// the fewest idle columns in the last tile (64 on a tie).
-int fused_width(int nx) {
-  int best = 64, waste = 1 << 30;
-  for (int w : {64, 80, 96}) {
-    const int m = ((nx - 2 + w - 1) / w) * w - (nx - 2);
-    if (m < waste) {
-      waste = m;
-      best = w;
-    }
-  }
-  return best;
-}
-
-template <class T, int TX>
-static void fused_sweep_w(hipStream_t s, int rp, int nx, int ny, int nz,
-                          const Batch<SweepArgs<T>>& B, int nb, int first, bool zero_x) {
-  if (zero_x) {
-    if (rp == 48)
-      fused_sweep<T, 4, 8, TX, kFT, true>(s, nx, ny, nz, B, nb, first);
-    else if (vector_shape(rp))
-      vfused_dispatch<T, TX, true>(s, rp, nx, ny, nz, B, nb, first);
-    else
-      fused_sweep<T, 8, 8, TX, 512, true>(s, nx, ny, nz, B, nb, first);
-    return;
-  }
-  if (vector_shape(rp)) {
-    vfused_dispatch<T, TX, false>(s, rp, nx, ny, nz, B, nb, first);
-    return;
-  }
-  switch (rp) {
-    case 416: fused_sweep<T, 4, 16, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 48: fused_sweep<T, 4, 8, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 44: fused_sweep<T, 4, 4, TX>(s, nx, ny, nz, B, nb, first); break;
-    // 512-thread workgroups: 8 or 12 rows with one F round and one S round
-    case 5088: fused_sweep<T, 8, 8, TX, 512>(s, nx, ny, nz, B, nb, first); break;
-    case 5084: fused_sweep<T, 8, 4, TX, 512>(s, nx, ny, nz, B, nb, first); break;
-    case 5816: fused_sweep<T, 8, 16, TX, 512>(s, nx, ny, nz, B, nb, first); break;
-    case 68: fused_sweep<T, 6, 8, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 88: fused_sweep<T, 8, 8, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 84: fused_sweep<T, 8, 4, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 1616: fused_sweep<T, 16, 16, TX>(s, nx, ny, nz, B, nb, first); break;
-    case 832: fused_sweep<T, 8, 32, TX>(s, nx, ny, nz, B, nb, first); break;
-    default: fused_sweep<T, 8, 16, TX>(s, nx, ny, nz, B, nb, first); break;
-  }
-}
-
-template <class T>
-void gsrb7_fused_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,
-                       int nu, int iadjoint, int tile_shape, bool zero_x) {
-  check_batch(nb);
-  const int first = iadjoint ? 0 : 1;
-  const int tile =
-      tile_shape > 0 && valid_tile(tile_shape) ? tile_shape
-                                               : fused_tile(nx, ny, nz, (int)sizeof(T));
-  int rp = tile % 10000;
-  const int w = tile / 10000 ? tile / 10000 : fused_width(nx);
-  if (vector_shape(rp) && nx < 16 / (int)sizeof(T) + 2) rp = 48;
-  if (zero_x && !zero_start_shape(rp)) {
-    for (int b = 0; b < nb; b++) fill<T>(s, c[b].x, (size_t)nx * ny * nz, T(0));
-    zero_x = false;
-  }
-  for (int it = 0; it < nu; it++) {
-    // sweep it reads x (even it) or xs and writes the other one
-    Batch<SweepArgs<T>> B;
-    for (int b = 0; b < nb; b++) {
-      const LevelArgs<T>& a = c[b];
-      B.v[b] = SweepArgs<T>{a.A.a[1], a.A.a[2], a.A.a[3], a.D, a.f,
-                            (it & 1) ? a.xs : a.x, (it & 1) ? a.x : a.xs};
-    }
-    const bool zx = zero_x && it == 0;
-    if (w == 80)
-      fused_sweep_w<T, 80>(s, rp, nx, ny, nz, B, nb, first, zx);
-    else if (w == 96)
-      fused_sweep_w<T, 96>(s, rp, nx, ny, nz, B, nb, first, zx);
-    else
-      fused_sweep_w<T, 64>(s, rp, nx, ny, nz, B, nb, first, zx);
-  }
-  if (nu & 1)
-    for (int b = 0; b < nb; b++) copy_interior<T>(s, nx, ny, nz, c[b].xs, c[b].x);
-}
-
-template <class T>
-void gsrb7_fused(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D, const T* fc,
-                 T* x, T* tmp, int nu, int iadjoint, int tile_shape) {
-  const LevelArgs<T> c{A, D, fc, x, tmp, nullptr};
-  gsrb7_fused_batch<T>(s, nx, ny, nz, &c, 1, nu, iadjoint, tile_shape);
-}
-
-int gsrb7_fused_launches(int nu) { return nu + (nu & 1); }
 
 template <class T>
 void gsrb7(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D, const T* fc, T* x,
@@ -2763,71 +1847,6 @@ void galerkin(hipStream_t s, int st, int nxf, int nyf, int nzf, const Ops<double
   }
 }
 
-size_t dense_work(int N) {
-  return N <= kGJ ? (size_t)N : (size_t)kGJ * kGJ + 2 * (size_t)kGJ * N;
-}
-
-static void dense_invert_batch(hipStream_t s, const Batch<InvertArgs>& B, int N, int nb,
-                               int form) {
-  if (N <= 64 && form != 1) {
-    k_dense_invert_reg<<<nb, 256, 0, s>>>(B, N);
-    return;
-  }
-  const size_t lds = ((size_t)N * N + 2 * N) * sizeof(double);
-  if (lds <= 64 * 1024 && (size_t)N * N <= (size_t)kInvPer * 1024) {
-    k_dense_invert_lds<<<nb, 1024, lds, s>>>(B, N);
-    return;
-  }
-  const unsigned nt = (unsigned)((N + kGJ - 1) / kGJ);
-  for (unsigned kb = 0; kb < nt; kb++) {
-    k_gj_diag<<<nb, 256, 0, s>>>(B, N, (int)kb);
-    k_gj_panels<<<dim3(nt, 2, nb), 256, 0, s>>>(B, N, (int)kb);
-    k_gj_update<<<dim3(nt, nt, nb), 256, 0, s>>>(B, N, (int)kb);
-  }
-}
-
-void dense_assemble_invert_batch(hipStream_t s, int nx, int ny, int nz, int N,
-                                 const InvertArgs* c, int nb, int form) {
-  check_batch(nb);
-  Batch<InvertArgs> B;
-  for (int b = 0; b < nb; b++) B.v[b] = c[b];
-  k_dense_assemble<<<dim3((N + kAsmRows - 1) / kAsmRows, nb), kBlock, 0, s>>>(nx, ny, nz, B, N);
-  dense_invert_batch(s, B, N, nb, form);
-}
-
-void dense_assemble(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* D,
-                    double* M, int N) {
-  Batch<InvertArgs> B;
-  B.v[0] = InvertArgs{A, D, M, nullptr, nullptr};
-  k_dense_assemble<<<dim3((N + kAsmRows - 1) / kAsmRows, 1), kBlock, 0, s>>>(nx, ny, nz, B, N);
-}
-
-void dense_invert(hipStream_t s, double* M, double* work, int N, int form, double* flag) {
-  Batch<InvertArgs> B;
-  B.v[0] = InvertArgs{Ops<double>{}, nullptr, M, work, flag};
-  dense_invert_batch(s, B, N, 1, form);
-}
-
-template <class T>
-void dense_solve_batch(hipStream_t s, int nx, int ny, int nz, int N, const DenseArgs<T>* c,
-                       int nb) {
-  check_batch(nb);
-  Batch<DenseArgs<T>> B;
-  for (int b = 0; b < nb; b++) B.v[b] = c[b];
-  if (((size_t)N * N + N) * sizeof(double) <= 64 * 1024 && N <= kDenseSmall)
-    k_dense_solve<T><<<nb, 128, 0, s>>>(nx, ny, nz, B, N);
-  else
-    k_dense_solve_rows<T><<<dim3((N + kBlock / 64 - 1) / (kBlock / 64), nb), kBlock, 0, s>>>(
-        nx, ny, nz, B, N);
-}
-
-template <class T>
-void dense_solve(hipStream_t s, int nx, int ny, int nz, const double* Minv, int N, const T* f,
-                 T* x) {
-  const DenseArgs<T> c{Minv, f, x};
-  dense_solve_batch<T>(s, nx, ny, nz, N, &c, 1);
-}
-
 // ------------------------------------------------------ explicit instances
 #define INST(T)                                                                                 \
   template void gsrb7<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*, T*, int, \
@@ -2850,11 +1869,6 @@ void dense_solve(hipStream_t s, int nx, int ny, int nz, const double* Minv, int 
   template void axpy_interior<T>(hipStream_t, int, int, int, double, const T*, T*);             \
   template void copy_interior<T>(hipStream_t, int, int, int, const T*, T*);                     \
   template void add_diag<T>(hipStream_t, size_t, const T*, const T*, T*, float*);               \
-  template void dense_solve<T>(hipStream_t, int, int, int, const double*, int, const T*, T*);  \
-  template void gsrb7_fused<T>(hipStream_t, int, int, int, const Ops<T>&, const T*, const T*, T*, \
-                               T*, int, int, int);                                              \
-  template void gsrb7_fused_batch<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int, int,  \
-                                     int, int, bool);                                           \
   template void gsrb27_batch<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int, int, int); \
   template void gsrb27_pairs_batch<T>(hipStream_t, int, int, int, const LevelArgs<T>*, int, int, \
                                       int);                                                     \
@@ -2865,8 +1879,7 @@ void dense_solve(hipStream_t s, int nx, int ny, int nz, const double* Minv, int 
                                    const TransferArgs<T>*, int);                                \
   template void prolong_add_batch<T>(hipStream_t, int, int, int, int, int, int,                   \
                                      const TransferArgs<T>*, int);                              \
-  template void damp_factor_batch<T>(hipStream_t, int, int, int, const DampArgs<T>*, int);       \
-  template void dense_solve_batch<T>(hipStream_t, int, int, int, int, const DenseArgs<T>*, int);
+  template void damp_factor_batch<T>(hipStream_t, int, int, int, const DampArgs<T>*, int);
 INST(double)
 INST(float)
 #undef INST
