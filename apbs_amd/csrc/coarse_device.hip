@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(512)
 // value is formed by the separate kernels' expressions in their order (the
 // reductions in the trees of k_damp_part and k_finish), so the cycle keeps its
 // bits.
-constexpr int kBotPts = 1728;     // points of the level with its boundary
+constexpr int kBotPts = 1728;     // points of the level with its boundary, by parity class
 constexpr int kBotInner = 1024;   // interior points, one per thread
 constexpr int kBotCoarse = 512;   // points of the coarsest level with its boundary
 constexpr int kBotN = 64;         // unknowns of the coarsest level
@@ -290,43 +290,69 @@ struct BottomPart {
   double* damp;
 };
 
-// part27's sums at LDS index e of x (rows of nx, planes of nxy) with the 26
-// coefficients in its order.
+// A point of the level in LDS.  The eight parity classes of (i, j, k) are eight
+// contiguous blocks of S points, so the points of a colour and every one of
+// their neighbours' classes lie next to each other and a colour step reads LDS
+// without bank conflicts (with points in grid order a colour's lanes are two or
+// more words apart).  xm .. zp lead to the neighbours, whose classes differ.
+struct BotPoint {
+  int e, xm, xp, ym, yp, zm, zp;
+  __device__ BotPoint(int i, int j, int k, int nx, int ny, int nz) {
+    const int mx = (nx + 1) / 2, my = (ny + 1) / 2, S = mx * my * ((nz + 1) / 2);
+    const int bi = i & 1, bj = j & 1, bk = k & 1;
+    e = (4 * bk + 2 * bj + bi) * S + ((k >> 1) * my + (j >> 1)) * mx + (i >> 1);
+    xp = bi ? 1 - S : S;
+    xm = bi ? -S : S - 1;
+    yp = bj ? mx - 2 * S : 2 * S;
+    ym = bj ? -2 * S : 2 * S - mx;
+    zp = bk ? mx * my - 4 * S : 4 * S;
+    zm = bk ? -4 * S : 4 * S - mx * my;
+  }
+};
+
+// part27's three sums at a point, with the 26 coefficients in its order.
 template <class T>
-__device__ __forceinline__ P27<T> part27_lds(const T (&c)[26], const T* x, int e, int nx,
-                                             int nxy) {
-  P27<T> r;
-  T o = c[0] * x[e + nx];
-  o += c[1] * x[e - nx];
-  o += c[2] * x[e + 1];
-  o += c[3] * x[e - 1];
-  o += c[4] * x[e + nx + 1];
-  o += c[5] * x[e + nx - 1];
-  o += c[6] * x[e - nx + 1];
-  o += c[7] * x[e - nx - 1];
-  const int q = e + nxy, m = e - nxy;
-  T u = c[8] * x[q];
-  u += c[9] * x[q + nx];
-  u += c[10] * x[q - nx];
-  u += c[11] * x[q + 1];
-  u += c[12] * x[q - 1];
-  u += c[13] * x[q + nx + 1];
-  u += c[14] * x[q + nx - 1];
-  u += c[15] * x[q - nx + 1];
-  u += c[16] * x[q - nx - 1];
-  T d = c[17] * x[m];
-  d += c[18] * x[m + nx];
-  d += c[19] * x[m - nx];
-  d += c[20] * x[m + 1];
-  d += c[21] * x[m - 1];
-  d += c[22] * x[m + nx + 1];
-  d += c[23] * x[m + nx - 1];
-  d += c[24] * x[m - nx + 1];
-  d += c[25] * x[m - nx - 1];
-  r.o = o;
-  r.u = u;
-  r.d = d;
-  return r;
+__device__ __forceinline__ T sum_o(const T (&c)[26], const T* x, const BotPoint& p) {
+  const T *r = x + p.e, *rp = r + p.yp, *rm = r + p.ym;
+  T o = c[0] * rp[0];
+  o += c[1] * rm[0];
+  o += c[2] * r[p.xp];
+  o += c[3] * r[p.xm];
+  o += c[4] * rp[p.xp];
+  o += c[5] * rp[p.xm];
+  o += c[6] * rm[p.xp];
+  o += c[7] * rm[p.xm];
+  return o;
+}
+
+template <class T>
+__device__ __forceinline__ T sum_u(const T (&c)[26], const T* x, const BotPoint& p) {
+  const T *r = x + p.e + p.zp, *rp = r + p.yp, *rm = r + p.ym;
+  T u = c[8] * r[0];
+  u += c[9] * rp[0];
+  u += c[10] * rm[0];
+  u += c[11] * r[p.xp];
+  u += c[12] * r[p.xm];
+  u += c[13] * rp[p.xp];
+  u += c[14] * rp[p.xm];
+  u += c[15] * rm[p.xp];
+  u += c[16] * rm[p.xm];
+  return u;
+}
+
+template <class T>
+__device__ __forceinline__ T sum_d(const T (&c)[26], const T* x, const BotPoint& p) {
+  const T *r = x + p.e + p.zm, *rp = r + p.yp, *rm = r + p.ym;
+  T d = c[17] * r[0];
+  d += c[18] * rp[0];
+  d += c[19] * rm[0];
+  d += c[20] * r[p.xp];
+  d += c[21] * r[p.xm];
+  d += c[22] * rp[p.xp];
+  d += c[23] * rp[p.xm];
+  d += c[24] * rm[p.xp];
+  d += c[25] * rm[p.xm];
+  return d;
 }
 
 template <class T>
@@ -405,8 +431,10 @@ __device__ __forceinline__ double wave_tree(double v) {
   return v;
 }
 
-template <class T>
-__global__ void __launch_bounds__(1024)
+// kNT: the most threads of the launch (its register budget); kQ: Minv's entries
+// per thread.
+template <class T, int kNT, int kQ>
+__global__ void __launch_bounds__(kNT)
     k_bottom(int nxf, int nyf, int nx, int ny, int nz, int nxc, int nyc, int nzc,
              Batch<BottomPart<T>> B, int nu) {
   __shared__ T sx[kBotPts];
@@ -439,6 +467,7 @@ __global__ void __launch_bounds__(1024)
   }
   const bool act = col >= 0;
   const int e = k * nxy + j * nx + i;
+  const BotPoint pt(i, j, k, nx, ny, nz);
   T c[26], D = T(1), f = T(0);
   if (act) {
     coef27<T>(c, a.A, (size_t)e, nx, (size_t)nxy);
@@ -450,29 +479,35 @@ __global__ void __launch_bounds__(1024)
     for (int q = 0; q < 26; q++) c[q] = T(0);
   }
   // Minv's entries, in flight through the first sweeps
-  double mv[16];
+  double mv[kQ];
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
+  for (int q = 0; q < kQ; q++) {
     const int t = tid + q * NT;
     mv[q] = t < N * N ? a.Minv[t] : 0.0;
   }
-  for (int t = tid; t < nxy * nz; t += NT) sx[t] = T(0);
+  for (int t = tid; t < kBotPts; t += NT) sx[t] = T(0);
   for (int t = tid; t < cxy * nzc; t += NT) sxc[t] = T(0);
   __syncthreads();
   auto smooth = [&](bool adj) {
     for (int it = 0; it < nu; it++)
-      for (int cc = 0; cc < 8; cc++) {
-        if (act && col == (adj ? 7 - cc : cc)) {
-          const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
-          sx[e] = (f + (s.o + s.u + s.d)) / D;
+      for (int h = 0; h < 2; h++) {
+        const int ck = adj ? 1 - h : h;
+        T u = T(0), d = T(0);
+        if (act && (k & 1) == ck) {
+          u = sum_u<T>(c, sx, pt);
+          d = sum_d<T>(c, sx, pt);
         }
-        __syncthreads();
+        for (int cc = 0; cc < 4; cc++) {
+          if (act && col == 4 * ck + (adj ? 3 - cc : cc))
+            sx[pt.e] = (f + (sum_o<T>(c, sx, pt) + u + d)) / D;
+          __syncthreads();
+        }
       }
   };
   smooth(false);
   if (act) {
-    const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
-    sr[e] = f + s.o + s.u + s.d - D * sx[e];
+    const T o = sum_o<T>(c, sx, pt), u = sum_u<T>(c, sx, pt), d = sum_d<T>(c, sx, pt);
+    sr[e] = f + o + u + d - D * sx[pt.e];
   }
   __syncthreads();
   const int ci = tid % cni + 1, cj = (tid / cni) % cnj + 1, ck = tid / (cni * cnj) + 1;
@@ -480,7 +515,7 @@ __global__ void __launch_bounds__(1024)
     sfc[tid] = (double)restrict27<T, int>(sr, (2 * ck * ny + 2 * cj) * nx + 2 * ci, nx, nxy);
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
+  for (int q = 0; q < kQ; q++) {
     const int t = tid + q * NT;
     if (t < N * N) pool[(t / N) * (kBotN + 1) + t % N] = mv[q];
   }
@@ -497,9 +532,7 @@ __global__ void __launch_bounds__(1024)
     double num = 0.0, den = 0.0;
     if (tid < N) {
       const int p = (ck * nyc + cj) * nxc + ci;
-      T cc[26];
-      coef27<T>(cc, a.Ac, (size_t)p, nxc, (size_t)cxy);
-      const P27<T> s = part27_lds<T>(cc, sxc, p, nxc, cxy);
+      const P27<T> s = part27<T>(a.Ac.a, sxc, (size_t)p, nxc, (size_t)cxy);
       const T xv = sxc[p];
       const T ax = (-s.o) + (-s.u) + (-s.d) + a.Dc[p] * xv;
       num += (double)xv * sfc[tid];
@@ -528,7 +561,7 @@ __global__ void __launch_bounds__(1024)
         if (bx) v += W * sxc[c0 + cxy + nxc + 1];
       }
     }
-    sx[e] = sx[e] + T(sdamp) * v;
+    sx[pt.e] = sx[pt.e] + T(sdamp) * v;
   }
   __syncthreads();
   smooth(true);
@@ -539,9 +572,9 @@ __global__ void __launch_bounds__(1024)
   for (int t = tid; t < 2 * kBotInner; t += NT) pool[t] = 0.0;
   __syncthreads();
   if (act) {
-    const P27<T> s = part27_lds<T>(c, sx, e, nx, nxy);
-    const T xv = sx[e];
-    const T ax = (-s.o) + (-s.u) + (-s.d) + D * xv;
+    const T o = sum_o<T>(c, sx, pt), u = sum_u<T>(c, sx, pt), d = sum_d<T>(c, sx, pt);
+    const T xv = sx[pt.e];
+    const T ax = (-o) + (-u) + (-d) + D * xv;
     const int q = (i - 1) + ni * ((j - 1) + nj * (k - 1));
     double nv = 0.0, dv = 0.0;
     nv += (double)xv * (double)f;
@@ -578,7 +611,8 @@ __global__ void __launch_bounds__(1024)
 
 bool bottom_fits(int nx, int ny, int nz, int nxc, int nyc, int nzc) {
   if (nx < 3 || ny < 3 || nz < 3 || nxc < 3 || nyc < 3 || nzc < 3) return false;
-  return (long)(nx - 2) * (ny - 2) * (nz - 2) <= kBotInner && (long)nx * ny * nz <= kBotPts &&
+  return (long)(nx - 2) * (ny - 2) * (nz - 2) <= kBotInner &&
+         8L * ((nx + 1) / 2) * ((ny + 1) / 2) * ((nz + 1) / 2) <= kBotPts &&
          (long)(nxc - 2) * (nyc - 2) * (nzc - 2) <= kBotN && (long)nxc * nyc * nzc <= kBotCoarse;
 }
 
@@ -591,10 +625,19 @@ void bottom_batch(hipStream_t s, const int above[3], const int level[3], const i
     B.v[b] = BottomPart<T>{to27(c[b].A), to27(c[b].Ac), c[b].D,    c[b].Dc,
                            c[b].r,       c[b].x,        c[b].Minv, c[b].damp};
   const int n = (level[0] - 2) * (level[1] - 2) * (level[2] - 2);
-  // at least 256 threads: Minv is held by them, 16 entries each
+  // whole wavefronts, 256 threads or more: four of them sum the level's products
   const int nt = n <= 256 ? 256 : (n + 63) / 64 * 64;
-  k_bottom<T><<<nb, nt, 0, s>>>(above[0], above[1], level[0], level[1], level[2], coarsest[0],
-                                coarsest[1], coarsest[2], B, nu);
+  auto launch = [&](auto kernel) {
+    kernel<<<nb, nt, 0, s>>>(above[0], above[1], level[0], level[1], level[2], coarsest[0],
+                             coarsest[1], coarsest[2], B, nu);
+  };
+  static_assert(kBotN * kBotN <= 16 * 256 && kBotN * kBotN <= 8 * 576, "Minv fits the threads");
+  if (nt <= 512)
+    launch(k_bottom<T, 512, 16>);
+  else if (nt <= 768)
+    launch(k_bottom<T, 768, 8>);
+  else
+    launch(k_bottom<T, 1024, 8>);
 }
 
 // Whether a rows code (100 kV + m) fits a level: a run and its boundary points
