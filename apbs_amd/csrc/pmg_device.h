@@ -52,6 +52,14 @@ template <class T>
 void gsrb7_fused(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D,
                  const T* fc, T* x, T* tmp, int nu, int iadjoint, int tile_shape = 0);
 int gsrb7_fused_launches(int nu);
+// One sweep of the block form (code 100 TY + KC: TY rows of KC planes a
+// workgroup) from x to xs, or from xs to x with flip.  Bitwise the fused sweep.
+template <class T>
+struct LevelArgs;
+bool block_sweep_fits(int nx, int word, int code);
+template <class T>
+void gsrb7_block_sweep(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,
+                       int first, bool flip, bool zero_x, int code);
 // whether the default fused sweep of a grid runs in the vector form (word 4 or 8)
 bool fused_vector(int nx, int ny, int nz, int word);
 template <class T>

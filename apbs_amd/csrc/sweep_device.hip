@@ -4,6 +4,8 @@
 // (src/pmgc/gsd.c:95-165) without FMA contraction.
 #include "stencil27.h"
 
+#include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 namespace pmg {
@@ -508,9 +510,43 @@ int fused_tile(int nx, int ny, int nz, int word) {
   return n <= 20000000L ? 7412 : 807412;
 }
 
+constexpr int kBlockTile = 9000000;  // tile codes of block shapes: this + 100 TY + KC
+
+// Block shape (block_sweep_device.hip) of nb grids swept together, or 0 where
+// the march is the faster: above 1.5M points in all in FP64 (113^3 26.5 us a
+// sweep against 29.7, 129^3 32.3 against 31.9) and 3.1M in FP32 (145^3 22.4
+// against 27.5, 161^3 31.9 against 30.0).  The shape is the one of 256 or more
+// workgroups (one a CU; all shapes of a grid too small for that) that loads the
+// fewest runs per run written, the larger workgroup on a tie; rows so long that
+// it loads more than 2.7 (129^3 in FP64) keep the march.
+static int block_tile(int nx, int ny, int nz, int word, int nb) {
+  const double pts = (double)nx * ny * nz * nb;
+  if (pts > (word == 8 ? 1.5e6 : 3.1e6)) return 0;
+  const int kV = 16 / word, R = (nx - 2 + kV - 1) / kV;
+  auto groups = [&](int TY, int KC) {
+    return (long)((ny - 2 + TY - 1) / TY) * ((nz - 2 + KC - 1) / KC) * nb;
+  };
+  const long want = std::min(256L, groups(1, 1));
+  int best = 0, lanes = 0;
+  double eff = 0.0;
+  for (int TY = 1; TY <= 8; TY++)
+    for (int KC = 1; KC <= 8; KC++) {
+      const int code = 100 * TY + KC, runs = (TY + 2) * KC + 2 * TY;
+      if (!block_sweep_fits(nx, word, code) || groups(TY, KC) < want) continue;
+      const double e = (double)TY * KC / runs;
+      if (e > eff + 1e-9 || (e > eff - 1e-9 && R * runs > lanes)) {
+        best = code;
+        eff = e;
+        lanes = R * runs;
+      }
+    }
+  return eff >= 0.37 || pts < 1.0e5 ? best : 0;
+}
+
 // Whether the default fused sweep of a grid runs in the vector form.
 bool fused_vector(int nx, int ny, int nz, int word) {
-  return vector_shape(fused_tile(nx, ny, nz, word) % 10000) && nx >= 16 / word + 2;
+  return nx >= 16 / word + 2 && (vector_shape(fused_tile(nx, ny, nz, word) % 10000) ||
+                                 block_tile(nx, ny, nz, word, 1) != 0);
 }
 
 // Tile width for an x extent: the one of 64 / 80 / 96 columns that leaves
@@ -565,6 +601,15 @@ void gsrb7_fused_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>
                        int nu, int iadjoint, int tile_shape, bool zero_x) {
   check_batch(nb);
   const int first = iadjoint ? 0 : 1;
+  int block = tile_shape >= kBlockTile ? tile_shape - kBlockTile : 0;
+  if (tile_shape == 0 && !fused_tile_env()) block = block_tile(nx, ny, nz, (int)sizeof(T), nb);
+  if (block && block_sweep_fits(nx, (int)sizeof(T), block)) {
+    for (int it = 0; it < nu; it++)
+      gsrb7_block_sweep<T>(s, nx, ny, nz, c, nb, first, (it & 1) != 0, zero_x && it == 0, block);
+    if (nu & 1)
+      for (int b = 0; b < nb; b++) copy_interior<T>(s, nx, ny, nz, c[b].xs, c[b].x);
+    return;
+  }
   const int tile =
       tile_shape > 0 && valid_tile(tile_shape) ? tile_shape
                                                : fused_tile(nx, ny, nz, (int)sizeof(T));

@@ -148,3 +148,58 @@ def test_row_tiles_fp32_bitwise(L, n3, code):
                                            mode) == 1
                 out.append(x)
             assert np.array_equal(out[0], out[1]), (adj, nu)
+
+
+@pytest.mark.parametrize("n3", [(17, 19, 21), (33, 33, 33), (67, 13, 20), (130, 6, 11), (7, 70, 3),
+                                (4, 5, 6)])
+@pytest.mark.parametrize("code", [101, 202, 204, 302, 402, 404])
+def test_block_sweep_bitwise(L, n3, code):
+    """The block form of the fused red-black sweep (100 TY + KC: TY rows of KC
+    planes) against the oracle's sweep, bit for bit, boundary values not zero:
+    partial blocks in both directions, an odd last run, both colour orders, odd
+    and even sweep counts."""
+    nx, ny, nz = n3
+    n = nx * ny * nz
+    rng = np.random.default_rng(sum(n3) + code)
+    a = np.zeros((4, nz, ny, nx))
+    for s in range(4):
+        a[s, 1:-1, 1:-1, 1:-1] = rng.uniform(0.1, 1.0, (nz - 2, ny - 2, nx - 2))
+    a[0, 1:-1, 1:-1, 1:-1] = rng.uniform(6.0, 12.0, (nz - 2, ny - 2, nx - 2))
+    a = np.ascontiguousarray(a.reshape(-1))
+    cc, fc, x0 = rng.uniform(0, 1, n), rng.normal(size=n), rng.normal(size=n)
+    O = od.lib()
+    for adj in (0, 1):
+        for nu in (1, 2, 3):
+            xg, xo = x0.copy(), x0.copy()
+            L.pmgtest_gsrb_tile(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj, 9000000 + code)
+            O.orc_gsrb(nx, ny, nz, 7, P(a), P(cc), P(fc), P(xo), nu, adj, 1)
+            assert np.array_equal(xg, xo), (adj, nu)
+
+
+@pytest.mark.parametrize("n3", [(33, 33, 33), (67, 13, 20), (6, 5, 6), (130, 6, 11)])
+@pytest.mark.parametrize("code", [101, 202, 204, 402, 404])
+def test_block_sweep_fp32_bitwise(L, n3, code):
+    """The FP32 block form against the scalar march (tile 48), from a given and
+    from a zero start (the interior then holds NaN and is not read)."""
+    fp = ctypes.POINTER(ctypes.c_float)
+    rng = np.random.default_rng(sum(n3) + code)
+    nx, ny, nz = n3
+    sh = (nz, ny, nx)
+    ops = [np.zeros(sh, np.float32) for _ in range(4)]
+    for o, (lo, hi) in zip(ops, ((0.1, 1.0),) * 3 + ((6.0, 12.0),)):
+        o[1:-1, 1:-1, 1:-1] = rng.uniform(lo, hi, (nz - 2, ny - 2, nx - 2))
+    fc = rng.normal(size=sh).astype(np.float32)
+    x0 = np.zeros(sh, np.float32)
+    x0[1:-1, 1:-1, 1:-1] = rng.normal(size=(nz - 2, ny - 2, nx - 2))
+    ptr = lambda v: v.ctypes.data_as(fp)  # noqa: E731
+    for zero in (0, 1):
+        for adj in (0, 1):
+            out = []
+            for tile in (9000000 + code, 48):
+                x = x0.copy()
+                if zero:
+                    x[1:-1, 1:-1, 1:-1] = np.nan
+                assert L.pmgtest_fused32(nx, ny, nz, *[ptr(o) for o in ops], ptr(fc), ptr(x), 2,
+                                         adj, tile, zero) == 1
+                out.append(x)
+            assert np.array_equal(out[0], out[1]), (zero, adj)
