@@ -314,13 +314,15 @@ __device__ inline double poly_chi(const double* c, double sm, double sm2) {
 // stops when all its points' windows have vanished: they stay zero.  Forming
 // the boxes per point and atom took 5334 us at 193^3 with 20,000 atoms (1259 us
 // so, next to the boundary kernel that shares the GPU) and 389 us at 97^3 with
-// 1,500 (181 us).
+// 1,500 (181 us); leaving out the atoms whose windows reach no face of a point
+// before the four windows are formed, 1190 and 148 us.
 template <int kOrd>
 __global__ void __launch_bounds__(kB)
     k_coef_spline(Geo g, AtomsDev A, Tiles T, double win, double irad, double ionmask, double epsw,
                   double epsp, const double* pc, double* kappa, double* epsx, double* epsy,
                   double* epsz) {
   __shared__ double sp[3][kB], sitot2[kB], sictot2[kB], sstot2[kB], ssctot2[kB], srad[kB];
+  __shared__ double sfar2[kB];
   __shared__ int b0[3][kB], b1[3][kB], sa[kB];
   __shared__ int wsum[kB / 64];
   const int tile = blockIdx.x;
@@ -379,6 +381,9 @@ __global__ void __launch_bounds__(kB)
       ssctot2[slot] = sctot2;
       srad[slot] = arad;
       sa[slot] = a;
+      // (a face lies half a spacing from its point; widened past rounding)
+      const double far = (arad + win + 0.5 * fmax(hx, fmax(hy, hzed))) * (1.0 + 1e-9);
+      sfar2[slot] = far * far;
     }
     __syncthreads();
     for (int e = 0; e < cnt; e++) {
@@ -413,11 +418,16 @@ __global__ void __launch_bounds__(kB)
         }
       };
       const double* cf = kOrd == 2 ? nullptr : pc + kSplCoef * sa[e];
+      const double far2 = sfar2[e];
 #pragma unroll
       for (int u = 0; u < 2; u++) {
         const int ku = k + 4 * u;
         if (!in[u] || ku < b0[2][e] || ku > b1[2][e]) continue;
         const double dz2 = (p2 - ku * hzed) * (p2 - ku * hzed);
+        // beyond the ion window, or with that already zero, only an atom whose
+        // dielectric window reaches a face half a spacing away changes the point
+        const double d2 = dz2 + dy2 + dx2;
+        if (d2 > far2 && (d2 >= x2i || !(v[u][0] > VPMGSMALL))) continue;
         const double qz = p2 - (ku + 0.5) * hzed;
         window(v[u][0], dz2 + dy2 + dx2, x2c, x2i, ar + irad, kOrd == 2 ? nullptr : cf + 8, false);
         window(v[u][1], dz2 + dy2 + qx * qx, s2c, s2, ar, cf, true);
