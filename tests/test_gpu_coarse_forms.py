@@ -203,3 +203,25 @@ def test_block_sweep_fp32_bitwise(L, n3, code):
                                          adj, tile, zero) == 1
                 out.append(x)
             assert np.array_equal(out[0], out[1]), (zero, adj)
+
+
+@pytest.mark.parametrize("st", [7, 27])
+@pytest.mark.parametrize("c3", [(3, 3, 3), (5, 3, 7), (6, 6, 6), (34, 3, 5), (81, 21, 5),
+                                (9, 33, 17)])
+def test_galerkin_bitwise(L, st, c3):
+    """The Galerkin product against the oracle's, bit for bit: one coarse
+    point, less and a little more than a wavefront of them, partial last
+    wavefronts and workgroups, rows that straddle wavefronts."""
+    f3 = tuple(2 * n - 1 for n in c3)
+    nf, nc = int(np.prod(f3)), int(np.prod(c3))
+    rng = np.random.default_rng(sum(c3) + st)
+    na = 4 if st == 7 else 14
+    a = np.zeros((na, f3[2], f3[1], f3[0]))
+    a[:, 1:-1, 1:-1, 1:-1] = rng.uniform(0.1, 1.0, (na, f3[2] - 2, f3[1] - 2, f3[0] - 2))
+    a = np.ascontiguousarray(a.reshape(-1))
+    ag, ao = np.zeros(14 * nc), np.zeros(14 * nc)
+    assert L.pmgtest_galerkin(*f3, st, P(a), *c3, P(ag)) == 1
+    od.lib().orc_galerkin(*f3, st, P(a), *c3, P(ao))
+    cut = (slice(None),) + (slice(1, -1),) * 3
+    sh = (14, c3[2], c3[1], c3[0])
+    assert np.array_equal(ag.reshape(sh)[cut], ao.reshape(sh)[cut])
