@@ -10,12 +10,12 @@
 
 #include "stencil27.h"
 
-#include <type_traits>
-
-#include <cstdio>
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
+#include <cstdio>
 #include <cstdlib>
+#include <type_traits>
 
 namespace pmg {
 
@@ -426,72 +426,93 @@ __device__ inline double block_sum(double v, double* sh) {
   return r;
 }
 
-// The interior points [begin, end) (x fastest) a reduction block owns: kParts
-// contiguous chunks, dealt so that XCD x (blocks x, x + 8, ...) owns the
-// chunks [x * kParts/8, (x + 1) * kParts/8), a contiguous slab of the grid.
-__device__ inline void part_range(int n, int& begin, int& end) {
-  const int b = blockIdx.x;
-  const int c = (b % 8) * (kParts / 8) + b / 8;
-  const int chunk = (n + kParts - 1) / kParts;
-  begin = c * chunk;
-  end = begin + chunk < n ? begin + chunk : n;
+// How the fine-grid reductions walk the interior: tiles of 256 consecutive
+// (i, j) columns, a column a thread, cut along k into runs of kc planes so that
+// there are at most kParts runs (one a block) where there are that few tiles.
+// XCD x (blocks x, x + 8, ...) owns a contiguous eighth of the runs.  A thread
+// keeps its column's operands of planes k - 1 and k in registers; with points
+// dealt in contiguous chunks every block read them again, and most came from
+// beyond the L2 (130 bytes a point for the 80 of k_jres_trial at 353^3).
+// Microseconds so, and before: k_jres_trial 82 (94) at 161^3 in FP64, 1078
+// (1217) at 353^3 with an FP32 correction; k_nresid7_xpay 76 (83), 434 (530).
+struct PartRuns {
+  int ntile, kc, items;
+};
+
+inline PartRuns part_runs(int nx, int ny, int nz) {
+  const int nk = std::max(1, nz - 2);
+  const int ntile = std::max(1, ((nx - 2) * (ny - 2) + kBlock - 1) / kBlock);
+  const int want = std::max(1, std::min(nk, kParts / ntile));
+  const int kc = (nk + want - 1) / want;
+  return {ntile, kc, ntile * ((nk + kc - 1) / kc)};
+}
+
+// f(first point, planes) for each run of this block
+template <class F>
+__device__ __forceinline__ void part_columns(int nx, int ny, int nz, PartRuns R, F f) {
+  const int ni = nx - 2, nij = ni * (ny - 2);
+  const int per = (R.items + 7) / 8, x = blockIdx.x % 8;
+  for (int e = blockIdx.x / 8; e < per; e += kParts / 8) {
+    const int item = x * per + e;
+    if (item >= R.items) break;
+    const int ch = item / R.ntile, t = (item - ch * R.ntile) * kBlock + threadIdx.x;
+    if (t >= nij) continue;
+    const int j = 1 + t / ni, i = 1 + t - (j - 1) * ni, k0 = 1 + ch * R.kc;
+    f(IX(i, j, k0, nx, ny), min(R.kc, nz - 1 - k0));
+  }
 }
 
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_nrm1_part(int nx, int ny, int nz, const T* __restrict__ x, double* part) {
+    k_nrm1_part(int nx, int ny, int nz, PartRuns R, const T* __restrict__ x, double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
-  int t0, t1;
-  part_range(n, t0, t1);
+  const size_t nxy = (size_t)nx * ny;
   double acc = 0.0;
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
 #pragma unroll 4
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    acc += fabs((double)x[IX(i, j, k, nx, ny)]);
-  }
+    for (int m = 0; m < planes; m++, p += nxy) acc += fabs((double)x[p]);
+  });
   double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 // The 7-point residual and the partial sums of its L1 norm in one pass: the
-// points are visited in k_nrm1_part's order (part_range), so the norm is
+// points are visited in k_nrm1_part's order (part_columns), so the norm is
 // bitwise that of storing r and calling k_nrm1_part.  r is stored when
 // non-null.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_resid7_nrm(int nx, int ny, int nz, const T* __restrict__ oE, const T* __restrict__ oN,
-                 const T* __restrict__ uC, const T* __restrict__ D, const T* __restrict__ fc,
-                 const T* __restrict__ x, T* __restrict__ r, float* __restrict__ r32,
-                 double* part) {
+    k_resid7_nrm(int nx, int ny, int nz, PartRuns R, const T* __restrict__ oE,
+                 const T* __restrict__ oN, const T* __restrict__ uC, const T* __restrict__ D,
+                 const T* __restrict__ fc, const T* __restrict__ x, T* __restrict__ r,
+                 float* __restrict__ r32, double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
   const size_t nxy = (size_t)nx * ny;
-  int t0, t1;
-  part_range(n, t0, t1);
   double acc = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    const size_t p = IX(i, j, k, nx, ny);
-    // every operand first; acc7's terms and order
-    const T x0 = x[p], xjp = x[p + nx], xjm = x[p - nx], xip = x[p + 1], xim = x[p - 1];
-    const T xkm = x[p - nxy], xkp = x[p + nxy];
-    const T vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
-    const T vUm = uC[p - nxy], vU = uC[p], vD = D[p];
-    T sv = fc[p];
-    sv += vN * xjp;
-    sv += vNm * xjm;
-    sv += vE * xip;
-    sv += vEm * xim;
-    sv += vUm * xkm;
-    sv += vU * xkp;
-    const T v = sv - vD * x0;
-    if (r) r[p] = v;
-    if (r32) r32[p] = (float)v;
-    acc += fabs((double)v);
-  }
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
+    T xkm = x[p - nxy], x0 = x[p], vUm = uC[p - nxy];
+    for (int m = 0; m < planes; m++, p += nxy) {
+      // every operand first; acc7's terms and order
+      const T xjp = x[p + nx], xjm = x[p - nx], xip = x[p + 1], xim = x[p - 1];
+      const T xkp = x[p + nxy];
+      const T vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
+      const T vU = uC[p], vD = D[p];
+      T sv = fc[p];
+      sv += vN * xjp;
+      sv += vNm * xjm;
+      sv += vE * xip;
+      sv += vEm * xim;
+      sv += vUm * xkm;
+      sv += vU * xkp;
+      const T v = sv - vD * x0;
+      if (r) r[p] = v;
+      if (r32) r32[p] = (float)v;
+      acc += fabs((double)v);
+      xkm = x0;
+      x0 = xkp;
+      vUm = vU;
+    }
+  });
   double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -499,21 +520,19 @@ __global__ void __launch_bounds__(kBlock)
 // The L1 norm partials of x (k_nrm1_part's order) and y = (float) x on the
 // interior, in one pass.
 __global__ void __launch_bounds__(kBlock)
-    k_nrm1_to32(int nx, int ny, int nz, const double* __restrict__ x, float* __restrict__ y,
+    k_nrm1_to32(int nx, int ny, int nz, PartRuns R, const double* __restrict__ x, float* __restrict__ y,
                 double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
-  int t0, t1;
-  part_range(n, t0, t1);
+  const size_t nxy = (size_t)nx * ny;
   double acc = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    const size_t p = IX(i, j, k, nx, ny);
-    const double v = x[p];
-    y[p] = (float)v;
-    acc += fabs(v);
-  }
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
+#pragma unroll 4
+    for (int m = 0; m < planes; m++, p += nxy) {
+      const double v = x[p];
+      y[p] = (float)v;
+      acc += fabs(v);
+    }
+  });
   double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -908,38 +927,38 @@ __global__ void __launch_bounds__(kBlock)
 
 // k_nresid7 with the L1-norm partials of the residual (order of k_nrm1_part).
 __global__ void __launch_bounds__(kBlock)
-    k_nresid7_nrm(int nx, int ny, int nz, const double* __restrict__ oC,
+    k_nresid7_nrm(int nx, int ny, int nz, PartRuns R, const double* __restrict__ oC,
                   const double* __restrict__ oE, const double* __restrict__ oN,
                   const double* __restrict__ uC, const double* __restrict__ cc,
                   const double* __restrict__ fc, const double* __restrict__ x,
                   double* __restrict__ r, Ions ions, double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
   const size_t nxy = (size_t)nx * ny;
-  int t0, t1;
-  part_range(n, t0, t1);
   double acc = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    const size_t p = IX(i, j, k, nx, ny);
-    // every operand first; acc7's terms and order
-    const double x0 = x[p], xjp = x[p + nx], xjm = x[p - nx], xip = x[p + 1], xim = x[p - 1];
-    const double xkm = x[p - nxy], xkp = x[p + nxy];
-    const double vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
-    const double vUm = uC[p - nxy], vU = uC[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
-    const double w = ncvec(vcc, x0, ions);
-    double s7 = vfc;
-    s7 += vN * xjp;
-    s7 += vNm * xjm;
-    s7 += vE * xip;
-    s7 += vEm * xim;
-    s7 += vUm * xkm;
-    s7 += vU * xkp;
-    const double v = s7 - vC * x0 - w;
-    r[p] = v;
-    acc += fabs(v);
-  }
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
+    double xkm = x[p - nxy], x0 = x[p], vUm = uC[p - nxy];
+    for (int m = 0; m < planes; m++, p += nxy) {
+      // every operand first; acc7's terms and order
+      const double xjp = x[p + nx], xjm = x[p - nx], xip = x[p + 1], xim = x[p - 1];
+      const double xkp = x[p + nxy];
+      const double vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
+      const double vU = uC[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
+      const double w = ncvec(vcc, x0, ions);
+      double s7 = vfc;
+      s7 += vN * xjp;
+      s7 += vNm * xjm;
+      s7 += vE * xip;
+      s7 += vEm * xim;
+      s7 += vUm * xkm;
+      s7 += vU * xkp;
+      const double v = s7 - vC * x0 - w;
+      r[p] = v;
+      acc += fabs(v);
+      xkm = x0;
+      x0 = xkp;
+      vUm = vU;
+    }
+  });
   double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -949,52 +968,57 @@ __global__ void __launch_bounds__(kBlock)
 // the same bits as k_xpay_int then k_nresid7_nrm.  The boundary layers of x
 // and z are zero, as y's is.
 __global__ void __launch_bounds__(kBlock)
-    k_nresid7_xpay(int nx, int ny, int nz, const double* __restrict__ oC,
+    k_nresid7_xpay(int nx, int ny, int nz, PartRuns R, const double* __restrict__ oC,
                    const double* __restrict__ oE, const double* __restrict__ oN,
                    const double* __restrict__ uC, const double* __restrict__ cc,
                    const double* __restrict__ fc, const double* __restrict__ x, double a,
                    const double* __restrict__ z, double* __restrict__ y,
                    double* __restrict__ r, Ions ions, double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
   const size_t nxy = (size_t)nx * ny;
-  int t0, t1;
-  part_range(n, t0, t1);
   double acc = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    const size_t p = IX(i, j, k, nx, ny);
-    // every operand first: the point and its neighbours p, +j, -j, +i, -i, -k, +k
-    const size_t q[7] = {p, p + nx, p - nx, p + 1, p - 1, p - nxy, p + nxy};
-    double xc[7], zc[7];
+  auto trial = [&](size_t q) {
+    double v = x[q];
+    v += a * z[q];
+    return v;
+  };
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
+    double ykm = trial(p - nxy), y0 = trial(p), vUm = uC[p - nxy];
+    for (int m = 0; m < planes; m++, p += nxy) {
+      // every operand first: the neighbours +j, -j, +i, -i and +k
+      const size_t q[5] = {p + nx, p - nx, p + 1, p - 1, p + nxy};
+      double xc[5], zc[5];
 #pragma unroll
-    for (int u = 0; u < 7; u++) {
-      xc[u] = x[q[u]];
-      zc[u] = z[q[u]];
-    }
-    const double vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
-    const double vUm = uC[p - nxy], vU = uC[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
-    double yc[7];
+      for (int u = 0; u < 5; u++) {
+        xc[u] = x[q[u]];
+        zc[u] = z[q[u]];
+      }
+      const double vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
+      const double vU = uC[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
+      double yc[5];
 #pragma unroll
-    for (int u = 0; u < 7; u++) {
-      double v = xc[u];
-      v += a * zc[u];
-      yc[u] = v;
+      for (int u = 0; u < 5; u++) {
+        double v = xc[u];
+        v += a * zc[u];
+        yc[u] = v;
+      }
+      const double w = ncvec(vcc, y0, ions);
+      double s7 = vfc;
+      s7 += vN * yc[0];
+      s7 += vNm * yc[1];
+      s7 += vE * yc[2];
+      s7 += vEm * yc[3];
+      s7 += vUm * ykm;
+      s7 += vU * yc[4];
+      const double v = s7 - vC * y0 - w;
+      acc += fabs(v);
+      y[p] = y0;
+      r[p] = v;
+      ykm = y0;
+      y0 = yc[4];
+      vUm = vU;
     }
-    const double w = ncvec(vcc, yc[0], ions);
-    double s7 = vfc;
-    s7 += vN * yc[1];
-    s7 += vNm * yc[2];
-    s7 += vE * yc[3];
-    s7 += vEm * yc[4];
-    s7 += vUm * yc[5];
-    s7 += vU * yc[6];
-    const double v = s7 - vC * yc[0] - w;
-    acc += fabs(v);
-    y[p] = yc[0];
-    r[p] = v;
-  }
+  });
   double s = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
@@ -1012,7 +1036,7 @@ __global__ void __launch_bounds__(kBlock)
 // read z and x at the same seven points); kZF selects z from zf.
 template <bool kZF>
 __global__ void __launch_bounds__(kBlock)
-    k_jres_trial(int nx, int ny, int nz, const double* __restrict__ oC,
+    k_jres_trial(int nx, int ny, int nz, PartRuns R, const double* __restrict__ oC,
                  const double* __restrict__ oE, const double* __restrict__ oN,
                  const double* __restrict__ uC, const double* __restrict__ D,
                  const double* __restrict__ cc, const double* __restrict__ fc,
@@ -1021,58 +1045,64 @@ __global__ void __launch_bounds__(kBlock)
                  double* __restrict__ y, double* __restrict__ rn, float* __restrict__ r32,
                  float* __restrict__ rn32, Ions ions, double* part) {
   __shared__ double sh[kBlock];
-  const int ni = nx - 2, nij = ni * (ny - 2), n = nij * (nz - 2);
   const size_t nxy = (size_t)nx * ny;
-  int t0, t1;
-  part_range(n, t0, t1);
   double acc_j = 0.0, acc_n = 0.0;
-  for (int t = t0 + threadIdx.x; t < t1; t += kBlock) {
-    const int k = 1 + t / nij, rem = t - (k - 1) * nij;
-    const int j = 1 + rem / ni, i = 1 + rem - (j - 1) * ni;
-    const size_t p = IX(i, j, k, nx, ny);
-    // the point and its neighbours in acc7's order: p, +j, -j, +i, -i, -k, +k
-    const size_t q[7] = {p, p + nx, p - nx, p + 1, p - 1, p - nxy, p + nxy};
-    double zc[7], xc[7];
+  auto zval = [&](size_t q) { return kZF ? (double)zf[q] : z[q]; };
+  part_columns(nx, ny, nz, R, [&](size_t p, int planes) {
+    // z and the trial value y = x + a z (k_xpay_int's arithmetic) of planes
+    // k - 1 and k
+    double zkm = zval(p - nxy), z0 = zval(p), ykm = x[p - nxy], y0 = x[p], vUm = uC[p - nxy];
+    ykm += a * zkm;
+    y0 += a * z0;
+    for (int m = 0; m < planes; m++, p += nxy) {
+      // the neighbours +j, -j, +i, -i and +k
+      const size_t q[5] = {p + nx, p - nx, p + 1, p - 1, p + nxy};
+      double zc[5], xc[5];
 #pragma unroll
-    for (int u = 0; u < 7; u++) {
-      zc[u] = kZF ? (double)zf[q[u]] : z[q[u]];
-      xc[u] = x[q[u]];
-    }
-    const double vfz = fz[p], vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
-    const double vUm = uC[p - nxy], vU = uC[p], vD = D[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
-    // acc7's terms and order at z
-    double sj = vfz;
-    sj += vN * zc[1];
-    sj += vNm * zc[2];
-    sj += vE * zc[3];
-    sj += vEm * zc[4];
-    sj += vUm * zc[5];
-    sj += vU * zc[6];
-    const double vj = sj - vD * zc[0];
-    acc_j += fabs(vj);
-    // y = x + a z at the seven points (k_xpay_int's arithmetic)
-    double yc[7];
+      for (int u = 0; u < 5; u++) {
+        zc[u] = zval(q[u]);
+        xc[u] = x[q[u]];
+      }
+      const double vfz = fz[p], vN = oN[p], vNm = oN[p - nx], vE = oE[p], vEm = oE[p - 1];
+      const double vU = uC[p], vD = D[p], vC = oC[p], vcc = cc[p], vfc = fc[p];
+      // acc7's terms and order at z
+      double sj = vfz;
+      sj += vN * zc[0];
+      sj += vNm * zc[1];
+      sj += vE * zc[2];
+      sj += vEm * zc[3];
+      sj += vUm * zkm;
+      sj += vU * zc[4];
+      const double vj = sj - vD * z0;
+      acc_j += fabs(vj);
+      double yc[5];
 #pragma unroll
-    for (int u = 0; u < 7; u++) {
-      double v = xc[u];
-      v += a * zc[u];
-      yc[u] = v;
+      for (int u = 0; u < 5; u++) {
+        double v = xc[u];
+        v += a * zc[u];
+        yc[u] = v;
+      }
+      const double w = ncvec(vcc, y0, ions);
+      double s7 = vfc;
+      s7 += vN * yc[0];
+      s7 += vNm * yc[1];
+      s7 += vE * yc[2];
+      s7 += vEm * yc[3];
+      s7 += vUm * ykm;
+      s7 += vU * yc[4];
+      const double v = s7 - vC * y0 - w;
+      acc_n += fabs(v);
+      if (r32) r32[p] = (float)vj;
+      y[p] = y0;
+      rn[p] = v;
+      if (rn32) rn32[p] = (float)v;
+      zkm = z0;
+      z0 = zc[4];
+      ykm = y0;
+      y0 = yc[4];
+      vUm = vU;
     }
-    const double w = ncvec(vcc, yc[0], ions);
-    double s7 = vfc;
-    s7 += vN * yc[1];
-    s7 += vNm * yc[2];
-    s7 += vE * yc[3];
-    s7 += vEm * yc[4];
-    s7 += vUm * yc[5];
-    s7 += vU * yc[6];
-    const double v = s7 - vC * yc[0] - w;
-    acc_n += fabs(v);
-    if (r32) r32[p] = (float)vj;
-    y[p] = yc[0];
-    rn[p] = v;
-    if (rn32) rn32[p] = (float)v;
-  }
+  });
   const double bj = block_sum(acc_j, sh);
   const double bn = block_sum(acc_n, sh);
   if (threadIdx.x == 0) {
@@ -1388,7 +1418,8 @@ void prolong_add(hipStream_t s, int nxc, int nyc, int nzc, int nxf, int nyf, int
 template <class T>
 void nrm1(hipStream_t s, int nx, int ny, int nz, const T* x, double* part, double* out,
           double* hout) {
-  k_nrm1_part<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, x, part);
+  const PartRuns R = part_runs(nx, ny, nz);
+  k_nrm1_part<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, x, part);
   {
     Batch<FinishArgs> F;
     F.v[0] = FinishArgs{part, out, hout};
@@ -1399,8 +1430,9 @@ void nrm1(hipStream_t s, int nx, int ny, int nz, const T* x, double* part, doubl
 template <class T>
 void resid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D, const T* fc,
                  const T* x, T* r, double* part, double* out, double* hout, float* r32) {
-  k_resid7_nrm<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, A.a[1], A.a[2], A.a[3], D, fc, x, r, r32,
-                                            part);
+  const PartRuns R = part_runs(nx, ny, nz);
+  k_resid7_nrm<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[1], A.a[2], A.a[3], D, fc, x, r,
+                                            r32, part);
   {
     Batch<FinishArgs> F;
     F.v[0] = FinishArgs{part, out, hout};
@@ -1410,7 +1442,8 @@ void resid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T
 
 void nrm1_to32(hipStream_t s, int nx, int ny, int nz, const double* x, float* y, double* part,
                double* out, double* hout) {
-  k_nrm1_to32<<<kParts, kBlock, 0, s>>>(nx, ny, nz, x, y, part);
+  const PartRuns R = part_runs(nx, ny, nz);
+  k_nrm1_to32<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, x, y, part);
   Batch<FinishArgs> F;
   F.v[0] = FinishArgs{part, out, hout};
   k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
@@ -1420,8 +1453,9 @@ void nresid7_xpay_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>&
                        const double* cc, const double* fc, const double* x, double a,
                        const double* z, double* y, double* r, const Ions& ions, double* part,
                        double* out, double* hout) {
-  k_nresid7_xpay<<<kParts, kBlock, 0, s>>>(nx, ny, nz, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc, x,
-                                           a, z, y, r, ions, part);
+  const PartRuns R = part_runs(nx, ny, nz);
+  k_nresid7_xpay<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc,
+                                           x, a, z, y, r, ions, part);
   Batch<FinishArgs> F;
   F.v[0] = FinishArgs{part, out, hout};
   k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
@@ -1432,12 +1466,13 @@ void jres_trial_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A
                      const double* x, double a, const double* z, const float* zf, double* y,
                      double* rn, float* r32, float* rn32, const Ions& ions, double* part,
                      double* out, double* hout, double* out2, double* hout2) {
+  const PartRuns R = part_runs(nx, ny, nz);
   if (zf)
-    k_jres_trial<true><<<kParts, kBlock, 0, s>>>(nx, ny, nz, A.a[0], A.a[1], A.a[2], A.a[3], D, cc,
-                                                 fc, fz, x, a, z, zf, y, rn, r32, rn32, ions,
+    k_jres_trial<true><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], D,
+                                                 cc, fc, fz, x, a, z, zf, y, rn, r32, rn32, ions,
                                                  part);
   else
-    k_jres_trial<false><<<kParts, kBlock, 0, s>>>(nx, ny, nz, A.a[0], A.a[1], A.a[2], A.a[3], D,
+    k_jres_trial<false><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], D,
                                                   cc, fc, fz, x, a, z, zf, y, rn, r32, rn32, ions,
                                                   part);
   Batch<FinishArgs> F;
@@ -1449,8 +1484,9 @@ void jres_trial_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A
 void nresid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* cc,
                   const double* fc, const double* x, double* r, const Ions& ions, double* part,
                   double* out, double* hout) {
-  k_nresid7_nrm<<<kParts, kBlock, 0, s>>>(nx, ny, nz, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc, x, r,
-                                          ions, part);
+  const PartRuns R = part_runs(nx, ny, nz);
+  k_nresid7_nrm<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc, x,
+                                          r, ions, part);
   {
     Batch<FinishArgs> F;
     F.v[0] = FinishArgs{part, out, hout};

@@ -319,6 +319,53 @@ int pmgtest_resid(int nx, int ny, int nz, int st, const double* a, const double*
   return 1;
 }
 
+int pmgtest_fine_passes(int nx, int ny, int nz, const double* a, const double* cc,
+                        const double* fc, const double* fz, const double* x, const double* z,
+                        int f32, double* out, double* norms) {
+  const size_t n = (size_t)nx * ny * nz;
+  OpsHolder A(a, n, 7);
+  double *dcc = up(cc, n), *dfc = up(fc, n), *dfz = up(fz, n), *dx = up(x, n), *dz = up(z, n),
+         *dD = up(nullptr, n), *part = up(nullptr, 2 * pmg::kParts), *dn = up(nullptr, 8);
+  std::vector<double> zero(n, 0.0);
+  double* v[8];
+  for (double*& p : v) p = up(zero.data(), n);
+  float *zf = nullptr, *r32 = nullptr;
+  TCHECK(hipMalloc(&zf, n * sizeof(float)));
+  TCHECK(hipMalloc(&r32, n * sizeof(float)));
+  pmg::Ions I{};
+  I.nion = 2;
+  I.q[0] = 1.0, I.q[1] = -1.0, I.sconc[0] = I.sconc[1] = 0.5;
+  pmg::add_diag<double>(0, n, A.ops.a[0], dcc, dD);
+  if (f32) {
+    pmg::convert<double, float>(0, n, dz, zf);
+    pmg::convert<float, double>(0, n, zf, dz);
+  }
+  pmg::fill<float>(0, r32, n, 0.0f);
+  // one pass: y, rn, the inner residual's FP32 image
+  pmg::jres_trial_nrm1(0, nx, ny, nz, A.ops, dD, dcc, dfc, dfz, dx, 1.0, dz, f32 ? zf : nullptr,
+                       v[0], v[1], r32, nullptr, I, part, dn, nullptr, dn + 1, nullptr);
+  pmg::convert<float, double>(0, n, r32, v[2]);
+  // the separate passes
+  pmg::resid<double>(0, 7, nx, ny, nz, A.ops, dD, dfz, dz, v[3]);
+  pmg::nrm1<double>(0, nx, ny, nz, v[3], part, dn + 2);
+  pmg::xpay_interior(0, nx, ny, nz, dx, 1.0, dz, v[4]);
+  pmg::nresid7(0, nx, ny, nz, A.ops, dcc, dfc, v[4], v[5], I);
+  pmg::nrm1<double>(0, nx, ny, nz, v[5], part, dn + 3);
+  pmg::resid7_nrm1<double>(0, nx, ny, nz, A.ops, dD, dfz, dz, v[6], part, dn + 4);
+  pmg::nresid7_nrm1(0, nx, ny, nz, A.ops, dcc, dfc, v[4], v[7], I, part, dn + 5);
+  for (int q = 0; q < 8; q++) down(out + q * n, v[q], n);
+  pmg::nresid7_xpay_nrm1(0, nx, ny, nz, A.ops, dcc, dfc, dx, 1.0, dz, v[0], v[1], I, part, dn + 6);
+  pmg::nrm1_to32(0, nx, ny, nz, v[1], r32, part, dn + 7);
+  TCHECK(hipDeviceSynchronize());
+  for (int q = 0; q < 2; q++) down(out + (8 + q) * n, v[q], n);
+  down(norms, dn, 8);
+  for (double* p : {dcc, dfc, dfz, dx, dz, dD, part, dn}) TCHECK(hipFree(p));
+  for (double* p : v) TCHECK(hipFree(p));
+  TCHECK(hipFree(zf));
+  TCHECK(hipFree(r32));
+  return 1;
+}
+
 int pmgtest_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, const double* in,
                      double* out) {
   const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;

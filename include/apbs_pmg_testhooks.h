@@ -18,6 +18,17 @@ int pmgtest_gsrb(int nx, int ny, int nz, int stencil, const double *a, const dou
 /* Vmresid7_1s / Vmresid27_1s (src/pmgc/matvecd.c:461-596) */
 int pmgtest_resid(int nx, int ny, int nz, int stencil, const double *a, const double *cc,
                   const double *fc, const double *x, double *r);
+/* No reference counterpart: the fine level's norm passes (ions +-1, inner
+ * diagonal a[0] + cc, boundary layers of x and z zero).  out holds ten arrays:
+ * the one-pass form's y = x + z, nonlinear residual at y and FP32 image of the
+ * residual fz + J z; the separate passes' fz + J z, y and nonlinear residual;
+ * the two residual-and-norm passes' residuals; the trial-point pass's y and
+ * residual.  norms, 8: inner and nonlinear of the one pass, of stored arrays,
+ * of the residual-and-norm passes; of the trial-point pass, and of its stored
+ * residual with an FP32 image.  f32: z is rounded to FP32 first. */
+int pmgtest_fine_passes(int nx, int ny, int nz, const double *a, const double *cc,
+                        const double *fc, const double *fz, const double *x, const double *z,
+                        int f32, double *out, double *norms);
 /* Vrestrc2 (src/pmgc/matvecd.c:801-913) */
 int pmgtest_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, const double *in,
                      double *out);

@@ -4,7 +4,8 @@ The blocked dense inverse (coarsest grids that cannot halve down to 64
 unknowns) against numpy, at one unknown past the one-workgroup form, at whole
 and partial 64-pivot blocks, and at N = 1000 (the 12^3 coarsest grid under
 353^3); and a whole solve whose coarsest grid takes that form, against the
-oracle.
+oracle.  The bottom of the cycle, the row and block sweeps, the Galerkin
+product and the fine level's norm passes at the edges of their tiles.
 """
 import ctypes
 
@@ -225,3 +226,41 @@ def test_galerkin_bitwise(L, st, c3):
     cut = (slice(None),) + (slice(1, -1),) * 3
     sh = (14, c3[2], c3[1], c3[0])
     assert np.array_equal(ag.reshape(sh)[cut], ao.reshape(sh)[cut])
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("n3", [(3, 3, 3), (17, 19, 21), (33, 9, 130), (66, 67, 35), (130, 131, 5),
+                                (517, 515, 4)])
+def test_fine_norm_passes(L, n3, f32):
+    """The fine level's one-pass forms against the separate passes, bit for
+    bit, and each norm against the sum of its array's magnitudes: partial
+    tiles of columns, runs of one and of many planes, a short last run, and
+    more tiles than blocks.  n eps bounds any order of n non-negative terms."""
+    nx, ny, nz = n3
+    n = nx * ny * nz
+    rng = np.random.default_rng(sum(n3) + f32)
+    cut = (slice(None),) + (slice(1, -1),) * 3
+
+    def inside(lo, hi, m=1):
+        v = np.zeros((m, nz, ny, nx))
+        v[cut] = rng.uniform(lo, hi, (m, nz - 2, ny - 2, nx - 2))
+        return np.ascontiguousarray(v.reshape(-1))
+
+    a, cc, fc, fz = inside(0.1, 1.0, 4), inside(0, 1), inside(-1, 1), inside(-1, 1)
+    x, z = inside(-3, 3), inside(-1, 1)
+    out, norms = np.zeros(10 * n), np.zeros(8)
+    assert L.pmgtest_fine_passes(nx, ny, nz, P(a), P(cc), P(fc), P(fz), P(x), P(z), f32, P(out),
+                                 P(norms)) == 1
+    o = out.reshape(10, nz, ny, nx)[cut]
+    for y in (0, 8):
+        assert np.array_equal(o[y], o[4])
+    for rn in (1, 7, 9):
+        assert np.array_equal(o[rn], o[5])
+    assert np.array_equal(o[6], o[3])
+    assert np.array_equal(o[2], o[3].astype(np.float32).astype(np.float64))
+    # inner norms 0, 2, 4; nonlinear ones 1, 3, 5, 6, 7: one order of points
+    assert norms[0] == norms[2] == norms[4]
+    assert norms[1] == norms[3] == norms[5] == norms[6] == norms[7]
+    for got, arr in ((norms[0], o[3]), (norms[1], o[5])):
+        ref = np.abs(arr).sum()
+        assert abs(got - ref) <= 2 * n * np.finfo(float).eps * ref
