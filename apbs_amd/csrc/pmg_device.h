@@ -257,6 +257,44 @@ struct LevelArgs {
   T* xs;
   T* r;
 };
+// One calculation's Jacobian diagonal on the fine level: out = N'(x), D = oC +
+// out and, with Df, its FP32 image (dcvec).
+struct DcArgs {
+  const double *cc, *x;
+  double* out;
+  const double* oC;
+  double* D;
+  float* Df;
+  Ions ions;
+};
+void dcvec_batch(hipStream_t s, size_t n, const DcArgs* c, int nb);
+
+// The same on a coarser level: out = P^T in, D = oC + out, Df its FP32 image
+// where given (restrict3 then add_diag over the whole level; out's boundary
+// layer is zero and stays).
+struct DiagArgs {
+  const double* in;
+  double* out;
+  const double* oC;
+  double* D;
+  float* Df;
+};
+void restrict_diag_batch(hipStream_t s, int nxf, int nyf, int nzf, int nxc, int nyc, int nzc,
+                         const DiagArgs* c, int nb);
+
+// One calculation of jres_trial_nrm1; all of a batch read z, or all zf.
+struct JresArgs {
+  Ops<double> A;  // (the four 7-point arrays)
+  const double *D, *cc, *fc, *fz, *x, *z;
+  const float* zf;
+  double *y, *rn;
+  float *r32, *rn32;
+  double *part, *out, *hout, *out2, *hout2;
+  Ions ions;
+};
+void jres_trial_nrm1_batch(hipStream_t s, int nx, int ny, int nz, double a, const JresArgs* c,
+                           int nb);
+
 // zero_x: every x starts at zero (its contents need not be cleared: the first
 // sweep does not read them)
 template <class T>

@@ -544,11 +544,15 @@ struct FinishArgs {
   double* hout;
 };
 
+struct FinishBatch {
+  FinishArgs v[2 * kMaxBatch];
+};
+
 // out[0] = sum(part[0..kParts-1]); ratio: out[0] = sum(a)/sum(b)
 // (and hout[0] = out[0] when hout is given); calculation blockIdx.x.  Only
 // the first nparts partial sums are read: the others are taken as +0.0, which
 // leaves the sum's bits as they are (no partial sum is -0.0).
-__global__ void __launch_bounds__(kBlock) k_finish(Batch<FinishArgs> B, int ratio, int nparts) {
+__global__ void __launch_bounds__(kBlock) k_finish(FinishBatch B, int ratio, int nparts) {
   __shared__ double sh[kBlock];
   const double* part = B.v[blockIdx.x].part;
   double* out = B.v[blockIdx.x].out;
@@ -618,13 +622,8 @@ __global__ void __launch_bounds__(kBlock) k_damp_part(int nx, int ny, int nz, Ba
 // ---------------------------------------------------------------- transfers
 // Restriction P^T (matvecd.c:801-913) with weights 1, 1/2, 1/4, 1/8.
 template <class T>
-__device__ __forceinline__ void restrict_body(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc,
-                                              const T* __restrict__ in, T* __restrict__ out,
-                                              T* __restrict__ zero) {
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  const int K = blockIdx.y + 1;
-  const int I = 1 + t % (nxc - 2), J = 1 + t / (nxc - 2);
-  if (J > nyc - 2) return;
+__device__ __forceinline__ T restrict_at(int nxf, int nyf, int I, int J, int K,
+                                         const T* __restrict__ in) {
   const T W1 = T(1.0), W2 = T(0.5), W4 = T(0.25), W8 = T(0.125);
   const int ii = 2 * I, jj = 2 * J, kk = 2 * K;
   const size_t sx = 1, sy = nxf, sz = (size_t)nxf * nyf;
@@ -658,7 +657,18 @@ __device__ __forceinline__ void restrict_body(int nxf, int nyf, int nzf, int nxc
   d += W8 * in[d0 - sx + sy];
   d += W8 * in[d0 + sx - sy];
   d += W8 * in[d0 - sx - sy];
-  out[IX(I, J, K, nxc, nyc)] = o + u + d;
+  return o + u + d;
+}
+
+template <class T>
+__device__ __forceinline__ void restrict_body(int nxf, int nyf, int nxc, int nyc,
+                                              const T* __restrict__ in, T* __restrict__ out,
+                                              T* __restrict__ zero) {
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  const int K = blockIdx.y + 1;
+  const int I = 1 + t % (nxc - 2), J = 1 + t / (nxc - 2);
+  if (J > nyc - 2) return;
+  out[IX(I, J, K, nxc, nyc)] = restrict_at<T>(nxf, nyf, I, J, K, in);
   if (zero) zero[IX(I, J, K, nxc, nyc)] = T(0);
 }
 
@@ -666,7 +676,37 @@ template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, Batch<TransferArgs<T>> B) {
   const TransferArgs<T>& a = B.v[blockIdx.z];
-  restrict_body<T>(nxf, nyf, nzf, nxc, nyc, nzc, a.in, a.out, a.zero);
+  restrict_body<T>(nxf, nyf, nxc, nyc, a.in, a.out, a.zero);
+}
+
+// restrict3 and the level's Jacobian diagonal, every point a thread: the
+// boundary layer of c keeps its values.  Launched apart for each calculation
+// and level with one pass over all diagonals behind them, a Newton step of
+// eight calculations at 65^3 took 48 launches here, 4 so.
+__device__ __forceinline__ void restrict_diag_body(int nxf, int nyf, int nxc, int nyc, int nzc,
+                                                   const double* __restrict__ in,
+                                                   double* __restrict__ out,
+                                                   const double* __restrict__ oC,
+                                                   double* __restrict__ D,
+                                                   float* __restrict__ Df) {
+  const unsigned t = blockIdx.x * kBlock + threadIdx.x, nx = nxc, ny = nyc;
+  const int I = (int)(t % nx), J = (int)(t / nx % ny), K = (int)(t / nx / ny);
+  if (K >= nzc) return;
+  const size_t p = IX(I, J, K, nxc, nyc);
+  double c;
+  if (I >= 1 && I <= nxc - 2 && J >= 1 && J <= nyc - 2 && K >= 1 && K <= nzc - 2)
+    out[p] = c = restrict_at<double>(nxf, nyf, I, J, K, in);
+  else
+    c = out[p];
+  const double v = oC[p] + c;
+  D[p] = v;
+  if (Df) Df[p] = (float)v;
+}
+
+__global__ void __launch_bounds__(kBlock)
+    k_restrict_diag(int nxf, int nyf, int nxc, int nyc, int nzc, Batch<DiagArgs> B) {
+  const DiagArgs& a = B.v[blockIdx.z];
+  restrict_diag_body(nxf, nyf, nxc, nyc, nzc, a.in, a.out, a.oC, a.D, a.Df);
 }
 
 // Trilinear prolongation and correction x_f += damp * P x_c (matvecd.c:935-1076
@@ -1035,15 +1075,14 @@ __global__ void __launch_bounds__(kBlock)
 // Every operand of a point is loaded before the arithmetic (the two stencils
 // read z and x at the same seven points); kZF selects z from zf.
 template <bool kZF>
-__global__ void __launch_bounds__(kBlock)
-    k_jres_trial(int nx, int ny, int nz, PartRuns R, const double* __restrict__ oC,
-                 const double* __restrict__ oE, const double* __restrict__ oN,
-                 const double* __restrict__ uC, const double* __restrict__ D,
-                 const double* __restrict__ cc, const double* __restrict__ fc,
-                 const double* __restrict__ fz, const double* __restrict__ x, double a,
-                 const double* __restrict__ z, const float* __restrict__ zf,
-                 double* __restrict__ y, double* __restrict__ rn, float* __restrict__ r32,
-                 float* __restrict__ rn32, Ions ions, double* part) {
+__device__ __forceinline__ void jres_body(
+    int nx, int ny, int nz, const PartRuns& R, const double* __restrict__ oC,
+    const double* __restrict__ oE, const double* __restrict__ oN, const double* __restrict__ uC,
+    const double* __restrict__ D, const double* __restrict__ cc, const double* __restrict__ fc,
+    const double* __restrict__ fz, const double* __restrict__ x, double a,
+    const double* __restrict__ z, const float* __restrict__ zf, double* __restrict__ y,
+    double* __restrict__ rn, float* __restrict__ r32, float* __restrict__ rn32, const Ions& ions,
+    double* part) {
   __shared__ double sh[kBlock];
   const size_t nxy = (size_t)nx * ny;
   double acc_j = 0.0, acc_n = 0.0;
@@ -1111,12 +1150,21 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+template <bool kZF>
+__global__ void __launch_bounds__(kBlock)
+    k_jres_trial(int nx, int ny, int nz, PartRuns R, double a, Batch<JresArgs> B) {
+  const JresArgs& c = B.v[blockIdx.y];
+  jres_body<kZF>(nx, ny, nz, R, c.A.a[0], c.A.a[1], c.A.a[2], c.A.a[3], c.D, c.cc, c.fc, c.fz, c.x,
+                 a, c.z, c.zf, c.y, c.rn, c.r32, c.rn32, c.ions, c.part);
+}
+
 // Vdc_vecpmg (mypdec.c:366-433) at every point; with oC given also the
 // diagonal D = oC + N'(x) and, with Df, its FP32 image (k_add_diag_levels'
 // values for this level) in the same pass.
-__global__ void k_dcvec(size_t n, const double* __restrict__ cc, const double* __restrict__ x,
-                        double* __restrict__ out, Ions I, const double* __restrict__ oC,
-                        double* __restrict__ D, float* __restrict__ Df) {
+__device__ __forceinline__ void dcvec_body(size_t n, const double* __restrict__ cc,
+                                           const double* __restrict__ x, double* __restrict__ out,
+                                           const Ions& I, const double* __restrict__ oC,
+                                           double* __restrict__ D, float* __restrict__ Df) {
   for (size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x; t < n; t += (size_t)gridDim.x * kBlock) {
     double o = 0.0;
     const double coef = cc[t], u = x[t];
@@ -1140,6 +1188,11 @@ __global__ void k_dcvec(size_t n, const double* __restrict__ cc, const double* _
       if (Df) Df[t] = (float)v;
     }
   }
+}
+
+__global__ void __launch_bounds__(kBlock) k_dcvec(size_t n, Batch<DcArgs> B) {
+  const DcArgs& a = B.v[blockIdx.y];
+  dcvec_body(n, a.cc, a.x, a.out, a.ions, a.oC, a.D, a.Df);
 }
 
 // ---------------------------------------------------------------- operators
@@ -1374,9 +1427,27 @@ void nresid7(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const 
                                                          A.a[3], cc, fc, x, r, ions);
 }
 
+void dcvec_batch(hipStream_t s, size_t n, const DcArgs* c, int nb) {
+  check_batch(nb);
+  Batch<DcArgs> B;
+  for (int b = 0; b < nb; b++) B.v[b] = c[b];
+  k_dcvec<<<dim3(nblocks(n), nb), kBlock, 0, s>>>(n, B);
+}
+
 void dcvec(hipStream_t s, size_t n, const double* cc, const double* x, double* out,
            const Ions& ions, const double* oC, double* D, float* Df) {
-  k_dcvec<<<nblocks(n), kBlock, 0, s>>>(n, cc, x, out, ions, oC, D, Df);
+  const DcArgs c{cc, x, out, oC, D, Df, ions};
+  dcvec_batch(s, n, &c, 1);
+}
+
+void restrict_diag_batch(hipStream_t s, int nxf, int nyf, int nzf, int nxc, int nyc, int nzc,
+                         const DiagArgs* c, int nb) {
+  check_batch(nb);
+  Batch<DiagArgs> B;
+  for (int b = 0; b < nb; b++) B.v[b] = c[b];
+  const size_t n = (size_t)nxc * nyc * nzc;
+  k_restrict_diag<<<dim3((unsigned)((n + kBlock - 1) / kBlock), 1, nb), kBlock, 0, s>>>(
+      nxf, nyf, nxc, nyc, nzc, B);
 }
 
 template <class T>
@@ -1421,7 +1492,7 @@ void nrm1(hipStream_t s, int nx, int ny, int nz, const T* x, double* part, doubl
   const PartRuns R = part_runs(nx, ny, nz);
   k_nrm1_part<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, x, part);
   {
-    Batch<FinishArgs> F;
+    FinishBatch F;
     F.v[0] = FinishArgs{part, out, hout};
     k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
   }
@@ -1434,7 +1505,7 @@ void resid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T
   k_resid7_nrm<T><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[1], A.a[2], A.a[3], D, fc, x, r,
                                             r32, part);
   {
-    Batch<FinishArgs> F;
+    FinishBatch F;
     F.v[0] = FinishArgs{part, out, hout};
     k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
   }
@@ -1444,7 +1515,7 @@ void nrm1_to32(hipStream_t s, int nx, int ny, int nz, const double* x, float* y,
                double* out, double* hout) {
   const PartRuns R = part_runs(nx, ny, nz);
   k_nrm1_to32<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, x, y, part);
-  Batch<FinishArgs> F;
+  FinishBatch F;
   F.v[0] = FinishArgs{part, out, hout};
   k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
 }
@@ -1456,9 +1527,27 @@ void nresid7_xpay_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>&
   const PartRuns R = part_runs(nx, ny, nz);
   k_nresid7_xpay<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc,
                                            x, a, z, y, r, ions, part);
-  Batch<FinishArgs> F;
+  FinishBatch F;
   F.v[0] = FinishArgs{part, out, hout};
   k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
+}
+
+void jres_trial_nrm1_batch(hipStream_t s, int nx, int ny, int nz, double a, const JresArgs* c,
+                           int nb) {
+  check_batch(nb);
+  const PartRuns R = part_runs(nx, ny, nz);
+  Batch<JresArgs> B;
+  FinishBatch F;
+  for (int b = 0; b < nb; b++) {
+    B.v[b] = c[b];
+    F.v[2 * b] = FinishArgs{c[b].part, c[b].out, c[b].hout};
+    F.v[2 * b + 1] = FinishArgs{c[b].part + kParts, c[b].out2, c[b].hout2};
+  }
+  if (c[0].zf)
+    k_jres_trial<true><<<dim3(kParts, nb), kBlock, 0, s>>>(nx, ny, nz, R, a, B);
+  else
+    k_jres_trial<false><<<dim3(kParts, nb), kBlock, 0, s>>>(nx, ny, nz, R, a, B);
+  k_finish<<<2 * nb, kBlock, 0, s>>>(F, 0, kParts);
 }
 
 void jres_trial_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A,
@@ -1466,19 +1555,9 @@ void jres_trial_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A
                      const double* x, double a, const double* z, const float* zf, double* y,
                      double* rn, float* r32, float* rn32, const Ions& ions, double* part,
                      double* out, double* hout, double* out2, double* hout2) {
-  const PartRuns R = part_runs(nx, ny, nz);
-  if (zf)
-    k_jres_trial<true><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], D,
-                                                 cc, fc, fz, x, a, z, zf, y, rn, r32, rn32, ions,
-                                                 part);
-  else
-    k_jres_trial<false><<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], D,
-                                                  cc, fc, fz, x, a, z, zf, y, rn, r32, rn32, ions,
-                                                  part);
-  Batch<FinishArgs> F;
-  F.v[0] = FinishArgs{part, out, hout};
-  F.v[1] = FinishArgs{part + kParts, out2, hout2};
-  k_finish<<<2, kBlock, 0, s>>>(F, 0, kParts);
+  const JresArgs c{A,  D,   cc,   fc,   fz,  x,    z,    zf,    y,
+                   rn, r32, rn32, part, out, hout, out2, hout2, ions};
+  jres_trial_nrm1_batch(s, nx, ny, nz, a, &c, 1);
 }
 
 void nresid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* cc,
@@ -1488,7 +1567,7 @@ void nresid7_nrm1(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, c
   k_nresid7_nrm<<<kParts, kBlock, 0, s>>>(nx, ny, nz, R, A.a[0], A.a[1], A.a[2], A.a[3], cc, fc, x,
                                           r, ions, part);
   {
-    Batch<FinishArgs> F;
+    FinishBatch F;
     F.v[0] = FinishArgs{part, out, hout};
     k_finish<<<1, kBlock, 0, s>>>(F, 0, kParts);
   }
@@ -1498,7 +1577,7 @@ template <class T>
 void damp_factor_batch(hipStream_t s, int nx, int ny, int nz, const DampArgs<T>* c, int nb) {
   check_batch(nb);
   Batch<DampPart<T>> B;
-  Batch<FinishArgs> F;
+  FinishBatch F;
   for (int b = 0; b < nb; b++) {
     B.v[b] = DampPart<T>{to27(c[b].A), c[b].D, c[b].x, c[b].w0, c[b].part};
     F.v[b] = FinishArgs{c[b].part, c[b].out, nullptr};

@@ -379,6 +379,27 @@ int pmgtest_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, const
 }
 
 // xf_out = xf + damp * P xc on the fine interior
+int pmgtest_restrict_diag(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, int nb,
+                          const double* in, const double* oC, double* out, double* D, float* Df) {
+  if (nb < 1 || nb > pmg::kMaxBatch) return 0;
+  const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;
+  double *di = up(in, nb * nf), *doC = up(oC, nb * nc), *dout = up(out, nb * nc),
+         *dD = up(nullptr, nb * nc);
+  float* df = nullptr;
+  TCHECK(hipMalloc(&df, nb * nc * sizeof(float)));
+  pmg::DiagArgs c[pmg::kMaxBatch];
+  for (int b = 0; b < nb; b++)
+    c[b] = pmg::DiagArgs{di + b * nf, dout + b * nc, doC + b * nc, dD + b * nc, df + b * nc};
+  pmg::restrict_diag_batch(0, nxf, nyf, nzf, nxc, nyc, nzc, c, nb);
+  TCHECK(hipDeviceSynchronize());
+  down(out, dout, nb * nc);
+  down(D, dD, nb * nc);
+  TCHECK(hipMemcpy(Df, df, nb * nc * sizeof(float), hipMemcpyDeviceToHost));
+  for (double* p : {di, doC, dout, dD}) TCHECK(hipFree(p));
+  TCHECK(hipFree(df));
+  return 1;
+}
+
 int pmgtest_prolong(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const double* xc,
                     double* xf, double damp) {
   const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;

@@ -771,7 +771,7 @@ struct PmgDev {
   // fillco's MDH boundary, and the coarsest level's dense inverse, on second
   // streams (pmgint::set_side_stream)
   int side = 1;
-  // the dense inverse's stream: set_diagonals forks it after the diagonals
+  // the dense inverse's stream: invert_coarsest forks it after the diagonals
   // are formed, the V-cycle joins it before the coarsest solve
   hipStream_t cs = nullptr;
   hipEvent_t cs_fork = nullptr, cs_join = nullptr;
@@ -1267,22 +1267,20 @@ void build_operators(PmgDev* d) {
   }
 }
 
-// D_l = oC_l + c_l for the given per-level Helmholtz arrays (and, for a
-// mixed-precision solve, its FP32 image Df_l in the same pass), levels first
-// and up.
-void diag_levels(PmgDev* d, bool use_cprime, int first) {
+// D_l = oC_l + c_l on every level (and, for a mixed-precision solve, its FP32
+// image Df_l in the same pass).
+void diag_levels(PmgDev* d) {
   const bool f32 = d->precision == 1 && d->h_mixed;
   pmg::DiagLevels dl{};
-  dl.nl = d->ntot - first;
+  dl.nl = d->ntot;
   dl.off[0] = 0;
-  for (int q = 0; q < dl.nl; q++) {
-    const int l = first + q;
+  for (int l = 0; l < dl.nl; l++) {
     DLevel& L = d->L[l];
-    dl.oC[q] = L.a[0];
-    dl.c[q] = use_cprime ? L.cprime : L.cc;
-    dl.D[q] = L.D;
-    dl.Df[q] = f32 ? L.Df : nullptr;
-    dl.off[q + 1] = dl.off[q] + L.n;
+    dl.oC[l] = L.a[0];
+    dl.c[l] = L.cc;
+    dl.D[l] = L.D;
+    dl.Df[l] = f32 ? L.Df : nullptr;
+    dl.off[l + 1] = dl.off[l] + L.n;
   }
   if (dl.nl > 0) pmg::add_diag_levels(d->s, dl);
 }
@@ -1292,10 +1290,8 @@ pmg::InvertArgs invert_args(PmgDev* d) {
   return pmg::InvertArgs{C.ops(), C.D, d->dense, d->dwork, d->hscal + kPivotFlag};
 }
 
-// The diagonals (levels first and up; the Newton Jacobian forms the fine one
-// with N'(u)), then the dense inverse of the coarsest level.
-void set_diagonals(PmgDev* d, bool use_cprime, int first = 0) {
-  diag_levels(d, use_cprime, first);
+// The dense inverse of the coarsest level, whose diagonal is formed.
+void invert_coarsest(PmgDev* d) {
   const DLevel& C = d->L[d->ntot - 1];
   // The inverse is first read by the coarsest solve, after the downward
   // half of the next V-cycle; a one-workgroup kernel, it runs on its own
@@ -1319,18 +1315,15 @@ void set_diagonals(PmgDev* d, bool use_cprime, int first = 0) {
   }
 }
 
-// set_diagonals for n calculations of one shape on the first one's stream:
+// invert_coarsest for n calculations of one shape on the first one's stream:
 // the dense inverses of all n in one launch.
-void set_diagonals_batch(PmgDev* const* ds, int n, bool use_cprime, int first = 0) {
+void invert_coarsest_batch(PmgDev* const* ds, int n) {
   if (n == 1) {
-    set_diagonals(ds[0], use_cprime, first);
+    invert_coarsest(ds[0]);
     return;
   }
   pmg::InvertArgs ia[pmg::kMaxBatch];
-  for (int b = 0; b < n; b++) {
-    diag_levels(ds[b], use_cprime, first);
-    ia[b] = invert_args(ds[b]);
-  }
+  for (int b = 0; b < n; b++) ia[b] = invert_args(ds[b]);
   const DLevel& C = ds[0]->L[ds[0]->ntot - 1];
   pmg::dense_assemble_invert_batch(ds[0]->s, C.nx, C.ny, C.nz, ds[0]->dn, ia, n);
 }
@@ -1343,8 +1336,8 @@ void join_dense(PmgDev* d) {
 }
 
 // FP32 images of the level operators (the stencil arrays, which do not
-// change within a solve); set_diagonals writes the FP32 diagonals, which
-// change with every Newton Jacobian.
+// change within a solve); the FP32 diagonals, which change with every Newton
+// Jacobian, are written with the FP64 ones.
 void sync_fp32_ops(PmgDev* d) {
   for (int l = 0; l < d->ntot; l++) {
     DLevel& L = d->L[l];
@@ -1589,22 +1582,44 @@ struct Trials {
   bool x_pending[pmg::kMaxBatch];
 };
 
-// The inner residual f + J z of calculation b's fine level (its L1 norm to
-// hscal[0]; its FP32 image to r32 when given) and, with trials, its trial
-// point and nonlinear residual (norm to hscal[1]) in the same pass.  With zf
-// given, z is read as (double) zf.
-void inner_resid(PmgDev* d, const double* f, const double* z, float* r32, Trials* tr, int b,
-                 const float* zf = nullptr) {
-  const DLevel& F = d->L[0];
-  if (tr) {
-    pmg::jres_trial_nrm1(d->s, F.nx, F.ny, F.nz, F.ops(), F.D, F.cc, F.fc, f, tr->u[b], 1.0, z,
-                         zf, tr->y[b], tr->rn[b], r32, tr->rn32[b], *tr->I[b], d->part, d->scal,
-                         d->hscal, d->scal + 8, d->hscal + 1);
-    tr->ok[b] = true;
-  } else {
-    pmg::resid7_nrm1<double>(d->s, F.nx, F.ny, F.nz, F.ops(), F.D, f, z, nullptr, d->part,
-                             d->scal, d->hscal, r32);
+// The inner residuals f + J z of m calculations' fine levels (L1 norms to
+// hscal[0]; FP32 images to r32 where given) and, with trials, their trial
+// points and nonlinear residuals (norms to hscal[1]) in the same pass, one
+// launch for all.  Entry q is calculation b[q]; zf, given for all or none, is
+// read as z = (double) zf.
+struct InnerResid {
+  PmgDev* d[pmg::kMaxBatch];
+  const double *f[pmg::kMaxBatch], *z[pmg::kMaxBatch];
+  float* r32[pmg::kMaxBatch];
+  const float* zf[pmg::kMaxBatch];
+  int b[pmg::kMaxBatch];
+  int m = 0;
+  void add(PmgDev* dev, const double* rhs, const double* sol, float* img, int calc,
+           const float* sol32 = nullptr) {
+    d[m] = dev, f[m] = rhs, z[m] = sol, r32[m] = img, b[m] = calc, zf[m] = sol32;
+    m++;
   }
+};
+
+void inner_resid(const InnerResid& R, Trials* tr) {
+  if (R.m == 0) return;
+  const DLevel& S = R.d[0]->L[0];
+  pmg::JresArgs ja[pmg::kMaxBatch];
+  for (int q = 0; q < R.m; q++) {
+    PmgDev* d = R.d[q];
+    const DLevel& F = d->L[0];
+    const int b = R.b[q];
+    if (!tr) {
+      pmg::resid7_nrm1<double>(d->s, F.nx, F.ny, F.nz, F.ops(), F.D, R.f[q], R.z[q], nullptr,
+                               d->part, d->scal, d->hscal, R.r32[q]);
+      continue;
+    }
+    ja[q] = pmg::JresArgs{F.ops(),   F.D,         F.cc,     F.fc,        R.f[q],       tr->u[b],
+                          R.z[q],    R.zf[q],     tr->y[b], tr->rn[b],   R.r32[q],     tr->rn32[b],
+                          d->part,   d->scal,     d->hscal, d->scal + 8, d->hscal + 1, *tr->I[b]};
+    tr->ok[b] = true;
+  }
+  if (tr) pmg::jres_trial_nrm1_batch(R.d[0]->s, S.nx, S.ny, S.nz, 1.0, ja, R.m);
 }
 
 // The trial norms of the calculations that computed a trial this round
@@ -1653,11 +1668,13 @@ void mvcs64_batch(PmgDev* const* ds, int n, double* const* const* X, const doubl
       }
     if (m == 0) break;
     run_vcycle<double>(act, cs, m);
+    InnerResid ir;
     for (int b = 0; b < n; b++) {
       if (!active[b]) continue;
       its[b]++;
-      inner_resid(ds[b], f[b], X[b][0], nullptr, tr, b);
+      ir.add(ds[b], f[b], X[b][0], nullptr, b);
     }
+    inner_resid(ir, tr);
     read_norms(ds, n, active, rsnrm, failed);
     read_trials(ds, n, active, tr);
     for (int b = 0; b < n; b++) {
@@ -1756,6 +1773,8 @@ void mixed_batch(PmgDev* const* ds, int n, double* const* const* X64, const doub
     }
     if (m == 0) break;
     run_vcycle<float>(act, cs, m);
+    // (every active calculation has run the same cycles: zf for all or none)
+    InnerResid ir;
     for (int b = 0; b < n; b++) {
       if (!active[b]) continue;
       PmgDev* d = ds[b];
@@ -1768,9 +1787,10 @@ void mixed_batch(PmgDev* const* ds, int n, double* const* const* X64, const doub
         pmg::axpy_interior_f32(d->s, F.nx, F.ny, F.nz, 1.0, F.xfl, X64[b][0],
                                x_zero && it[b] == 0);
       it[b]++;
-      inner_resid(d, f[b], X64[b][0], F.w0f, tr, b, direct ? F.xfl : nullptr);
+      ir.add(d, f[b], X64[b][0], F.w0f, b, direct ? F.xfl : nullptr);
       pending[b] = direct;
     }
+    inner_resid(ir, tr);
     read_norms(ds, n, active, rsnrm, failed);
     read_trials(ds, n, active, tr);
   }
@@ -1876,19 +1896,29 @@ void newton_batch(Vpmg* const* th, int n, double* relres, int* iters, int* inner
         idx[m++] = b;
       }
     if (m == 0) break;
-    // Jacobian diagonal on all levels
+    // Jacobian diagonal on all levels: cprime, oC + cprime and its FP32 image,
+    // a launch a level for all calculations
+    pmg::DcArgs dc[pmg::kMaxBatch];
+    pmg::DiagArgs da[pmg::kMaxBatch];
+    auto df32 = [&](PmgDev* d, int l) {
+      return d->precision == 1 && d->h_mixed ? d->L[l].Df : nullptr;
+    };
     for (int q = 0; q < m; q++) {
       PmgDev* d = ad[q];
-      DLevel* L = d->L;
+      const DLevel& F = d->L[0];
       st[idx[q]].iters++;
-      // cprime and the fine diagonal oC + cprime (and its FP32 image) in one pass
-      pmg::dcvec(d->s, d->n, L[0].cc, d->u, L[0].cprime, st[idx[q]].I, L[0].a[0], L[0].D,
-                 d->precision == 1 && d->h_mixed ? L[0].Df : nullptr);
-      for (int l = 1; l < d->ntot; l++)
-        pmg::restrict3<double>(d->s, L[l - 1].nx, L[l - 1].ny, L[l - 1].nz, L[l].nx, L[l].ny,
-                               L[l].nz, L[l - 1].cprime, L[l].cprime);
+      dc[q] = pmg::DcArgs{F.cc, d->u, F.cprime, F.a[0], F.D, df32(d, 0), st[idx[q]].I};
     }
-    set_diagonals_batch(ad, m, true, 1);
+    pmg::dcvec_batch(ad[0]->s, ad[0]->n, dc, m);
+    for (int l = 1; l < ad[0]->ntot; l++) {
+      const DLevel &P = ad[0]->L[l - 1], &C = ad[0]->L[l];
+      for (int q = 0; q < m; q++) {
+        DLevel* L = ad[q]->L;
+        da[q] = pmg::DiagArgs{L[l - 1].cprime, L[l].cprime, L[l].a[0], L[l].D, df32(ad[q], l)};
+      }
+      pmg::restrict_diag_batch(ad[0]->s, P.nx, P.ny, P.nz, C.nx, C.ny, C.nz, da, m);
+    }
+    invert_coarsest_batch(ad, m);
     // inner solve: the V-cycle clears the coarse corrections itself; the
     // fine one starts at zero
     double errs[pmg::kMaxBatch], rr[pmg::kMaxBatch];
@@ -2814,7 +2844,8 @@ static int solve_group(Vpmg* const* th, int n, int* ok) {
   if (newton) {
     newton_batch(th, n, relres, iters, inner, good);
   } else {
-    set_diagonals_batch(ds, n, false);
+    for (int b = 0; b < n; b++) diag_levels(ds[b]);
+    invert_coarsest_batch(ds, n);
     double* X[pmg::kMaxBatch][24];
     double* const* Xp[pmg::kMaxBatch];
     const double* fp[pmg::kMaxBatch];

@@ -32,6 +32,11 @@ int pmgtest_fine_passes(int nx, int ny, int nz, const double *a, const double *c
 /* Vrestrc2 (src/pmgc/matvecd.c:801-913) */
 int pmgtest_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, const double *in,
                      double *out);
+/* No reference counterpart: the restriction with the level's Jacobian diagonal,
+ * for nb calculations (arrays one after another): out = P^T in on the interior
+ * (its boundary layer as given), D = oC + out everywhere, Df its FP32 image. */
+int pmgtest_restrict_diag(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, int nb,
+                          const double *in, const double *oC, double *out, double *D, float *Df);
 /* VinterpPMG2 + Vxaxpy (src/pmgc/matvecd.c:935-1076, mgcsd.c:485-487) */
 int pmgtest_prolong(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const double *xc,
                     double *xf, double damp);

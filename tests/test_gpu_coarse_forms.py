@@ -264,3 +264,29 @@ def test_fine_norm_passes(L, n3, f32):
     for got, arr in ((norms[0], o[3]), (norms[1], o[5])):
         ref = np.abs(arr).sum()
         assert abs(got - ref) <= 2 * n * np.finfo(float).eps * ref
+
+
+@pytest.mark.parametrize("c3", [(3, 3, 3), (9, 33, 17), (17, 16, 16), (41, 5, 11)])
+@pytest.mark.parametrize("nb", [1, 3, 8])
+def test_restrict_with_diagonal(L, c3, nb):
+    """The restricted Helmholtz term with the diagonal it gives, for one and
+    for several calculations, against the restriction alone, bit for bit; the
+    boundary layer keeps its values and enters the diagonal."""
+    f3 = tuple(2 * n - 1 for n in c3)
+    nf, nc = int(np.prod(f3)), int(np.prod(c3))
+    rng = np.random.default_rng(sum(c3) + nb)
+    x, oC, out = rng.normal(size=nb * nf), rng.normal(size=nb * nc), rng.normal(size=nb * nc)
+    ref = out.copy()
+    for b in range(nb):
+        r = ref[b * nc:(b + 1) * nc].copy()
+        L.pmgtest_restrict(*f3, *c3, P(np.ascontiguousarray(x[b * nf:(b + 1) * nf])), P(r))
+        sh = (c3[2], c3[1], c3[0])
+        cut = (slice(1, -1),) * 3
+        ref[b * nc:(b + 1) * nc].reshape(sh)[cut] = r.reshape(sh)[cut]
+    D, Df = np.zeros(nb * nc), np.zeros(nb * nc, np.float32)
+    fp = ctypes.POINTER(ctypes.c_float)
+    assert L.pmgtest_restrict_diag(*f3, *c3, nb, P(x), P(oC), P(out), P(D),
+                                   Df.ctypes.data_as(fp)) == 1
+    assert np.array_equal(out, ref)
+    assert np.array_equal(D, oC + ref)
+    assert np.array_equal(Df, (oC + ref).astype(np.float32))
