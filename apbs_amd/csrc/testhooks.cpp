@@ -411,6 +411,24 @@ int pmgtest_prolong(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const 
   return 1;
 }
 
+int pmgtest_prolong32(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const float* xc,
+                      float* xf, double damp) {
+  const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;
+  float *dc = nullptr, *df = nullptr;
+  double* dd = up(&damp, 1);
+  TCHECK(hipMalloc(&dc, nc * sizeof(float)));
+  TCHECK(hipMalloc(&df, nf * sizeof(float)));
+  TCHECK(hipMemcpy(dc, xc, nc * sizeof(float), hipMemcpyHostToDevice));
+  TCHECK(hipMemcpy(df, xf, nf * sizeof(float), hipMemcpyHostToDevice));
+  pmg::prolong_add<float>(0, nxc, nyc, nzc, nxf, nyf, nzf, dc, df, dd);
+  TCHECK(hipDeviceSynchronize());
+  TCHECK(hipMemcpy(xf, df, nf * sizeof(float), hipMemcpyDeviceToHost));
+  TCHECK(hipFree(dc));
+  TCHECK(hipFree(df));
+  TCHECK(hipFree(dd));
+  return 1;
+}
+
 int pmgtest_galerkin_form(int nxf, int nyf, int nzf, int st, const double* af, int nxc, int nyc,
                           int nzc, double* ac, int form) {
   if (form < 0 || form > 4) return 0;

@@ -40,6 +40,8 @@ int pmgtest_restrict_diag(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, 
 /* VinterpPMG2 + Vxaxpy (src/pmgc/matvecd.c:935-1076, mgcsd.c:485-487) */
 int pmgtest_prolong(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const double *xc,
                     double *xf, double damp);
+int pmgtest_prolong32(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const float *xc,
+                      float *xf, double damp);
 /* VbuildG_7 / VbuildG_27 (src/pmgc/buildGd.c:450-3115) */
 int pmgtest_galerkin(int nxf, int nyf, int nzf, int stencil, const double *af, int nxc, int nyc,
                      int nzc, double *ac);

@@ -290,3 +290,35 @@ def test_restrict_with_diagonal(L, c3, nb):
     assert np.array_equal(out, ref)
     assert np.array_equal(D, oC + ref)
     assert np.array_equal(Df, (oC + ref).astype(np.float32))
+
+
+@pytest.mark.parametrize("word", [4, 8])
+@pytest.mark.parametrize("c3", [(3, 3, 3), (4, 3, 5), (5, 9, 4), (34, 6, 7), (41, 17, 9)])
+def test_prolongation_runs(L, c3, word):
+    """x_f + damp P x_c in runs of 16 bytes against the terms added one by one
+    in their order, bit for bit: rows of 5 points and up, a last run that
+    leaves the row, the first run's boundary point, the boundary layer kept."""
+    dt = np.float32 if word == 4 else np.float64
+    f3 = tuple(2 * n - 1 for n in c3)
+    rng = np.random.default_rng(sum(c3) + word)
+    xc = np.zeros((c3[2], c3[1], c3[0]), dt)
+    xc[1:-1, 1:-1, 1:-1] = rng.normal(size=tuple(n - 2 for n in xc.shape))
+    xf = rng.normal(size=(f3[2], f3[1], f3[0])).astype(dt)
+    damp = 0.8125 + rng.uniform(0, 0.1)
+    k, j, i = np.meshgrid(*(np.arange(1, n - 1) for n in xf.shape), indexing="ij")
+    w = (0.5 ** (i % 2 + j % 2 + k % 2)).astype(dt)
+    v = np.zeros(i.shape, dt)
+    for dz in (0, 1):
+        for dy in (0, 1):
+            for dx in (0, 1):
+                on = (dx <= i % 2) & (dy <= j % 2) & (dz <= k % 2)
+                c = xc[np.where(on, k // 2 + dz, 0), np.where(on, j // 2 + dy, 0),
+                       np.where(on, i // 2 + dx, 0)]
+                v = np.where(on, v + w * c, v)
+    ref = xf.copy()
+    ref[1:-1, 1:-1, 1:-1] = ref[1:-1, 1:-1, 1:-1] + dt(damp) * v
+    got = np.ascontiguousarray(xf)
+    ct = ctypes.POINTER(ctypes.c_float if word == 4 else ctypes.c_double)
+    f = L.pmgtest_prolong32 if word == 4 else L.pmgtest_prolong
+    assert f(*c3, *f3, xc.ctypes.data_as(ct), got.ctypes.data_as(ct), ctypes.c_double(damp)) == 1
+    assert np.array_equal(got, ref)
