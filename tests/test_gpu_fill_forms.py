@@ -37,3 +37,25 @@ def test_dense_tiles(srfm, chgm, dims, h):
     # both potentials are converged to 1e-12 of the residual: the forces agree
     # to that times the operator's conditioning, far inside 1e-8
     assert diff <= 1e-8 * big
+
+
+@pytest.mark.parametrize("srfm", ["spl2", "spl3", "spl4"])
+@pytest.mark.parametrize("swin", [-0.2, 0.0])
+def test_windows_of_no_width(srfm, swin):
+    """A spline window that is empty (0) or inside out (the core's radius the
+    larger, r - swin): every point of an atom's box within the core is zero, so
+    no point may be passed over for lying beyond the outer radius.  Maps bitwise
+    the oracle's."""
+    atoms = synth.globule(40, (5.0,) * 3, 11, net_charge=1)[:3]
+    pbe = dict(pdie=2.0, sdie=78.54, srfm=srfm, chgm="spl2", swin=swin, srad=1.4, sdens=10.0,
+               temp=298.15, bcfl="zero", ions=[(1, 0.15, 2.0), (-1, 0.15, 2.0)])
+    c = od.mol_center(atoms[0])
+    mol = driver.Molecule(*atoms)
+    g = driver.Calc(mol, driver.manual_mgparm([65, 65, 65], c, grid=[0.25] * 3), pbe)
+    g.fillco()
+    nlev, dime = od.check_nlev([65, 65, 65])
+    o = od.OrcCalc(od.make_params(dime, [0.25] * 3, c, nlev, pbe), atoms)
+    o.fillco()
+    for name in ("epsx", "epsy", "epsz", "kappa"):
+        off = int((~np.isclose(g.array(name), o.array(name), 0, 0, equal_nan=True)).sum())
+        assert off == 0, (name, off)
