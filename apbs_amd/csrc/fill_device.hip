@@ -1024,6 +1024,8 @@ __global__ void __launch_bounds__(kB)
   part[((size_t)c * 6 + f) * mx + t] = val;
 }
 
+// Bound by the loads' latency: with each waited for before the next, 312
+// chunks (17^3, 5,000 atoms) took about 78 us, eight in flight about 18.
 __global__ void __launch_bounds__(kB)
     k_bc_mdh_sum(Geo g, int nch, int mx, const double* part, double* gx, double* gy, double* gz) {
   const int f = blockIdx.y;
@@ -1032,6 +1034,7 @@ __global__ void __launch_bounds__(kB)
   int i, j, k;
   face_point(g, f, t, i, j, k);
   double val = part[(size_t)f * mx + t];
+#pragma unroll 8
   for (int c = 1; c < nch; c++) val += part[((size_t)c * 6 + f) * mx + t];
   *face_slot(g, f, i, j, k, gx, gy, gz) = val;
 }
@@ -1755,12 +1758,16 @@ void mol_maps(hipStream_t s, const Geo& g, const unsigned char* atom_flags,
 
 // Chunks of the atom list: enough that the FP64 kernel's launch holds about
 // 2,048 workgroups (8 a CU; a 65^3 grid's faces alone are 30), of 16 atoms or
-// more.
-static int bc_mdh_chunks(const Geo& g, int natoms) {
+// more.  The FP32 kernel takes up to eight chunks of 512 atoms or more beyond
+// that: it holds four times the workgroups, of a quarter of the work, and on
+// large grids the rule's few chunks leave its last round of them short (353^3
+// with 5,000 atoms, two chunks 1422 us, eight 1368; 2,000 atoms 575, three 566).
+static int bc_mdh_chunks(const Geo& g, int natoms, bool fp32_terms) {
   const long mx = std::max((long)g.ny * g.nz, std::max((long)g.nx * g.nz, (long)g.nx * g.ny));
   const long groups = 6 * ((mx / kMdhRun + kB - 1) / kB);
   const long want = std::max(1L, 2048 / groups);
-  return (int)std::max(1L, std::min(want, (long)natoms / 16));
+  const long rule = std::max(1L, std::min(want, (long)natoms / 16));
+  return (int)(fp32_terms ? std::max(rule, std::min(8L, (long)natoms / 512)) : rule);
 }
 
 // Threads of the largest face: one per run of kMdhRun points.
@@ -1773,8 +1780,9 @@ size_t bc_mdh_scratch(const Geo& g, int natoms) {
   size_t mx = (size_t)g.ny * g.nz;
   if ((size_t)g.nx * g.nz > mx) mx = (size_t)g.nx * g.nz;
   if ((size_t)g.nx * g.ny > mx) mx = (size_t)g.nx * g.ny;
-  // partial sums, then the per-atom factors (FP64) or float4 atoms (two doubles each)
-  return (size_t)bc_mdh_chunks(g, natoms) * 6 * mx + 2 * (size_t)(natoms > 0 ? natoms : 1);
+  // partial sums (FP32 terms take as many chunks or more), then the per-atom
+  // factors (FP64) or float4 atoms (two doubles each)
+  return (size_t)bc_mdh_chunks(g, natoms, true) * 6 * mx + 2 * (size_t)(natoms > 0 ? natoms : 1);
 }
 
 void bc_mdh(hipStream_t s, const Geo& g, const double* xf, const double* yf, const double* zf,
@@ -1783,7 +1791,7 @@ void bc_mdh(hipStream_t s, const Geo& g, const double* xf, const double* yf, con
   int mx = g.ny * g.nz;
   if (g.nx * g.nz > mx) mx = g.nx * g.nz;
   if (g.nx * g.ny > mx) mx = g.nx * g.ny;
-  const int nch = bc_mdh_chunks(g, A.n);
+  const int nch = bc_mdh_chunks(g, A.n, fp32_terms);
   // the per-atom data follow the partial sums in the scratch buffer (6 * mx
   // * nch doubles: an even count, so the float4 array is 16-byte aligned)
   double* fac = part + (size_t)nch * 6 * mx;
