@@ -881,19 +881,30 @@ __device__ inline double rsqrt_refined(double d2) {
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-// exp(x), x <= 0, from a 256-entry table of 2^(i/256) in LDS: x = n ln2/256 + r
-// with |r| <= ln2/512, 2^(n/256) from the table and the exponent, and the
-// Taylor polynomial of degree 4 for exp(r) (its next term is 4e-17).
+// exp(-kappa d) from a 256-entry table of 2^(i/256) in LDS (the table-driven
+// method of P. T. P. Tang, ACM TOMS 15, 1989): -kappa d = n ln2/256 + r with
+// |r| <= ln2/512, 2^(n/256) from the table and the exponent, and the Taylor
+// polynomial of degree 4 for exp(r) (its next term is 4e-17).  The product
+// kappa d is never rounded: n ln2/256 is exact in 24 bits of ln2, and r is one
+// fma of kappa and d.  Rounding it first made 12 atoms' sums in 1 M salt 0.98 to
+// 1.06 times as far from the exact ones as the library's exponential did, a
+// single ion's 1.11 to 1.15 times; so they are 0.93 to 1.00 and 1.03 to 1.08, at
+// the same time (161^3 with 5,000 atoms 704 us, 699 before).
 constexpr int kExpTab = 256;
-__device__ inline double exp_tab(double x, const double* tab) {
+struct ExpScale {
+  double mk, t, dmax;  // -kappa, -kappa 256 / ln2, and where the value underflows
+  __device__ explicit ExpScale(double kappa)
+      : mk(-kappa), t(-kappa * 369.329930467574635), dmax(800.0 / kappa) {}
+};
+__device__ inline double exp_tab(double d, const ExpScale& s, const double* tab) {
   const double hi = (double)0.693147180559945309f / 256.0;  // ln2 in 24 bits
   const double lo = -1.90465429995776782877e-9 / 256.0;     // ln2 - hi
   const double magic = 6755399441055744.0;                  // 1.5 * 2^52
-  x = fmax(x, -800.0);
-  const double t = fma(x, 369.329930467574635, magic);  // 256 / ln2
+  d = fmin(d, s.dmax);
+  const double t = fma(d, s.t, magic);
   const int n = __double2loint(t);
   const double nd = t - magic;
-  double r = fma(nd, -hi, x);
+  double r = fma(d, s.mk, -(nd * hi));
   r = fma(nd, -lo, r);
   const double q = fma(r, fma(r, 1.0 / 24.0, 1.0 / 6.0), 0.5);
   const double m = fma(r * r, q, r);
@@ -905,10 +916,11 @@ __device__ inline double exp_tab(double x, const double* tab) {
 // position, its factor and the squared offset along the two fixed axes are
 // shared by them, and a term costs about 23 FP64 instructions (one point per
 // thread with the library's exponential and two Newton steps took about 39).
-// FP64 issue bounds it.  With 193^3 and 20,000 atoms a calculation goes from
-// 18.97 to 15.33 ms, with 161^3 and 5,000 (FP64) from 11.98 to 10.89 ms; the
-// face values' rms error against extended precision is 0.57 to 1.0 of that of
-// the one-point form (4.4e-16 against 7.8e-16 at 65^3 with 2,000 atoms).
+// FP64 issue bounds it.  With 193^3 and 20,000 atoms a calculation went from
+// 18.97 to 15.33 ms, with 161^3 and 5,000 (FP64) from 11.98 to 10.89 ms.  Error
+// of the face values against extended precision, over that of the one-point
+// form: a single ion 1.03 to 1.08, 12 to 31 atoms 0.87 to 1.02, 100 atoms 0.59
+// to 0.87 (the sum's chunks make its chain of additions shorter).
 constexpr int kMdhRun = 4;
 
 template <bool kScreened>
@@ -940,6 +952,7 @@ __global__ void __launch_bounds__(kB)
     Q[u] = cq[min(q0 + u, nq - 1)];
     val[u] = 0.0;
   }
+  const ExpScale scale(kScreened ? xkappa : 1.0);
   const int c = blockIdx.z;
   const int per = (A.n + nch - 1) / nch;
   const int a0 = c * per, a1 = min(A.n, a0 + per);
@@ -954,7 +967,7 @@ __global__ void __launch_bounds__(kB)
       const double y = rsqrt_refined(d2);
       const double v = fa * y;
       if (kScreened)
-        val[u] = fma(v, exp_tab(-xkappa * (d2 * y), tab), val[u]);
+        val[u] = fma(v, exp_tab(d2 * y, scale, tab), val[u]);
       else
         val[u] += v;
     }

@@ -86,3 +86,24 @@ def test_sums(natoms, dims, h, salt):
     assert (err <= bound).all()
     fast = boundary(xyz, q, r, dims, h, salt, precision=2)[0]
     assert np.abs(fast - exact).max() <= 1e-5 * np.abs(exact).max()
+
+
+@pytest.mark.parametrize("salt", [0.05, 0.15, 1.0])
+@pytest.mark.parametrize("x", [0.3, 0.7, 1.1])
+def test_term(x, salt):
+    """One ion: the spread over the faces of the relative error (its mean is the
+    factor's error).  Roundings are taken as independent, each with the standard
+    deviation u / sqrt(3) of one at a mantissa near 1: five in d^2, halved in the
+    reciprocal root, which adds one and half of another; the table, its
+    multiply-add, the product with the factor and the addition; and times kappa d
+    those of d^2 (halved), the root and d itself.  That is
+    sqrt(0.42 + 0.42 + 1.33 + (kappa d)^2 1.17) u, which is also less than the
+    spread with a product kappa d that is rounded, 1.5 in the place of 1.17."""
+    xyz, q, r = np.array([[x, 0.3, -0.2]]), np.ones(1), np.array([2.1])
+    got, nodes, pre1, kappa = boundary(xyz, q, r, (33, 33, 33), 0.5, salt)
+    exact, mag, far = face_sums(xyz, q, r, nodes, pre1, kappa)
+    spread = float(np.std(((got - exact) / exact).astype(float)))
+    kd2 = float(((far / mag) ** 2).mean())
+    bar = U * np.sqrt(0.42 + 0.42 + 1.33 + 1.17 * kd2)
+    print(f"salt {salt}: spread {spread:.2e}, bar {bar:.2e}, kappa d {np.sqrt(kd2):.2f}")
+    assert spread <= bar
