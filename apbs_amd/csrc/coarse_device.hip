@@ -652,31 +652,60 @@ static bool rows_fit(int nx, int word, int code) {
   return (2 * m + 1) * R <= 512 && (long)(2 * m + 4) * nx * word <= 64 * 1024;
 }
 
-// The rows form of a level, or 0.  Below rows of 40 points the square tiles
-// are faster (33^3: FP64 9.7 us a sweep against 10.8, FP32 9.0 against 9.8),
-// from 115 to 130 in FP64 the colour pairs no slower (129^3 94.2 against
-// 95.5).  FP32 takes 8-byte runs up to rows of 104 points (97^3 24.4 against
-// 25.4), 16-byte runs above (129^3 48.0 against 50.4).  m, the row pairs of a
-// workgroup, follows how its runs fill whole wavefronts and its tiles the 256
-// CUs: 3 up to 52 points and from 93 to 104 (49^3 FP64 m = 3 11.4, 4 13.3;
-// 97^3 41.8, 45.4), else 4 (65^3 m = 3 18.3, 4 15.4, 5 17.2; 81^3 30.3, 26.9,
-// 27.7), and 2 where 4 no longer fits or rows are longer than 144.
-static int rows_code(int nx, int word) {
+// Points of a run in the rows form of rows of nx points, or 0 for another form.
+// Below rows of 40 points the square tiles are faster (33^3: FP64 9.5 us a sweep
+// against 10.9, FP32 9.0 against 9.7), from 115 to 130 in FP64 the colour pairs
+// are the faster or close (117^3 77.3 against 74.5, 121^3 79.8 and 79.7, 125^3
+// 85.2 and 88.8, 129^3 92.8 and 95.3).  FP32 takes 8-byte runs up to rows of 104 points (89^3
+// 20.8 us against 21.3 with 16 bytes, 97^3 24.4 and 24.4), 16-byte runs above
+// (113^3 34.8 against 37.5, 129^3 47.9 and 50.5).
+static int rows_run(int nx, int word) {
   if (nx < 40 || (word == 8 && nx > 114 && nx <= 130)) return 0;
   const int kV = word == 4 && nx > 104 ? 4 : 2;
-  int m = kV == 4 ? (nx <= 144 ? 4 : 2) : (nx <= 52 || (nx > 92 && nx <= 104) ? 3 : 4);
-  while (m > 1 && !rows_fit(nx, word, 100 * kV + m)) m = m == 4 ? 2 : m - 1;
-  return rows_fit(nx, word, 100 * kV + m) ? 100 * kV + m : 0;
+  return rows_fit(nx, word, 100 * kV + 1) ? kV : 0;
+}
+
+// The rows form of nb levels swept together, or 0.  The row pairs m of a
+// workgroup, 1 to 6: a launch takes as long as the CU with the most work, which
+// runs ceil(workgroups / 256) workgroups of so many wavefronts each (and their
+// barriers, about half a wavefront's time), so m is the one that makes this
+// least, the largest on a tie, where fewer rows are computed twice.  us a sweep
+// (m: time): 49^3 FP64 2: 14.7, 3: 11.2, 4: 13.2; 65^3 3: 18.2, 4: 15.6, 5: 17.2;
+// 73^3 4: 23.5, 5: 24.0, 6: 20.4; 97^3 2: 45.3, 3: 42.0, 4: 45.5; eight levels
+// of 45^3 3: 37.8, 6: 32.9; FP32 81^3 4: 18.4, 5: 17.1.  Over 148 shapes (40 to
+// 177 points a row, ragged ones and batches of eight among them) the rule's m
+// is 1.2 % slower than the fastest on average; at worst 9 % (eight levels of
+// 105^3 in FP32) and 8 % (77^3, m = 2 for 3).
+static int rows_code(int nx, int ny, int nz, int word, int nb) {
+  const int kV = rows_run(nx, word);
+  if (kV == 0) return 0;
+  const int R = (nx - 2 + kV - 1) / kV;
+  int best = 0;
+  long least = 0;
+  for (int m = 1; m <= 6; m++) {
+    if (!rows_fit(nx, word, 100 * kV + m)) continue;
+    const long groups = (long)((ny - 2 + 2 * m - 1) / (2 * m)) * ((nz - 1) / 2) * nb;
+    const long cost = (groups + 255) / 256 * (2 * (((2 * m + 1) * R + 63) / 64) + 1);
+    if (best == 0 || cost <= least) {
+      best = 100 * kV + m;
+      least = cost;
+    }
+  }
+  return best;
 }
 
 // The square tiles are for levels of at most 49^2 points a plane: larger planes
 // with short rows take the colour pairs.
 bool gsrb27_use_planes(int nx, int ny, int nz, int word) {
-  return nz >= 3 && (rows_code(nx, word) != 0 || (nx <= 49 && ny <= 49));
+  return nz >= 3 && (rows_run(nx, word) != 0 || (nx <= 49 && ny <= 49));
 }
 
-int gsrb27_planes_tile(int nx, int ny, int nz, int word) {
-  if (const int code = rows_code(nx, word)) return code;
+bool gsrb27_planes_fits(int nx, int word, int tile) {
+  return tile == 8 || tile == 16 || rows_fit(nx, word, tile);
+}
+
+int gsrb27_planes_tile(int nx, int ny, int nz, int word, int nb) {
+  if (const int code = rows_code(nx, ny, nz, word, nb)) return code;
   const long groups = (long)((nx - 2 + 15) / 16) * ((ny - 2 + 15) / 16) * ((nz - 2) / 2);
   return groups >= 64 ? 16 : 8;
 }
@@ -687,9 +716,7 @@ void gsrb27_planes_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<
   check_batch(nb);
   if (nx < 3 || ny < 3 || nz < 3) return;
   constexpr int word = (int)sizeof(T);
-  if (tile != 8 && tile != 16 && tile != 32 && !(tile >= 100 && rows_fit(nx, word, tile)))
-    tile = gsrb27_planes_tile(nx, ny, nz, word);
-  if (tile == 32) tile = 16;
+  if (!gsrb27_planes_fits(nx, word, tile)) tile = gsrb27_planes_tile(nx, ny, nz, word, nb);
   const bool rows = tile >= 100;
   for (int it = 0; it < nu; it++) {
     // sweep it reads x (even it) or xs and writes the other one

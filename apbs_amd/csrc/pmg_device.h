@@ -69,13 +69,14 @@ void gsrb27(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D, 
 // of the even or odd planes), ping-ponging between x and xs (level-size
 // scratch).  Only interior points are written, so x and xs must hold the same
 // boundary values (zero on the coarse levels).  Bitwise the result of gsrb27,
-// ending in x.  tile: 8 or 16 (square tiles of a plane; 32 takes 16), or
-// 100 kV + m (2m whole rows a workgroup, runs of kV points a lane) where that
-// fits the row; other values take gsrb27_planes_tile.
+// ending in x.  tile: 8 or 16 (square tiles of a plane) or 100 kV + m (2m whole
+// rows a workgroup, runs of kV points a lane) where that fits the row
+// (gsrb27_planes_fits); other values take gsrb27_planes_tile.
 template <class T>
 void gsrb27_planes(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D,
                    const T* fc, T* x, T* xs, int nu, int iadjoint, int tile = 0);
-int gsrb27_planes_tile(int nx, int ny, int nz, int word);
+bool gsrb27_planes_fits(int nx, int word, int tile);
+int gsrb27_planes_tile(int nx, int ny, int nz, int word, int nb = 1);
 // The same 8-colour sweeps in place with the two colours of each (j, k)
 // parity (c, c ^ 1) in one launch, one wavefront per row: 4 launches per
 // sweep.  Rows of up to 128 interior points (nx <= 130).  Bitwise gsrb27.

@@ -151,6 +151,32 @@ def test_row_tiles_fp32_bitwise(L, n3, code):
             assert np.array_equal(out[0], out[1]), (adj, nu)
 
 
+@pytest.mark.parametrize("n3", [(40, 5, 4), (45, 9, 9), (49, 97, 33), (41, 33, 97), (45, 33, 97),
+                                (69, 67, 69), (73, 73, 73), (105, 111, 41), (145, 41, 17)])
+def test_row_rule_bitwise(L, n3):
+    """The sweep in the form the dispatch takes, on levels for which the rule
+    gives 1 to 6 row pairs a workgroup, in FP64 against the oracle and in FP32
+    against one launch per colour, bit for bit."""
+    fp = ctypes.POINTER(ctypes.c_float)
+    nx, ny, nz = n3
+    a, cc, fc, x0 = _level(n3, sum(n3))
+    af, cf, ff, xf = (v.astype(np.float32) for v in (a, cc, fc, x0))
+    D = af[:nx * ny * nz] + cf
+    for adj in (0, 1):
+        xg, xo = x0.copy(), x0.copy()
+        assert L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), 2, adj, 1) == 1
+        od.lib().orc_gsrb(nx, ny, nz, 27, P(a), P(cc), P(fc), P(xo), 2, adj, 1)
+        assert np.array_equal(xg, xo), adj
+        out = []
+        for mode in (1, 0):
+            x = xf.copy()
+            assert L.pmgtest_gsrb27_32(nx, ny, nz, af.ctypes.data_as(fp), D.ctypes.data_as(fp),
+                                       ff.ctypes.data_as(fp), x.ctypes.data_as(fp), 2, adj,
+                                       mode) == 1
+            out.append(x)
+        assert np.array_equal(out[0], out[1]), adj
+
+
 @pytest.mark.parametrize("n3", [(17, 19, 21), (33, 33, 33), (67, 13, 20), (130, 6, 11), (7, 70, 3),
                                 (4, 5, 6)])
 @pytest.mark.parametrize("code", [101, 202, 204, 302, 402, 404])
