@@ -54,6 +54,8 @@ void gsrb7_fused(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T
 int gsrb7_fused_launches(int nu);
 // One sweep of the block form (code 100 TY + KC: TY rows of KC planes a
 // workgroup) from x to xs, or from xs to x with flip.  Bitwise the fused sweep.
+// In a tile shape of the fused sweep a block shape is kBlockTile + its code.
+constexpr int kBlockTile = 9000000;
 template <class T>
 struct LevelArgs;
 bool block_sweep_fits(int nx, int word, int code);

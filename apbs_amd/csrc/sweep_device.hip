@@ -510,8 +510,6 @@ int fused_tile(int nx, int ny, int nz, int word) {
   return n <= 20000000L ? 7412 : 807412;
 }
 
-constexpr int kBlockTile = 9000000;  // tile codes of block shapes: this + 100 TY + KC
-
 // Block shape (block_sweep_device.hip) of nb grids swept together, or 0 where
 // the march is the faster: above 1.5M points in all in FP64 (113^3 26.5 us a
 // sweep against 29.7, 129^3 32.3 against 31.9) and 3.1M in FP32 (145^3 22.4

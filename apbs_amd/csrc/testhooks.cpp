@@ -28,6 +28,16 @@ double* up(const double* h, size_t n) {
 void down(double* h, const double* d, size_t n) {
   TCHECK(hipMemcpy(h, d, n * sizeof(double), hipMemcpyDeviceToHost));
 }
+// Whether a forced form is one the kernels have for rows of nx points: a tile of
+// the fused 7-point sweep (0 the default, block shapes where they fit), a mode of
+// the 27-point one (see the header).
+bool tile7_ok(int nx, int word, int tile) {
+  return tile < pmg::kBlockTile || pmg::block_sweep_fits(nx, word, tile - pmg::kBlockTile);
+}
+bool mode27_ok(int nx, int word, int mode) {
+  if (mode >= 2 && mode <= 4) return nx <= 130 && (mode != 4 || word == 4);
+  return mode == 0 || mode == 1 || pmg::gsrb27_planes_fits(nx, word, mode);
+}
 struct OpsHolder {
   std::vector<double*> ptr;
   pmg::Ops<double> ops{};
@@ -186,6 +196,7 @@ int pmgtest_stream_copy(size_t n, int reps) {
 // or 4 (FP32); sweeps even and positive; tile 0 = the library's default.
 int pmgtest_fused_sweeps(int n, int word, int sweeps, int tile, double* us_per_sweep) {
   if (n < 3 || sweeps <= 0 || (sweeps & 1) || (word != 4 && word != 8)) return 0;
+  if (!tile7_ok(n, word, tile)) return 0;
   *us_per_sweep = word == 8 ? fused_sweeps_us<double>(n, sweeps, tile)
                             : fused_sweeps_us<float>(n, sweeps, tile);
   return 1;
@@ -211,24 +222,20 @@ int pmgtest_dense_invert(int N, const double* M, double* out, int form) {
 // Average microseconds per Galerkin call on a synthetic nf^3 level (see
 // galerkin_us); form as pmgtest_galerkin_form
 int pmgtest_galerkin_time(int nf, int st, int form, int reps, double* us) {
-  if (nf < 5 || (nf & 1) == 0 || (st != 7 && st != 27) || reps <= 0 || form < 0 || form > 4) return 0;
+  if (nf < 5 || (nf & 1) == 0 || (st != 7 && st != 27) || reps <= 0 || form < 0 || form > 2) return 0;
   *us = galerkin_us(nf, st, form, reps);
   return 1;
 }
 
 // Average microseconds per 27-point sweep on an n^3 level (see gs27_sweeps_us)
 int pmgtest_gs27_sweeps(int n, int word, int sweeps, int mode, double* us_per_sweep) {
-  if (n < 3 || sweeps <= 0 || (word != 4 && word != 8)) return 0;
+  if (n < 3 || sweeps <= 0 || (word != 4 && word != 8) || !mode27_ok(n, word, mode)) return 0;
   *us_per_sweep = word == 8 ? gs27_sweeps_us<double>(n, sweeps, mode)
                             : gs27_sweeps_us<float>(n, sweeps, mode);
   return 1;
 }
 
-// 27-point sweeps with the kernel form forced: mode 0 one launch per colour,
-// 1 per plane parity (tile by level size), 2 per colour pair (rows of up to
-// 128 interior points; the vector kernel where the row allows it), 3 per
-// colour pair with one point per lane, 8 / 16 / 32 per plane parity with
-// that tile
+// 27-point sweeps with the kernel form forced (see the header)
 int pmgtest_gsrb27_mode(int nx, int ny, int nz, const double* a, const double* cc,
                         const double* fc, double* x, int nu, int iadjoint, int mode) {
   return gsrb_impl(nx, ny, nz, 27, a, cc, fc, x, nu, iadjoint, mode);
@@ -252,6 +259,7 @@ int pmgtest_gsrb_tile(int nx, int ny, int nz, const double* a, const double* cc,
 // default shape).  The result is written back to x.
 int pmgtest_gsrb_zero(int nx, int ny, int nz, const double* a, const double* cc,
                       const double* fc, double* x, int iadjoint, int tile) {
+  if (!tile7_ok(nx, 8, tile)) return 0;
   const size_t n = (size_t)nx * ny * nz;
   OpsHolder A(a, n, 7);
   double *dcc = up(cc, n), *dfc = up(fc, n), *dx = up(x, n), *dD = up(nullptr, n);
@@ -270,6 +278,7 @@ int pmgtest_gsrb_zero(int nx, int ny, int nz, const double* a, const double* cc,
 
 int gsrb_impl(int nx, int ny, int nz, int st, const double* a, const double* cc, const double* fc,
               double* x, int nu, int iadjoint, int tile) {
+  if (st == 7 ? !tile7_ok(nx, 8, tile) : !mode27_ok(nx, 8, tile)) return 0;
   const size_t n = (size_t)nx * ny * nz;
   OpsHolder A(a, n, st);
   double *dcc = up(cc, n), *dfc = up(fc, n), *dx = up(x, n), *dD = up(nullptr, n);
@@ -284,7 +293,6 @@ int gsrb_impl(int nx, int ny, int nz, int st, const double* a, const double* cc,
   } else if (tile == 0) {
     pmg::gsrb27<double>(0, nx, ny, nz, A.ops, dD, dfc, dx, nu, iadjoint);
   } else if (tile == 2 || tile == 3) {
-    if (nx > 130) return 0;
     const pmg::LevelArgs<double> c{A.ops, dD, dfc, dx, nullptr, nullptr};
     pmg::gsrb27_pairs_form<double>(0, nx, ny, nz, &c, 1, nu, iadjoint, tile - 2);
   } else {
@@ -378,7 +386,6 @@ int pmgtest_restrict(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, const
   return 1;
 }
 
-// xf_out = xf + damp * P xc on the fine interior
 int pmgtest_restrict_diag(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, int nb,
                           const double* in, const double* oC, double* out, double* D, float* Df) {
   if (nb < 1 || nb > pmg::kMaxBatch) return 0;
@@ -400,6 +407,7 @@ int pmgtest_restrict_diag(int nxf, int nyf, int nzf, int nxc, int nyc, int nzc, 
   return 1;
 }
 
+// xf_out = xf + damp * P xc on the fine interior
 int pmgtest_prolong(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, const double* xc,
                     double* xf, double damp) {
   const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;
@@ -431,7 +439,7 @@ int pmgtest_prolong32(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, cons
 
 int pmgtest_galerkin_form(int nxf, int nyf, int nzf, int st, const double* af, int nxc, int nyc,
                           int nzc, double* ac, int form) {
-  if (form < 0 || form > 4) return 0;
+  if (form < 0 || form > 2) return 0;
   const size_t nf = (size_t)nxf * nyf * nzf, nc = (size_t)nxc * nyc * nzc;
   OpsHolder A(af, nf, st);
   double* out[14];
@@ -507,7 +515,7 @@ int pmgtest_nonlinear(int nx, int ny, int nz, const double* a, const double* cc,
 int pmgtest_fused32(int nx, int ny, int nz, const float* oE, const float* oN, const float* uC,
                     const float* D, const float* fc, float* x, int nu, int iadjoint, int tile,
                     int zero) {
-  if (nx < 3 || ny < 3 || nz < 3 || (!zero && nu < 1)) return 0;
+  if (nx < 3 || ny < 3 || nz < 3 || (!zero && nu < 1) || !tile7_ok(nx, 4, tile)) return 0;
   const size_t n = (size_t)nx * ny * nz;
   auto upf = [&](const float* h) {
     float* d = nullptr;
@@ -532,8 +540,7 @@ int pmgtest_fused32(int nx, int ny, int nz, const float* oE, const float* oN, co
 // FP32 27-point sweeps in a given form on explicit arrays (see the header)
 int pmgtest_gsrb27_32(int nx, int ny, int nz, const float* a, const float* D, const float* fc,
                       float* x, int nu, int iadjoint, int mode) {
-  if (nx < 3 || ny < 3 || nz < 3 || nu < 1) return 0;
-  if (mode >= 2 && mode <= 4 && nx > 130) return 0;
+  if (nx < 3 || ny < 3 || nz < 3 || nu < 1 || !mode27_ok(nx, 4, mode)) return 0;
   const size_t n = (size_t)nx * ny * nz;
   auto upf = [&](const float* h) {
     float* d = nullptr;

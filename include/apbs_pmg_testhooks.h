@@ -45,10 +45,10 @@ int pmgtest_prolong32(int nxc, int nyc, int nzc, int nxf, int nyf, int nzf, cons
 /* VbuildG_7 / VbuildG_27 (src/pmgc/buildGd.c:450-3115) */
 int pmgtest_galerkin(int nxf, int nyf, int nzf, int stencil, const double *af, int nxc, int nyc,
                      int nzc, double *ac);
-/* The same with the kernel form forced: 1 one thread per coefficient, 2 one
- * 32-lane group per coefficient, 0, 3 or 4 the solver's kernel (loops unrolled
- * at compile time, directions that share their loads in one thread); all give
- * the same bits */
+/* The same with the kernel form forced: 0 the solver's kernel (loops unrolled
+ * at compile time, directions that share their loads in one thread), 1 one
+ * thread per coefficient, 2 one 32-lane group per coefficient; all give the
+ * same bits.  0 on other forms. */
 int pmgtest_galerkin_form(int nxf, int nyf, int nzf, int stencil, const double *af, int nxc,
                           int nyc, int nzc, double *ac, int form);
 /* VbuildA_fv (src/pmgc/buildAd.c:105-281) */
@@ -62,7 +62,8 @@ int pmgtest_nonlinear(int nx, int ny, int nz, const double *a, const double *cc,
                       const double *fc, const double *x, int nion, const double *q,
                       const double *sconc, double *out_r, double *out_d);
 /* pmgtest_gsrb (7-point) with an explicit tile shape of the fused sweep
- * (rows*100 + planes: 416, 48, 816, 88, 84, 1616, 832). */
+ * (rows*100 + planes: 416, 48, 816, 88, 84, 1616, 832), or a block shape
+ * (9000000 + rows*100 + planes); returns 0 where a block does not fit the row. */
 int pmgtest_gsrb_tile(int nx, int ny, int nz, const double *a, const double *cc,
                       const double *fc, double *x, int nu, int iadjoint, int tile);
 /* Two fused 7-point sweeps from a zero start (the first smoothing of a
@@ -80,13 +81,14 @@ int pmgtest_fused32(int nx, int ny, int nz, const float *oE, const float *oN, co
                     int zero);
 /* pmgtest_gsrb (27-point) with the kernel form forced: mode 0 one launch per
  * colour, 1 one launch per plane parity (tile by level size), 2 one launch
- * per colour pair (nx <= 130, else returns 0; the vector kernel where the
- * row allows it), 3 the colour pair with one point per lane, 8 / 16 / 32 one
- * launch per plane parity with that square tile.  All give the same bits. */
+ * per colour pair (nx <= 130; the vector kernel where the row allows it), 3 the
+ * colour pair with one point per lane, 4 (FP32) the vector kernel with 8-byte runs,
+ * 8 / 16 one launch per plane parity with that square tile, 100 kV + m with 2m
+ * whole rows and runs of kV points.  All give the same bits; returns 0 where
+ * the form does not fit the row. */
 int pmgtest_gsrb27_mode(int nx, int ny, int nz, const double *a, const double *cc,
                         const double *fc, double *x, int nu, int iadjoint, int mode);
-/* FP32 27-point sweeps in a given form (mode as pmgtest_gsrb27_mode, and 4
- * the colour-pair vector kernel with 8-byte runs) on
+/* FP32 27-point sweeps in a given form (mode as pmgtest_gsrb27_mode) on
  * explicit arrays: a holds the 14 stencil arrays (oC first, unused), D the
  * diagonal; every array nx*ny*nz floats.  Result in x; 0 on bad sizes. */
 int pmgtest_gsrb27_32(int nx, int ny, int nz, const float *a, const float *D, const float *fc,

@@ -110,29 +110,49 @@ def _level(n3, seed):
         x.reshape(-1)
 
 
-@pytest.mark.parametrize("n3", [(17, 17, 17), (9, 11, 13), (45, 43, 41), (4, 5, 4), (70, 21, 6),
-                                (81, 81, 9), (131, 8, 7), (177, 13, 5)])
-@pytest.mark.parametrize("code", [201, 202, 203, 205, 210])
+def _rows_fit(nx, word, code):
+    """A tile of 2m rows in runs of kV points: at most 512 lanes and 64 KB."""
+    kv, m = divmod(code, 100)
+    runs = -(-(nx - 2) // kv)
+    return (2 * m + 1) * runs <= 512 and (2 * m + 4) * nx * word <= 65536 and nx >= kv + 2
+
+
+def _block_fits(nx, word, code):
+    """TY rows of KC planes and their halo: at most 1,024 lanes and 64 KB."""
+    ty, kc = divmod(code, 100)
+    kv = 16 // word
+    runs = -(-(nx - 2) // kv)
+    return (runs * ((ty + 2) * kc + 2 * ty) <= 1024 and
+            (kc + 2) * (ty + 2) * nx * word <= 65536 and nx >= kv + 2)
+
+
+def _fitting(shapes, codes, word, fits):
+    return [(n3, c) for n3 in shapes for c in codes if fits(n3[0], word, c)]
+
+
+@pytest.mark.parametrize("n3,code", _fitting(
+    [(17, 17, 17), (9, 11, 13), (45, 43, 41), (4, 5, 4), (70, 21, 6), (81, 81, 9), (131, 8, 7),
+     (177, 13, 5)], [201, 202, 203, 204, 205, 206, 210], 8, _rows_fit))
 def test_row_tiles_bitwise(L, n3, code):
     """The whole-row plane sweep (code 100 kV + m: runs of kV points, 2m rows
     a workgroup) against the oracle's 8-colour sweep, bit for bit: partial
     tiles, rows of 2 to 175 points, odd ends of the last run, both orders and
-    odd and even sweep counts.  Codes that do not fit a row take the square
-    tiles."""
+    odd and even sweep counts."""
     nx, ny, nz = n3
     a, cc, fc, x0 = _level(n3, sum(n3) + code)
     O = od.lib()
     for adj in (0, 1):
         for nu in (2, 3):
             xg, xo = x0.copy(), x0.copy()
-            L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj, code)
+            assert L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj,
+                                         code) == 1
             O.orc_gsrb(nx, ny, nz, 27, P(a), P(cc), P(fc), P(xo), nu, adj, 1)
             assert np.array_equal(xg, xo), (adj, nu)
 
 
-@pytest.mark.parametrize("n3", [(17, 17, 17), (9, 11, 13), (45, 43, 41), (6, 5, 4), (81, 81, 9),
-                                (131, 8, 7), (178, 13, 5)])
-@pytest.mark.parametrize("code", [203, 401, 402, 404, 405, 410])
+@pytest.mark.parametrize("n3,code", _fitting(
+    [(17, 17, 17), (9, 11, 13), (45, 43, 41), (6, 5, 4), (81, 81, 9), (131, 8, 7), (178, 13, 5)],
+    [203, 206, 401, 402, 404, 405, 406, 410], 4, _rows_fit))
 def test_row_tiles_fp32_bitwise(L, n3, code):
     """The FP32 rows forms (8- and 16-byte runs) against one launch per colour."""
     fp = ctypes.POINTER(ctypes.c_float)
@@ -177,9 +197,9 @@ def test_row_rule_bitwise(L, n3):
         assert np.array_equal(out[0], out[1]), adj
 
 
-@pytest.mark.parametrize("n3", [(17, 19, 21), (33, 33, 33), (67, 13, 20), (130, 6, 11), (7, 70, 3),
-                                (4, 5, 6)])
-@pytest.mark.parametrize("code", [101, 202, 204, 302, 402, 404])
+@pytest.mark.parametrize("n3,code", _fitting(
+    [(17, 19, 21), (33, 33, 33), (67, 13, 20), (130, 6, 11), (7, 70, 3), (4, 5, 6)],
+    [101, 202, 203, 204, 302, 303, 402, 404], 8, _block_fits))
 def test_block_sweep_bitwise(L, n3, code):
     """The block form of the fused red-black sweep (100 TY + KC: TY rows of KC
     planes) against the oracle's sweep, bit for bit, boundary values not zero:
@@ -198,13 +218,15 @@ def test_block_sweep_bitwise(L, n3, code):
     for adj in (0, 1):
         for nu in (1, 2, 3):
             xg, xo = x0.copy(), x0.copy()
-            L.pmgtest_gsrb_tile(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj, 9000000 + code)
+            assert L.pmgtest_gsrb_tile(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj,
+                                       9000000 + code) == 1
             O.orc_gsrb(nx, ny, nz, 7, P(a), P(cc), P(fc), P(xo), nu, adj, 1)
             assert np.array_equal(xg, xo), (adj, nu)
 
 
-@pytest.mark.parametrize("n3", [(33, 33, 33), (67, 13, 20), (6, 5, 6), (130, 6, 11)])
-@pytest.mark.parametrize("code", [101, 202, 204, 402, 404])
+@pytest.mark.parametrize("n3,code", _fitting(
+    [(33, 33, 33), (67, 13, 20), (6, 5, 6), (130, 6, 11)], [101, 202, 203, 204, 305, 402, 404], 4,
+    _block_fits))
 def test_block_sweep_fp32_bitwise(L, n3, code):
     """The FP32 block form against the scalar march (tile 48), from a given and
     from a zero start (the interior then holds NaN and is not read)."""
@@ -230,6 +252,33 @@ def test_block_sweep_fp32_bitwise(L, n3, code):
                                          adj, tile, zero) == 1
                 out.append(x)
             assert np.array_equal(out[0], out[1]), (zero, adj)
+
+
+def test_forms_that_do_not_fit_are_refused(L):
+    """A forced form that a row does not fit is refused, not replaced by
+    another; the largest that fits is taken."""
+    fp = ctypes.POINTER(ctypes.c_float)
+    for nx, word, code in ((70, 8, 207), (70, 8, 208), (131, 4, 407), (131, 4, 408)):
+        n = nx * 4 * 4
+        ok = int(_rows_fit(nx, word, code))
+        assert ok == (code % 100 == 7)
+        one, f32 = np.ones(14 * n), np.ones(14 * n, np.float32)
+        if word == 8:
+            got = L.pmgtest_gsrb27_mode(nx, 4, 4, P(one), P(one), P(one), P(one.copy()), 1, 0, code)
+        else:
+            p = f32.ctypes.data_as(fp)
+            got = L.pmgtest_gsrb27_32(nx, 4, 4, p, p, p, f32.copy().ctypes.data_as(fp), 1, 0, code)
+        assert got == ok, (nx, word, code)
+    for nx, code in ((130, 203), (130, 204)):
+        one = np.ones(4 * nx * 4 * 4)
+        assert _block_fits(nx, 8, code) == (code == 203)
+        for f in (lambda t: L.pmgtest_gsrb_tile(nx, 4, 4, P(one), P(one), P(one), P(one.copy()), 2,
+                                                0, t),
+                  lambda t: L.pmgtest_gsrb_zero(nx, 4, 4, P(one), P(one), P(one), P(one.copy()), 0,
+                                                t)):
+            assert f(9000000 + code) == int(code == 203)
+    one = np.ones(14 * 64)
+    assert L.pmgtest_gsrb27_mode(4, 4, 4, P(one), P(one), P(one), P(one.copy()), 1, 0, 32) == 0
 
 
 @pytest.mark.parametrize("st", [7, 27])

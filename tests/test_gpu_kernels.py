@@ -73,13 +73,13 @@ def test_gsrb_bitwise(L, O, st, n3, adj):
 
 @pytest.mark.parametrize("n3", [(17, 17, 17), (9, 11, 13), (45, 43, 41), (5, 5, 4),
                                 (70, 21, 6), (81, 81, 9), (3, 3, 3), (130, 7, 6), (129, 6, 7)])
-@pytest.mark.parametrize("mode", [1, 2, 3, 8, 16, 32])
+@pytest.mark.parametrize("mode", [1, 2, 3, 8, 16])
 def test_gsrb27_plane_sweeps_bitwise(L, O, n3, mode):
     """The plane-parity 27-point sweep (one launch per plane parity, tiles
     with recomputed margins) and the colour-pair sweep (mode 2 the vector
     kernel, 16-byte runs per lane; mode 3 one wavefront per row) give the
-    oracle's 8-colour sweep bit for bit: every
-    tile size, partial tiles, forward and adjoint, even and odd sweep
+    oracle's 8-colour sweep bit for bit: both
+    square tiles, partial tiles, forward and adjoint, even and odd sweep
     counts, rows of 1 to 128 interior points."""
     rng = np.random.default_rng(sum(n3) + mode)
     nx, ny, nz = n3
@@ -91,7 +91,8 @@ def test_gsrb27_plane_sweeps_bitwise(L, O, n3, mode):
     for adj in (0, 1):
         for nu in (2, 3):
             xg, xo = x0.copy(), x0.copy()
-            L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj, mode)
+            assert L.pmgtest_gsrb27_mode(nx, ny, nz, P(a), P(cc), P(fc), P(xg), nu, adj,
+                                         mode) == 1
             O.orc_gsrb(nx, ny, nz, 27, P(a), P(cc), P(fc), P(xo), nu, adj, 1)
             assert np.array_equal(xg, xo), (n3, mode, adj, nu)
 
@@ -323,16 +324,15 @@ def test_transfers_bitwise(L, O):
     assert np.array_equal(interior(fg, f3), interior(fo, f3))
 
 
-@pytest.mark.parametrize("form", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("st,f3,c3", [(7, (17, 17, 17), (9, 9, 9)),
                                       (27, (17, 17, 17), (9, 9, 9)),
                                       (7, (65, 57, 61), (33, 29, 31)),
                                       (27, (65, 57, 61), (33, 29, 31))])
 def test_galerkin_bitwise(L, O, st, f3, c3, form):
-    """Every kernel form (one thread, one 32-lane group, one thread with the
-    loops unrolled at compile time per coefficient) and the size-based
-    choice; the 33x29x31 level has more coarse points than the group form's
-    cut-off, so form 0 takes a per-thread kernel there."""
+    """The solver's kernel (form 0) and the general sum by one thread and by one
+    32-lane group per coefficient, on a small level and on one of many partial
+    workgroups."""
     rng = np.random.default_rng(5 + st)
     nf, nc = np.prod(f3), np.prod(c3)
     af = rand_op(rng, f3, st)
