@@ -375,6 +375,13 @@ void dense_assemble_invert_batch(hipStream_t s, int nx, int ny, int nz, int N,
   dense_invert_batch(s, B, N, nb, form);
 }
 
+void dense_invert_batch(hipStream_t s, int N, const InvertArgs* c, int nb, int form) {
+  check_batch(nb);
+  Batch<InvertArgs> B;
+  for (int b = 0; b < nb; b++) B.v[b] = c[b];
+  dense_invert_batch(s, B, N, nb, form);
+}
+
 void dense_assemble(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* D,
                     double* M, int N) {
   Batch<InvertArgs> B;
@@ -383,9 +390,8 @@ void dense_assemble(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A,
 }
 
 void dense_invert(hipStream_t s, double* M, double* work, int N, int form, double* flag) {
-  Batch<InvertArgs> B;
-  B.v[0] = InvertArgs{Ops<double>{}, nullptr, M, work, flag};
-  dense_invert_batch(s, B, N, 1, form);
+  const InvertArgs c{Ops<double>{}, nullptr, M, work, flag};
+  dense_invert_batch(s, N, &c, 1, form);
 }
 
 template <class T>

@@ -384,6 +384,8 @@ struct InvertArgs {
 };
 void dense_assemble_invert_batch(hipStream_t s, int nx, int ny, int nz, int N,
                                  const InvertArgs* c, int nb, int form = 0);
+// The inverses alone, of matrices that are assembled (A and D are not read).
+void dense_invert_batch(hipStream_t s, int N, const InvertArgs* c, int nb, int form = 0);
 
 // ----------------------------------------------------- coarsest level (dense)
 // Assemble the dense (N x N) operator of the interior of a 27-point level with

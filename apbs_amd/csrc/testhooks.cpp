@@ -219,6 +219,28 @@ int pmgtest_dense_invert(int N, const double* M, double* out, int form) {
   return 1;
 }
 
+// The pivot flags of nb inverses of N x N matrices (one after another) in one
+// launch, as a batched solve makes them: 0, or the 1-based first bad pivot.
+int pmgtest_dense_pivots(int N, int nb, const double* M, double* flags) {
+  if (N <= 0 || N > 4096 || nb < 1 || nb > pmg::kMaxBatch) return 0;
+  const size_t nn = (size_t)N * N;
+  double *dM = up(M, nb * nn), *dw = up(nullptr, nb * pmg::dense_work(N)), *hf = nullptr;
+  TCHECK(hipHostMalloc(&hf, nb * sizeof(double), hipHostMallocDefault));
+  pmg::InvertArgs c[pmg::kMaxBatch];
+  for (int b = 0; b < nb; b++) {
+    hf[b] = 0.0;
+    c[b] = pmg::InvertArgs{pmg::Ops<double>{}, nullptr, dM + b * nn, dw + b * pmg::dense_work(N),
+                           hf + b};
+  }
+  pmg::dense_invert_batch(0, N, c, nb);
+  TCHECK(hipDeviceSynchronize());
+  for (int b = 0; b < nb; b++) flags[b] = hf[b];
+  TCHECK(hipFree(dM));
+  TCHECK(hipFree(dw));
+  TCHECK(hipHostFree(hf));
+  return 1;
+}
+
 // Average microseconds per Galerkin call on a synthetic nf^3 level (see
 // galerkin_us); form as pmgtest_galerkin_form
 int pmgtest_galerkin_time(int nf, int st, int form, int reps, double* us) {

@@ -105,6 +105,10 @@ int pmgtest_gs27_sweeps(int n, int word, int sweeps, int mode, double *us_per_sw
  * band form, mgsubd.c:244-255): the dense inverse of the coarsest level's
  * operator, form 0 (by size: registers for N <= 64) or 1 (LDS / blocks). */
 int pmgtest_dense_invert(int N, const double *M, double *out, int form);
+/* No reference counterpart: the pivot flags of nb such inverses (matrices one
+ * after another) made in one launch: 0, or the 1-based index of the first pivot
+ * that is not positive and finite (mlinpckd.c:194-233). */
+int pmgtest_dense_pivots(int N, int nb, const double *M, double *flags);
 /* No reference counterpart: microseconds per Galerkin call (form as above)
  * on a synthetic nf^3 operator of stencil st (nf odd). */
 int pmgtest_galerkin_time(int nf, int st, int form, int reps, double *us);

@@ -52,18 +52,22 @@ def check_same(alone, batched, label):
         assert (sb["iters"], sb["inner"], sb["outer"]) == (sa["iters"], sa["inner"], sa["outer"])
 
 
+@pytest.mark.parametrize("dime", [49, 57, 97])
 @pytest.mark.parametrize("npbe,precision", [(False, 0), (False, 1), (True, 0), (True, 1)])
-def test_batch_equals_alone(npbe, precision):
+def test_batch_equals_alone(npbe, precision, dime):
+    """49^3; 57^3, whose coarsest grids (8^3) are inverted by blocks of pivots,
+    each with its own panels; 97^3, whose first coarse levels take a row tile
+    chosen for the whole batch."""
     mols = molecules(5, 40)
     alone = []
     for m in mols:
-        c = calc(m, 49, npbe, precision)
+        c = calc(m, dime, npbe, precision)
         c.solve()
         alone.append(results(c))
         c.release()
-    calcs = [calc(m, 49, npbe, precision) for m in mols]
+    calcs = [calc(m, dime, npbe, precision) for m in mols]
     assert driver.solve_batch(calcs) == [1] * len(calcs)
-    check_same(alone, [results(c) for c in calcs], f"npbe {npbe} precision {precision}")
+    check_same(alone, [results(c) for c in calcs], f"npbe {npbe} precision {precision} {dime}^3")
     iters = {r[2]["iters"] for r in alone}
     if npbe:
         print(f"Newton step counts in the batch: {sorted(iters)}")

@@ -50,6 +50,44 @@ def test_blocked_dense_inverse(L, N):
     assert np.abs(A @ out - np.eye(N)).max() <= tol
 
 
+@pytest.mark.parametrize("N", [27, 64, 80, 90, 128, 216, 1000])
+def test_first_bad_pivot_is_reported(L, N):
+    """Matrices inverted in one launch, in the register, LDS and blocked forms:
+    positive definite ones are not flagged; one whose leading minors are positive
+    up to row p is flagged p + 1, in the first block of pivots, at a block's first
+    and last row and in the partial last block; of several bad pivots, in one
+    block or in two, the first; a NaN as well."""
+    rng = np.random.default_rng(N)
+    A = rng.uniform(-1, 0, (N, N))
+    A = 0.5 * (A + A.T)
+    np.fill_diagonal(A, 0.0)
+    A[np.diag_indices(N)] = -A.sum(axis=1) + rng.uniform(0.5, 2.0, N)
+    rows = sorted({0, 5, min(63, N - 1), min(64, N - 1), min(127, N - 2), N - 1})
+    mats, want = [A], [0]
+    for p in rows:
+        B = A.copy()
+        B[p, p] = -1.0 - np.abs(A[p]).sum()
+        mats.append(B)
+        want.append(p + 1)
+    for first, second in ((3, 9), (min(20, N - 2), N - 1)):
+        B = A.copy()
+        B[second, second] = -1.0e6
+        B[first, first] = -1.0e6
+        mats.append(B)
+        want.append(first + 1)
+    B = A.copy()
+    B[N // 2, N // 2] = np.nan
+    mats.append(B)
+    want.append(N // 2 + 1)
+    got = []
+    for b in range(0, len(mats), 8):
+        m = np.ascontiguousarray(np.stack(mats[b:b + 8]))
+        flags = np.full(len(m), -1.0)
+        assert L.pmgtest_dense_pivots(N, len(m), P(m), P(flags)) == 1
+        got += list(flags)
+    assert got == want
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("dims", [(57, 57, 57), (49, 57, 57)])
 def test_solve_on_a_large_coarsest_grid(dims, precision):

@@ -19,15 +19,15 @@ from apbs_amd import driver, synth
 
 pytestmark = pytest.mark.gpu
 
-DIME, H = 33, 0.5
+H = 0.5
 
 
-def calc(diel, precision, npbe):
+def calc(diel, precision, npbe, dime):
     atoms = synth.globule(30, (4.0,) * 3, 5, net_charge=1)[:3]
     mol = driver.Molecule(*atoms)
     c = mol.center
-    origin = c - 10.0
-    shape = (43, 43, 43)
+    origin = c - 0.25 * (dime - 1) - 2.0  # (the box and 2 A around it)
+    shape = (dime + 10,) * 3
     maps = {k: driver.Map(np.full(shape, diel), origin, (0.5,) * 3)
             for k in ("dielx", "diely", "dielz")}
     ions = [(1, 0.0, 2.0), (-1, 0.0, 2.0)]
@@ -36,15 +36,20 @@ def calc(diel, precision, npbe):
         ions = [(1, 0.15, 2.0), (-1, 0.15, 2.0)]
     pbe = dict(pdie=2.0, sdie=78.54, srfm="spl2", chgm="spl2", swin=0.3, srad=1.4, sdens=10.0,
                temp=298.15, bcfl="mdh", ions=ions, npbe=npbe, maps=maps)
-    g = driver.Calc(mol, driver.manual_mgparm([DIME] * 3, c, grid=[H] * 3), pbe,
+    g = driver.Calc(mol, driver.manual_mgparm([dime] * 3, c, grid=[H] * 3), pbe,
                     precision=precision)
     g._keep = (mol, maps)
     return g
 
 
-@pytest.mark.parametrize("precision,npbe", [(0, False), (1, False), (0, True), (1, True)])
-def test_negative_dielectric_is_reported(precision, npbe, capfd):
-    bad = calc(-5.0, precision, npbe)
+@pytest.mark.parametrize("precision,npbe,dime", [(0, False, 33), (1, False, 33), (0, True, 33),
+                                                 (1, True, 33), (0, False, 57), (1, False, 57)])
+def test_negative_dielectric_is_reported(precision, npbe, dime, capfd):
+    """33^3: a coarsest grid inverted in registers; 57^3: one of 8^3 (216
+    unknowns), inverted by blocks of pivots (in lpbe, where a pivot is what
+    reports it: in npbe a diverging iteration may also end at its limit of
+    steps with finite norms)."""
+    bad = calc(-5.0, precision, npbe, dime)
     bad.fillco()
     with pytest.raises(RuntimeError):
         bad.solve()
@@ -55,7 +60,7 @@ def test_negative_dielectric_is_reported(precision, npbe, capfd):
         assert "not positive definite" in err, err
     # the device and the library stay usable: the same object solves again
     # after a valid fill is impossible (its maps are fixed), so a fresh one
-    good = calc(20.0, precision, npbe)
+    good = calc(20.0, precision, npbe, dime)
     good.fillco()
     good.solve()
     st = good.stats()
