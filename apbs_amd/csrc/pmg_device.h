@@ -89,8 +89,8 @@ void gsrb27_pairs(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const 
 // its tile choice, coarse_device.hip).
 bool gsrb27_use_planes(int nx, int ny, int nz, int word);
 // Whether the colour-pair form is the one for a level that is not
-// plane-parity: rows of up to 128 interior points (81^3: 40 against 62 us per
-// FP64 sweep, 28 against 40 FP32; 97^3: 79 against 87; 65^3: 23 against 34).
+// plane-parity: rows of up to 128 interior points (one launch per colour against
+// the pairs at 129^3 in FP64: 177 and 94 us a sweep).
 bool gsrb27_use_pairs(int nx);
 
 // ------------------------------------------------------- residual / matvec
@@ -309,7 +309,7 @@ void gsrb27_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, 
 template <class T>
 void gsrb27_pairs_batch(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,
                         int nu, int iadjoint);
-// The same with the kernel chosen: form 0 the vector kernel (16-byte runs per
+// The same with the kernel chosen: form 0 the vector kernel (runs of two points a
 // lane) where the row allows it, 1 the one-point-per-lane kernel.
 template <class T>
 void gsrb27_pairs_form(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,

@@ -172,9 +172,9 @@ __global__ void __launch_bounds__(kBlock)
 // The vector form of the colour-pair launch.  In the form above a lane loads
 // one word per operand, with the lanes two words apart, so its 54 loads per
 // point keep the texture addresser (four lanes per clock) busy for most of
-// the launch.  Here a lane owns a run of kV consecutive points of a row (16
-// bytes: 4 floats or 2 doubles, both colours): each of the 26 coefficient
-// terms, f and D is one 16-byte load, and each of the 9 neighbouring rows of
+// the launch.  Here a lane owns a run of kV consecutive points of a row (8 or
+// 16 bytes, both colours): each of the 26 coefficient terms, f and D is one
+// load, and each of the 9 neighbouring rows of
 // x one window of kV + 2 values.  The A points of the run are updated first
 // (their row neighbours are B points, still old) and written to a row buffer
 // in LDS; after a barrier the B points take their new A neighbours from it.
@@ -1337,11 +1337,13 @@ void gsrb27(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const T* D, 
   gsrb27_batch<T>(s, nx, ny, nz, &c, 1, nu, iadjoint);
 }
 
-// The colour-pair sweeps with the vector kernel of kV-element runs.
-template <class T, int kV>
+// The colour-pair sweeps with the vector kernel.
+constexpr int kPairRun = 2;  // points of a run
+
+template <class T>
 static void vpair_launch(hipStream_t s, int nx, int ny, int nz, const Batch<Args27<T>>& B,
                          int nb, int nu, int iadjoint) {
-  const int R = (nx - 2 + kV - 1) / kV;
+  const int R = (nx - 2 + kPairRun - 1) / kPairRun;
   // workgroup size: whole rows, fewest idle lanes
   int NT = kBlock, idle = 1 << 30;
   for (int t = 64; t <= kBlock; t += 64) {
@@ -1362,38 +1364,26 @@ static void vpair_launch(hipStream_t s, int nx, int ny, int nz, const Batch<Args
       if (j0 > ny - 2 || k0 > nz - 2) continue;
       const long rows = (long)((ny - 2 - j0) / 2 + 1) * ((nz - 2 - k0) / 2 + 1);
       const dim3 g((unsigned)((rows + RB - 1) / RB), 1, (unsigned)nb);
-      k_gsrb27_vpair<T, kV><<<g, NT, (size_t)RB * nx * sizeof(T), s>>>(nx, ny, nz, B, pa, cj, ck,
-                                                                       R, RB);
+      k_gsrb27_vpair<T, kPairRun><<<g, NT, (size_t)RB * nx * sizeof(T), s>>>(nx, ny, nz, B, pa,
+                                                                             cj, ck, R, RB);
     }
 }
 
-// The colour-pair form.  Form 0 (the default): the vector kernel where a row
-// holds at least one run plus its boundary points and fits one workgroup,
-// with 16-byte runs in FP64 and 8-byte runs in FP32 (16-byte runs for rows
-// of 80 to 90 points), else the one-point-per-lane kernel; form 1 that
-// kernel; form 2 the vector kernel with 8-byte runs (FP32).  Per sweep (4
-// launches), us, FP32 8-byte runs / 16-byte runs / one point per lane: 57^3
-// 14.9 / - / 16.4, 65^3 15.3 / 19.9 / 16.6, 81^3 23.7 / 23.1 / 28.1, 97^3
-// 29.2 / 31.0 / 40.1, 113^3 43.1 / 45.0 / 57.4, 129^3 53.2 / 54.9 / 75.1;
-// FP64 16-byte runs / one point per lane: 65^3 20.8 / 23.3, 81^3 35.4 /
-// 40.3, 97^3 45.6 / 79.6, 129^3 95.2 / 162.7.
+// The colour-pair form, for the levels that gsrb27_use_planes leaves: rows of
+// fewer than 40 points on planes of more than 49 rows, and in FP64 rows of 115 to
+// 130.  Form 0 (the default): the vector kernel with runs of two points where a
+// row holds one run plus its boundary points and fits one workgroup, else the
+// one-point-per-lane kernel; form 1 that kernel.  Per sweep (4 launches), us, runs
+// and one point per lane: 129^3 FP64 93.9 and 161.7; 33x65x65 18.5 and 20.9 (FP32
+// 14.7 and 15.0).
 template <class T>
 void gsrb27_pairs_form(hipStream_t s, int nx, int ny, int nz, const LevelArgs<T>* c, int nb,
                        int nu, int iadjoint, int form) {
   check_batch(nb);
   const Batch<Args27<T>> B = args27(c, nb);
-  constexpr int kV = 16 / (int)sizeof(T), kV8 = 8 / (int)sizeof(T);
-  const bool wide = sizeof(T) == 8 || (nx >= 80 && nx <= 90);
-  if (form == 0 && wide && nx >= kV + 2 && (nx - 2 + kV - 1) / kV <= kBlock) {
-    vpair_launch<T, kV>(s, nx, ny, nz, B, nb, nu, iadjoint);
+  if (form == 0 && nx >= kPairRun + 2 && (nx - 2 + kPairRun - 1) / kPairRun <= kBlock) {
+    vpair_launch<T>(s, nx, ny, nz, B, nb, nu, iadjoint);
     return;
-  }
-  if constexpr (kV8 >= 2) {
-    if ((form == 2 || (form == 0 && !wide)) && nx >= kV8 + 2 &&
-        (nx - 2 + kV8 - 1) / kV8 <= kBlock) {
-      vpair_launch<T, kV8>(s, nx, ny, nz, B, nb, nu, iadjoint);
-      return;
-    }
   }
   for (int it = 0; it < nu; it++)
     for (int h = 0; h < 4; h++) {
@@ -1421,7 +1411,6 @@ void gsrb27_pairs(hipStream_t s, int nx, int ny, int nz, const Ops<T>& A, const 
 }
 
 bool gsrb27_use_pairs(int nx) { return nx >= 3 && nx <= 130; }
-
 
 template <class T>
 void resid_batch(hipStream_t s, int st, int nx, int ny, int nz, const LevelArgs<T>* c, int nb) {

@@ -35,7 +35,7 @@ bool tile7_ok(int nx, int word, int tile) {
   return tile < pmg::kBlockTile || pmg::block_sweep_fits(nx, word, tile - pmg::kBlockTile);
 }
 bool mode27_ok(int nx, int word, int mode) {
-  if (mode >= 2 && mode <= 4) return nx <= 130 && (mode != 4 || word == 4);
+  if (mode == 2 || mode == 3) return nx <= 130;
   return mode == 0 || mode == 1 || pmg::gsrb27_planes_fits(nx, word, mode);
 }
 struct OpsHolder {
@@ -120,7 +120,7 @@ double gs27_sweeps_us(int n, int sweeps, int mode) {
   auto run = [&](int nu) {
     if (mode == 0)
       pmg::gsrb27<T>(0, n, n, n, ops, D, fc, x, nu, 0);
-    else if (mode >= 2 && mode <= 4) {
+    else if (mode == 2 || mode == 3) {
       const pmg::LevelArgs<T> c{ops, D, fc, x, nullptr, nullptr};
       pmg::gsrb27_pairs_form<T>(0, n, n, n, &c, 1, nu, 0, mode - 2);
     }
@@ -576,7 +576,7 @@ int pmgtest_gsrb27_32(int nx, int ny, int nz, const float* a, const float* D, co
   const pmg::LevelArgs<float> c{ops, dD, df, dx, dt, nullptr};
   if (mode == 0)
     pmg::gsrb27_batch<float>(0, nx, ny, nz, &c, 1, nu, iadjoint);
-  else if (mode >= 2 && mode <= 4)
+  else if (mode == 2 || mode == 3)
     pmg::gsrb27_pairs_form<float>(0, nx, ny, nz, &c, 1, nu, iadjoint, mode - 2);
   else
     pmg::gsrb27_planes_batch<float>(0, nx, ny, nz, &c, 1, nu, iadjoint, mode == 1 ? 0 : mode);

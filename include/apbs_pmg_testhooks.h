@@ -82,8 +82,7 @@ int pmgtest_fused32(int nx, int ny, int nz, const float *oE, const float *oN, co
 /* pmgtest_gsrb (27-point) with the kernel form forced: mode 0 one launch per
  * colour, 1 one launch per plane parity (tile by level size), 2 one launch
  * per colour pair (nx <= 130; the vector kernel where the row allows it), 3 the
- * colour pair with one point per lane, 4 (FP32) the vector kernel with 8-byte runs,
- * 8 / 16 one launch per plane parity with that square tile, 100 kV + m with 2m
+ * colour pair with one point per lane, 8 / 16 one launch per plane parity with that square tile, 100 kV + m with 2m
  * whole rows and runs of kV points.  All give the same bits; returns 0 where
  * the form does not fit the row. */
 int pmgtest_gsrb27_mode(int nx, int ny, int nz, const double *a, const double *cc,

@@ -77,7 +77,7 @@ def test_gsrb_bitwise(L, O, st, n3, adj):
 def test_gsrb27_plane_sweeps_bitwise(L, O, n3, mode):
     """The plane-parity 27-point sweep (one launch per plane parity, tiles
     with recomputed margins) and the colour-pair sweep (mode 2 the vector
-    kernel, 16-byte runs per lane; mode 3 one wavefront per row) give the
+    kernel, runs of two points per lane; mode 3 one wavefront per row) give the
     oracle's 8-colour sweep bit for bit: both
     square tiles, partial tiles, forward and adjoint, even and odd sweep
     counts, rows of 1 to 128 interior points."""
@@ -175,7 +175,7 @@ def test_resid7_fp32_bitwise(L, n3):
 
 @pytest.mark.parametrize("n3", [(81, 81, 9), (45, 43, 41), (17, 17, 17), (9, 11, 13),
                                 (7, 6, 5), (130, 7, 6), (129, 6, 7)])
-@pytest.mark.parametrize("mode", [2, 3, 4, 1])
+@pytest.mark.parametrize("mode", [2, 3, 1])
 def test_gsrb27_fp32_forms_bitwise(L, n3, mode):
     """FP32 27-point sweeps: the colour-pair kernels (vector and one point
     per lane) and the plane-parity sweep give the per-colour kernel's bits
