@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "pmg_device.h"
+#include "vpmg_internal.h"
 
 #define TCHECK(x)                                                                          \
   do {                                                                                     \
@@ -178,6 +179,12 @@ double galerkin_us(int nf, int st, int form, int reps) {
 }
 
 extern "C" {
+
+// The host fill of a new object's partition array (vpmg_internal.h)
+int pmgtest_host_fill(double* p, size_t n, double v, int fail_at) {
+  pmgint::host_fill(p, n, v, fail_at);
+  return 1;
+}
 
 // Calibration for hardware byte counters: reps copies of n doubles (n*8
 // bytes read and n*8 bytes written per launch) between two device buffers.

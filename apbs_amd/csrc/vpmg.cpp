@@ -20,8 +20,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <string>
-#include <system_error>
 #include <limits>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -90,31 +90,32 @@ double* host_array(size_t n) {
   return p;
 }
 
-// p[0 .. n) = v.  The first touch of a large array is bound by its page faults
-// and one core's stores (353^3: 47 ms of a focused calculation's 157), so it is
-// shared by up to kFillThreads threads, 4 MB or more each.
+}  // namespace
+
+// The first touch of a large array is bound by its page faults and one core's
+// stores (353^3: 47 ms of a focused calculation's 157), so it is shared by up to
+// kFillThreads threads, 4 MB or more each.
 constexpr int kFillThreads = 8;
-void host_fill(double* p, size_t n, double v) {
+void pmgint::host_fill(double* p, size_t n, double v, int fail_at) {
   const size_t per = 512 * 1024;
   const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
   const int nt = (int)std::min<size_t>(std::min((unsigned)kFillThreads, hw), n / per);
   std::vector<std::thread> th;
-  th.reserve(nt > 0 ? nt : 1);
   size_t done = 0;
   try {
+    th.reserve(nt > 0 ? nt : 1);
     for (int t = 0; t + 1 < nt; t++) {
+      if (t == fail_at) throw std::bad_alloc();
       const size_t end = done + n / nt;
       th.emplace_back([=] { std::fill(p + done, p + end, v); });
       done = end;
     }
-  } catch (const std::system_error&) {
-    // no more threads: the rest is filled here
+  } catch (const std::exception&) {
+    // no more threads, or no memory for one: the rest is filled here
   }
   std::fill(p + done, p + n, v);
   for (std::thread& t : th) t.join();
 }
-
-}  // namespace
 
 // =================================================================== Valist
 
@@ -3137,7 +3138,7 @@ extern "C" void Vpmg_unsetPart(Vpmg* thee) {
     al->atoms[a].partID = 1.0;
   }
   upload_part(d);
-  if (d->mirror) host_fill(thee->pvec, d->n, 1.0);
+  if (d->mirror) pmgint::host_fill(thee->pvec, d->n, 1.0);
   HIPCHECK(hipStreamSynchronize(d->s));
   d->forces_valid = false;
 }

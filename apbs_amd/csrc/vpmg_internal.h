@@ -19,4 +19,8 @@ size_t footprint_bytes(int nx, int ny, int nz, int nlev, bool newton, bool mixed
 // contention (measured 3% fewer served solves/s).
 void set_side_stream(Vpmg* pmg, bool on);
 
+// p[0 .. n) = v on the host, by several threads where that pays.  fail_at is for
+// tests: the start of thread fail_at fails (-1: none).
+void host_fill(double* p, size_t n, double v, int fail_at = -1);
+
 }  // namespace pmgint

@@ -111,6 +111,10 @@ int pmgtest_dense_pivots(int N, int nb, const double *M, double *flags);
 /* No reference counterpart: microseconds per Galerkin call (form as above)
  * on a synthetic nf^3 operator of stencil st (nf odd). */
 int pmgtest_galerkin_time(int nf, int st, int form, int reps, double *us);
+/* No reference counterpart: p[0 .. n) = v by the host threads that fill a new
+ * object's partition array; thread fail_at cannot be started (-1: all can).
+ * Touches no device. */
+int pmgtest_host_fill(double *p, size_t n, double v, int fail_at);
 /* No reference counterpart: reps device copies of n doubles, the known-size
  * calibration for hardware byte counters (FETCH_SIZE / WRITE_SIZE). */
 int pmgtest_stream_copy(size_t n, int reps);

@@ -4,6 +4,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 
 import pytest
 
@@ -142,3 +143,21 @@ def test_footprint_estimate_host_only(lib):
     assert fp(97, serve.NPBE, 1) < big
     words = 161 ** 3 * 8
     assert 25 * words < big < 60 * words
+
+
+@pytest.mark.parametrize("n", [1000, 512 * 1024 * 3 + 5, 512 * 1024 * 9 + 7])
+@pytest.mark.parametrize("fail_at", [-1, 0, 1, 6])
+def test_host_fill(lib, n, fail_at):
+    """The threaded fill writes every value, whichever thread cannot be started:
+    its share is the caller's, and threads that run are waited for.  (In a
+    process of its own: an exception out of it ends the process.)"""
+    code = f"""
+import ctypes, numpy as np
+L = ctypes.CDLL({LIB!r})
+a = np.zeros({n} + 2)
+f = L.pmgtest_host_fill
+f.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_double, ctypes.c_int]
+assert f(a[1:].ctypes.data, {n}, 1.5, {fail_at}) == 1
+assert a[0] == 0 and a[-1] == 0 and (a[1:-1] == 1.5).all()
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=60)
