@@ -180,12 +180,13 @@ __device__ inline void tile_bounds(const Geo& g, const Tiles& T, int tile, int l
 // atoms, in ascending atom index (the order of the reference's per-atom loop).
 // An atom's contribution is a product of one weight per axis, so the weights
 // of its (at most 6) nodes per axis are evaluated once per tile: the list is
-// read kB atoms at a time, the atoms that reach the tile keep their order in
-// LDS with their node ranges, one thread per (atom, axis) fills the weight
-// table, and a point then costs a range test and three multiplications per
-// atom.  Evaluating the splines and the divisions per point and atom took
-// 800 us at 193^3 with 20,000 atoms (466 us so, next to the boundary kernel
-// that shares the GPU) and 68 us at 97^3 with 1,500 (20 us).
+// read kChargeCap atoms at a time, the atoms that reach the tile keep their
+// order in LDS with their node ranges, one thread per (atom, axis) fills the
+// weight table, and a point then costs a range test and three multiplications
+// per atom.  44 us at 193^3 with 20,000 atoms, 12 us at 97^3 with 1,500.  Beside
+// the FP64 boundary kernel, whose workgroups fill the chip, the former takes 1600
+// us (466 beside that kernel's one-point form, 800 with the splines and divisions
+// evaluated per point and atom; the latter 20 and 68 us).
 constexpr int kChargeCap = 128;  // atoms per table pass
 
 __global__ void __launch_bounds__(kB)
@@ -311,11 +312,11 @@ __device__ inline double poly_chi(const double* c, double sm, double sm2) {
 // kB atoms at a time: each thread forms one atom's box and radii (six
 // divisions, four squares), the atoms whose box meets the tile keep their
 // order in LDS, and every point walks those with integer tests first.  A wave
-// stops when all its points' windows have vanished: they stay zero.  Forming
-// the boxes per point and atom took 5334 us at 193^3 with 20,000 atoms (1259 us
-// so, next to the boundary kernel that shares the GPU) and 389 us at 97^3 with
-// 1,500 (181 us); leaving out the atoms whose windows reach no face of a point
-// before the four windows are formed, 1190 and 148 us.
+// stops when all its points' windows have vanished: they stay zero.  1055 us at
+// 193^3 with 20,000 atoms and 150 us at 97^3 with 1,500; at the former beside the
+// boundary kernel that shares the GPU 1220 us, 5334 with the boxes formed per
+// point and atom and 1259 with the four windows formed for every listed atom (the
+// latter 389 and 181 us).
 template <int kOrd>
 __global__ void __launch_bounds__(kB)
     k_coef_spline(Geo g, AtomsDev A, Tiles T, double win, double irad, double ionmask, double epsw,
@@ -984,8 +985,8 @@ __global__ void __launch_bounds__(kB)
 // absolute error of a few 1e-6 A; 1 / d is the hardware reciprocal square
 // root and exp(-kappa d) the hardware 2^x of -kappa log2(e) d, each about
 // one ulp.  A term is within about 1e-6 relative of the FP64 term (the
-// exponent's argument, at most a few tens, dominates); the partial sums and
-// their order are those of k_bc_mdh.
+// exponent's argument, at most a few tens, dominates); chunks of atoms are
+// summed and their sums added in order as in k_bc_mdh.
 __global__ void __launch_bounds__(kB)
     k_bc_mdh_atoms32(AtomsDev A, double pre1, double xkappa, double cx, double cy, double cz,
                      float4* at) {

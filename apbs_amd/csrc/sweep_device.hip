@@ -480,9 +480,12 @@ static int fused_tile_env() {
   return t;
 }
 
-// Default shape for a grid and word size: the vector form, with the rows x
+// The march's default shape for a grid and word size (the grids block_tile
+// leaves to it): the vector form, with the rows x
 // planes per workgroup that were fastest in standalone sweeps (us per sweep;
-// the best shape moves with how the workgroups fill the chip):
+// the best shape moves with how the workgroups fill the chip).  The shapes for
+// fewer points serve long rows and batches; a single 65^3 or 97^3 grid, and
+// 129^3 in FP32, take a block:
 //   FP32: up to 2.5M points 4 x 8 (65^3 12.2, 97^3 15.0, 129^3 20.3); up to
 //         5.5M 4 x 10 (161^3 29.7 against 36.5 for 4 x 8 and 50.2 for the
 //         scalar form); up to 20M 8 x 16 (193^3 49.3 against 70.8 for the
@@ -511,12 +514,17 @@ int fused_tile(int nx, int ny, int nz, int word) {
 }
 
 // Block shape (block_sweep_device.hip) of nb grids swept together, or 0 where
-// the march is the faster: above 1.5M points in all in FP64 (113^3 26.5 us a
-// sweep against 29.7, 129^3 32.3 against 31.9) and 3.1M in FP32 (145^3 22.4
-// against 27.5, 161^3 31.9 against 30.0).  The shape is the one of 256 or more
-// workgroups (one a CU; all shapes of a grid too small for that) that loads the
-// fewest runs per run written, the larger workgroup on a tie; rows so long that
-// it loads more than 2.7 (129^3 in FP64) keep the march.
+// the march is taken: above 1.5M points in all in FP64 (113^3 block 26.2 us a
+// sweep, march 29.1; 129^3 31.2 and 30.8) and 3.1M in FP32 (145^3 22.4 and 27.5,
+// 161^3 31.9 and 30.0; long rows meet earlier, 225x97x97 20.9 and 20.2).  The
+// shape is the one of 256 or more workgroups (one a CU; all shapes of a grid too
+// small for that) that loads the fewest runs per run written, the larger
+// workgroup on a tie.  Rows of more than 130 points in FP64 (258 in FP32) leave
+// shapes that load three runs and more for one written; from 100,000 points such
+// a grid keeps the march, which is right for the larger (161x97x97 FP64 28.1 and
+// 24.5) and not for the smaller ones (161x65x65 13.5 and 18.1).  At 129 points the
+// shape of 2 rows and 3 planes, 2.7 runs for one, is the faster: 129x129x65 18.2
+// and 23.5, 129x97x97 17.9 and 23.5, 129x65x65 10.3 and 16.8.
 static int block_tile(int nx, int ny, int nz, int word, int nb) {
   const double pts = (double)nx * ny * nz * nb;
   if (pts > (word == 8 ? 1.5e6 : 3.1e6)) return 0;
