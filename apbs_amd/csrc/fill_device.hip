@@ -1772,15 +1772,20 @@ void mol_maps(hipStream_t s, const Geo& g, const unsigned char* atom_flags,
 
 // Chunks of the atom list: enough that the FP64 kernel's launch holds about
 // 2,048 workgroups (8 a CU; a 65^3 grid's faces alone are 30), of 16 atoms or
-// more.  The FP32 kernel takes up to eight chunks of 512 atoms or more beyond
-// that: it holds four times the workgroups, of a quarter of the work, and on
-// large grids the rule's few chunks leave its last round of them short (353^3
-// with 5,000 atoms, two chunks 1422 us, eight 1368; 2,000 atoms 575, three 566).
+// more.  Fewer than 64 atoms on grids that leave the chip most of its workgroups
+// (97^3 and less) take chunks of 8 in FP64: a thread's four points an atom are
+// then what the launch waits for (33^3: 10 atoms in one chunk 11.2 us, in two
+// 9.2, 30 atoms in one 20.7, in four 10.9).  The FP32 kernel takes up to eight chunks of 512 atoms or
+// more beyond that: it holds four times the workgroups, of a quarter of the
+// work, and on large grids the rule's few chunks leave its last round of them
+// short (353^3 with 5,000 atoms, two chunks 1422 us, eight 1368; 2,000 atoms 575,
+// three 566).
 static int bc_mdh_chunks(const Geo& g, int natoms, bool fp32_terms) {
   const long mx = std::max((long)g.ny * g.nz, std::max((long)g.nx * g.nz, (long)g.nx * g.ny));
   const long groups = 6 * ((mx / kMdhRun + kB - 1) / kB);
   const long want = std::max(1L, 2048 / groups);
-  const long rule = std::max(1L, std::min(want, (long)natoms / 16));
+  const long most = !fp32_terms && natoms < 64 && want > 32 ? (natoms + 7L) / 8 : natoms / 16;
+  const long rule = std::max(1L, std::min(want, most));
   return (int)(fp32_terms ? std::max(rule, std::min(8L, (long)natoms / 512)) : rule);
 }
 
@@ -1794,9 +1799,10 @@ size_t bc_mdh_scratch(const Geo& g, int natoms) {
   size_t mx = (size_t)g.ny * g.nz;
   if ((size_t)g.nx * g.nz > mx) mx = (size_t)g.nx * g.nz;
   if ((size_t)g.nx * g.ny > mx) mx = (size_t)g.nx * g.ny;
-  // partial sums (FP32 terms take as many chunks or more), then the per-atom
-  // factors (FP64) or float4 atoms (two doubles each)
-  return (size_t)bc_mdh_chunks(g, natoms, true) * 6 * mx + 2 * (size_t)(natoms > 0 ? natoms : 1);
+  // partial sums of either kernel, then the per-atom factors (FP64) or float4
+  // atoms (two doubles each)
+  const int nch = std::max(bc_mdh_chunks(g, natoms, false), bc_mdh_chunks(g, natoms, true));
+  return (size_t)nch * 6 * mx + 2 * (size_t)(natoms > 0 ? natoms : 1);
 }
 
 void bc_mdh(hipStream_t s, const Geo& g, const double* xf, const double* yf, const double* zf,

@@ -64,21 +64,21 @@ def boundary(xyz, q, r, dims, h, salt, precision=0):
 
 
 @pytest.mark.parametrize("salt", [0.15, 0.0])
-@pytest.mark.parametrize("natoms,dims,h", [(31, (33, 33, 33), 0.5), (32, (33, 33, 33), 0.5),
-                                           (300, (33, 49, 41), 0.875), (2000, (49, 49, 49), 1.0),
-                                           (5000, (17, 17, 17), 4.0)])
+@pytest.mark.parametrize("natoms,dims,h", [(8, (33, 33, 33), 0.5), (9, (33, 33, 33), 0.5),
+                                           (31, (33, 33, 33), 0.5), (63, (41, 33, 41), 0.75),
+                                           (64, (41, 33, 41), 0.75), (300, (33, 49, 41), 0.875),
+                                           (2000, (49, 49, 49), 1.0), (5000, (17, 17, 17), 4.0)])
 def test_sums(natoms, dims, h, salt):
-    """Atom counts around the turn from one chunk to two (32), ordinary ones, and
-    many more atoms than boundary points: 312 chunks of 16 or 17 atoms, whose sum
-    is as long as its unrolled loop and remainder.  The FP32-term sum within
-    1e-5 of the largest value."""
+    """Atom counts around the turns from one chunk to two (8) and from chunks of
+    8 atoms to chunks of 16 (64), ordinary ones, and many more atoms than
+    boundary points: 312 chunks, whose sum is as long as its unrolled loop and
+    remainder.  The FP32-term sum within 1e-5 of the largest value."""
     rad = max(2.6, (natoms / 120.0) ** (1.0 / 3.0) * 6.0)
     xyz, q, r, _ = synth.globule(natoms, (rad,) * 3, 5, net_charge=-2)
     got, nodes, pre1, kappa = boundary(xyz, q, r, dims, h, salt)
     exact, mag, far = face_sums(xyz, q, r, nodes, pre1, kappa)
     err = np.abs(got - exact)
-    # (n/c + c: one chunk of 31, two of 16, then 16 to 18 atoms a chunk, up to
-    # 312 chunks)
+    # (n/c + c: up to 18 atoms a chunk, up to 312 chunks)
     bound = U * ((16 + min(natoms + 1, 330)) * mag + 6 * far)
     rms = float(np.linalg.norm(err.astype(float)) / np.linalg.norm(exact.astype(float)))
     print(f"{natoms} atoms, salt {salt}: rms error {rms:.2e}, largest error over its bound "
