@@ -382,10 +382,11 @@ __global__ void __launch_bounds__(kB)
       ssctot2[slot] = sctot2;
       srad[slot] = arad;
       sa[slot] = a;
-      // (a face lies half a spacing from its point; widened past rounding; with a
-      // negative win the core reaches past the outer radius: no test then)
+      // (a face lies half a spacing from its point; widened past rounding; a window
+      // of no width, or a negative one, puts the core's radius at or past the outer
+      // one: no test then)
       const double far = (arad + win + 0.5 * fmax(hx, fmax(hy, hzed))) * (1.0 + 1e-9);
-      sfar2[slot] = win >= 0.0 ? far * far : HUGE_VAL;
+      sfar2[slot] = itot2 > ictot2 ? far * far : HUGE_VAL;
     }
     __syncthreads();
     for (int e = 0; e < cnt; e++) {

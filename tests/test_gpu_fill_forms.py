@@ -59,3 +59,25 @@ def test_windows_of_no_width(srfm, swin):
     for name in ("epsx", "epsy", "epsz", "kappa"):
         off = int((~np.isclose(g.array(name), o.array(name), 0, 0, equal_nan=True)).sum())
         assert off == 0, (name, off)
+
+
+@pytest.mark.parametrize("srfm", ["spl2", "spl3", "spl4"])
+@pytest.mark.parametrize("swin", [0.0, 1e-20, 0.5])
+def test_nodes_on_the_window_edges(srfm, swin):
+    """Nodes and face centres exactly at an atom's radii: atoms on nodes, radii
+    and radii with the ion's a multiple of half the spacing.  With a window of no
+    width (0, or too little to change the radius) such a point is in the core."""
+    xyz = np.array([[0.0, 0.0, 0.0], [5.0, -1.0, 2.0], [-5.5, 4.0, -3.0]])
+    atoms = (xyz, np.array([1.0, -0.5, 0.5]), np.array([2.0, 1.5, 1.75]))
+    pbe = dict(pdie=2.0, sdie=78.54, srfm=srfm, chgm="spl2", swin=swin, srad=1.4, sdens=10.0,
+               temp=298.15, bcfl="zero", ions=[(1, 0.15, 2.0), (-1, 0.15, 2.0)])
+    c = np.zeros(3)
+    mol = driver.Molecule(*atoms)
+    g = driver.Calc(mol, driver.manual_mgparm([65, 65, 65], c, grid=[0.5] * 3), pbe)
+    g.fillco()
+    nlev, dime = od.check_nlev([65, 65, 65])
+    o = od.OrcCalc(od.make_params(dime, [0.5] * 3, c, nlev, pbe), atoms)
+    o.fillco()
+    for name in ("epsx", "epsy", "epsz", "kappa"):
+        off = int((~np.isclose(g.array(name), o.array(name), 0, 0, equal_nan=True)).sum())
+        assert off == 0, (name, off)
