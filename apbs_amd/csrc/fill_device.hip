@@ -147,8 +147,8 @@ __device__ inline void tile_point(const Tiles& T, int tile, int tid, int r, int&
   k = tz * kTile + tid / (kTile * kTile) + 4 * r;
 }
 
-// Threads of a workgroup that hold `keep` get consecutive slots from `base`
-// in thread order (a list stays in its order); returns the slot, or -1.
+// Threads of a workgroup that hold `keep` get consecutive slots from 0 in
+// thread order (a list stays in its order); returns the slot, or -1.
 // `cnt` receives the number kept.
 __device__ inline int ordered_slot(bool keep, int* wsum, int& cnt) {
   const int lane = threadIdx.x % 64, w = threadIdx.x / 64;

@@ -389,7 +389,7 @@ void dense_invert_batch(hipStream_t s, int N, const InvertArgs* c, int nb, int f
 
 // ----------------------------------------------------- coarsest level (dense)
 // Assemble the dense (N x N) operator of the interior of a 27-point level with
-// diagonal D, then invert it in place (Gauss-Jordan, SPD, one workgroup).
+// diagonal D, then invert it in place (Gauss-Jordan, SPD).
 void dense_assemble(hipStream_t s, int nx, int ny, int nz, const Ops<double>& A, const double* D,
                     double* M, int N);
 // form 0: registers for N <= 64 (one barrier per pivot), else LDS, else blocks;

@@ -94,10 +94,9 @@ double fused_sweeps_us(int n, int sweeps, int tile) {
   return 1e3 * ms / sweeps;
 }
 
-// The 27-point 8-colour sweeps alone on an n^3 coarse-level operator: mode 0
-// one launch per colour, mode 1 one per plane parity (tile by level size),
-// 8 / 16 / 32 one per plane parity with that tile.  One untimed call, then
-// one timed call of `sweeps` sweeps; microseconds per sweep.
+// The 27-point 8-colour sweeps alone on an n^3 coarse-level operator, in the form
+// mode names (see the header): two untimed sweeps, then `sweeps` timed ones;
+// microseconds per sweep.
 template <class T>
 double gs27_sweeps_us(int n, int sweeps, int mode) {
   const size_t N = (size_t)n * n * n;
